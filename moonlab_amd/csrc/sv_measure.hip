@@ -67,15 +67,29 @@ __global__ __launch_bounds__(kMeasThreads) void k_outcome_probs(const cplx_t<R> 
     }
 }
 
-// out[o] = sum over c of partial[c][o], c ascending
-__global__ void k_sum_columns(const double *__restrict__ partial, uint64_t rows, uint64_t cols,
-                              double *__restrict__ out)
+// out[o] = sum over c of partial[c][o] in a fixed order.  WIDE: one workgroup
+// per outcome (rows c = t, t + 256, ... per thread, then a butterfly); else
+// one thread per outcome, c ascending.
+template <bool WIDE>
+__global__ __launch_bounds__(kMeasThreads) void k_sum_columns(const double *__restrict__ partial, uint64_t rows,
+                                                              uint64_t cols, double *__restrict__ out)
 {
-    const uint64_t o = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (o >= cols) return;
-    double s = 0.0;
-    for (uint64_t c = 0; c < rows; c++) s += partial[c * cols + o];
-    out[o] = s;
+    if constexpr (WIDE) {
+        __shared__ double wsum[kMeasThreads / 64];
+        const uint64_t o = blockIdx.x;
+        double s = 0.0;
+        for (uint64_t c = threadIdx.x; c < rows; c += kMeasThreads) s += partial[c * cols + o];
+        s = wave_total(s);
+        if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = s;
+        __syncthreads();
+        if (threadIdx.x == 0) out[o] = ((wsum[0] + wsum[1]) + wsum[2]) + wsum[3];
+    } else {
+        const uint64_t o = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+        if (o >= cols) return;
+        double s = 0.0;
+        for (uint64_t c = 0; c < rows; c++) s += partial[c * cols + o];
+        out[o] = s;
+    }
 }
 
 // mode 0: zero the amplitudes whose masked bits differ from want; mode 1:
@@ -130,7 +144,15 @@ hipError_t launch_outcome_probs(const SvDev &s, const int *qubits, int k, double
             (const cplx_t<double> *)s.amps, s.n, g, cb, d);
     e = hipGetLastError();
     if (e == hipSuccess) {
-        k_sum_columns<<<(unsigned)((nout + 255) / 256), 256, 0, s.stream>>>(d, rows, nout, d + nout * rows);
+        // The column sums are a chain of dependent loads: one thread walking
+        // 512 rows (24 qubits, 3 measured) took 78 us, a workgroup per
+        // column 4 us.  Up to 16 rows the chain is short (under 4 us) and
+        // there may be 2^20 columns: one thread each.
+        if (rows > 16)
+            k_sum_columns<true><<<(unsigned)nout, kMeasThreads, 0, s.stream>>>(d, rows, nout, d + nout * rows);
+        else
+            k_sum_columns<false><<<(unsigned)((nout + 255) / 256), kMeasThreads, 0, s.stream>>>(d, rows, nout,
+                                                                                                d + nout * rows);
         e = hipGetLastError();
     }
     if (e == hipSuccess)

@@ -10,14 +10,14 @@
 // tile, qubits 0..7 are thread-index bits, qubits 8..11 are the e bits, and
 // qubits >= 12 are bits of the tile number, so per-qubit sums come from 11
 // wave reductions per tile plus a per-tile total.  Each block walks a fixed
-// set of tiles and leaves n+1 FP64 partials; a final one-block kernel sums
-// the partials in block order.  Grid size and tile assignment depend only on
+// set of tiles and leaves n+1 FP64 partials; a final kernel sums each
+// value's partials in a fixed order.  Grid size and tile assignment depend only on
 // n, so every result is bit-reproducible run to run and independent of what
 // else shares the GPU.
 //
-// States below 2^12 amplitudes are reduced by one block that sums each
-// qubit's probabilities sequentially in index order -- the reference's own
-// summation order (measurement.c:99-103).
+// States below 2^12 amplitudes are one partly filled tile of the same kernel
+// (a block that summed each qubit's probabilities one after another in index
+// order took 60 us at 10 qubits, this 5 us).
 #include "sv_device.h"
 #include "sv_internal.h"
 
@@ -47,8 +47,9 @@ __device__ __forceinline__ double prob(const cplx_t<R> &x)
     return fmar(r, r, i * i);
 }
 
-// n >= 12: tiles of 4096 amplitudes.
-template <typename R>
+// Tiles of 4096 amplitudes (n < 12: one tile of dim < 4096, FULL false; its
+// missing amplitudes count as 0).
+template <typename R, bool FULL>
 __global__ __launch_bounds__(kRedThreads) void k_reduce_tiles(const cplx_t<R> *__restrict__ a, int n,
                                                               uint64_t ntiles,
                                                               double *__restrict__ partial,
@@ -63,7 +64,8 @@ __global__ __launch_bounds__(kRedThreads) void k_reduce_tiles(const cplx_t<R> *_
         const cplx_t<R> *t = a + (tile << kTileBits);
         double p[kEpt];
 #pragma unroll
-        for (int e = 0; e < kEpt; e++) p[e] = prob<R>(t[e * kRedThreads + tid]);
+        for (int e = 0; e < kEpt; e++)
+            p[e] = FULL || e * kRedThreads + tid < (1 << n) ? prob<R>(t[e * kRedThreads + tid]) : 0.0;
         double tot = 0.0, hb0 = 0.0, hb1 = 0.0, hb2 = 0.0, hb3 = 0.0;
 #pragma unroll
         for (int e = 0; e < kEpt; e++) {
@@ -106,39 +108,32 @@ __global__ __launch_bounds__(kRedThreads) void k_reduce_tiles(const cplx_t<R> *_
     if (tid < nvals) partial[(size_t)blockIdx.x * nvals + tid] = acc;
 }
 
-// n < 12: one block, sequential sums in index order.
-template <typename R>
-__global__ __launch_bounds__(kRedThreads) void k_reduce_small(const cplx_t<R> *__restrict__ a, int n,
-                                                              double *__restrict__ partial,
-                                                              double *__restrict__ tile_sums)
+// Sum of column v of the partials [blocks][nvals] by one workgroup: thread t
+// takes rows t, t + 256, ..., then a wave butterfly and the four waves in
+// order.  Call with all 256 threads; the result is valid on every thread.
+__device__ __forceinline__ double column_sum(const double *__restrict__ partial, int blocks, int nvals, int v)
 {
-    __shared__ double p[1 << kTileBits];
-    const int dim = 1 << n;
-    for (int i = threadIdx.x; i < dim; i += blockDim.x) p[i] = prob<R>(a[i]);
+    __shared__ double red[kRedThreads / 64];
+    double s = 0.0;
+#pragma unroll 4
+    for (int b = threadIdx.x; b < blocks; b += kRedThreads) s += partial[(size_t)b * nvals + v];
+    s = wave_sum(s);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
     __syncthreads();
-    const int v = threadIdx.x;
-    if (v <= n) {
-        double s = 0.0;
-        if (v == 0) {
-            for (int i = 0; i < dim; i++) s += p[i];
-            if (tile_sums) tile_sums[0] = s;
-        } else {
-            const int mk = 1 << (v - 1);
-            for (int i = 0; i < dim; i++)
-                if (i & mk) s += p[i];
-        }
-        partial[v] = s;
-    }
+    return ((red[0] + red[1]) + red[2]) + red[3];
 }
 
-__global__ void k_reduce_final(const double *__restrict__ partial, int blocks, int nvals,
-                               double *__restrict__ out)
+// One workgroup per value.  Latency bound: with one thread per value adding
+// up to 2048 rows one after another (a dependent load and add each) this
+// kernel took 60 us at 20 qubits, 200 us at 24 and 760 us at 30, more than
+// the pass over the state it finishes below 27 qubits; 256 rows at a time
+// it takes 3-5 us at every size.
+__global__ __launch_bounds__(kRedThreads) void k_reduce_final(const double *__restrict__ partial, int blocks,
+                                                              int nvals, double *__restrict__ out)
 {
-    const int v = threadIdx.x;
-    if (v >= nvals) return;
-    double s = 0.0;
-    for (int b = 0; b < blocks; b++) s += partial[(size_t)b * nvals + v];
-    out[v] = s;
+    const int v = blockIdx.x;
+    const double s = column_sum(partial, blocks, nvals, v);
+    if (threadIdx.x == 0) out[v] = s;
 }
 
 // Inclusive prefix of the tile sums (one block, fixed chunking).
@@ -375,25 +370,24 @@ void reduce_geometry(int n, int *tile_bits, uint64_t *ntiles, int *blocks)
     *blocks = (int)(*ntiles < (uint64_t)kMaxRedBlocks ? *ntiles : kMaxRedBlocks);
 }
 
+// The block partials of norm and P(1), [blocks][n + 1], and the tile sums
+// when ts is not null (geometry of reduce_geometry).
+static hipError_t reduce_tiles(const void *amps, int n, int prec, uint64_t ntiles, int blocks, double *partial,
+                               double *ts, hipStream_t st)
+{
+    auto go = [&](auto kernel, auto *a) { kernel<<<blocks, kRedThreads, 0, st>>>(a, n, ntiles, partial, ts); };
+    const bool full = n >= kTileBits;
+    if (prec == MOONLAB_HIP_C64) go(full ? k_reduce_tiles<float, true> : k_reduce_tiles<float, false>, (const float2 *)amps);
+    else go(full ? k_reduce_tiles<double, true> : k_reduce_tiles<double, false>, (const double2 *)amps);
+    return hipGetLastError();
+}
+
 hipError_t launch_reduce_z(const SvDev &s, const ReduceWs &w, bool want_tiles)
 {
     double *ts = want_tiles ? w.tile_sums : nullptr;
-    if (s.n < kTileBits) {
-        if (s.prec == MOONLAB_HIP_C64)
-            k_reduce_small<float><<<1, kRedThreads, 0, s.stream>>>((const float2 *)s.amps, s.n, w.partial, ts);
-        else
-            k_reduce_small<double><<<1, kRedThreads, 0, s.stream>>>((const double2 *)s.amps, s.n, w.partial, ts);
-    } else {
-        if (s.prec == MOONLAB_HIP_C64)
-            k_reduce_tiles<float><<<w.blocks, kRedThreads, 0, s.stream>>>(
-                (const float2 *)s.amps, s.n, w.ntiles, w.partial, ts);
-        else
-            k_reduce_tiles<double><<<w.blocks, kRedThreads, 0, s.stream>>>(
-                (const double2 *)s.amps, s.n, w.ntiles, w.partial, ts);
-    }
-    hipError_t e = hipGetLastError();
+    hipError_t e = reduce_tiles(s.amps, s.n, s.prec, w.ntiles, w.blocks, w.partial, ts, s.stream);
     if (e != hipSuccess) return e;
-    k_reduce_final<<<1, 64, 0, s.stream>>>(w.partial, s.n < kTileBits ? 1 : w.blocks, s.n + 1, w.out);
+    k_reduce_final<<<s.n + 1, kRedThreads, 0, s.stream>>>(w.partial, w.blocks, s.n + 1, w.out);
     return hipGetLastError();
 }
 
@@ -438,7 +432,7 @@ hipError_t launch_xy(const SvDev &s, int q, double *d_partial, int blocks, doubl
         k_xy<double><<<g, 256, 0, s.stream>>>((const double2 *)s.amps, np, q, d_partial);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    k_reduce_final<<<1, 64, 0, s.stream>>>(d_partial, g, 2, d_out);
+    k_reduce_final<<<2, kRedThreads, 0, s.stream>>>(d_partial, g, 2, d_out);
     return hipGetLastError();
 }
 
@@ -456,7 +450,7 @@ hipError_t launch_pauli(const SvDev &s, uint64_t x, uint64_t z, double *d_partia
         k_pauli<double><<<g, 256, 0, s.stream>>>((const double2 *)s.amps, np, p, x, z, cr, ci, d_partial);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    k_reduce_final<<<1, 64, 0, s.stream>>>(d_partial, g, 1, d_out);
+    k_reduce_final<<<1, kRedThreads, 0, s.stream>>>(d_partial, g, 1, d_out);
     return hipGetLastError();
 }
 
@@ -470,7 +464,7 @@ hipError_t launch_zmask(const SvDev &s, uint64_t mask, double *d_partial, int bl
         k_zmask<double><<<g, 256, 0, s.stream>>>((const double2 *)s.amps, dim, mask, d_partial);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    k_reduce_final<<<1, 64, 0, s.stream>>>(d_partial, g, 1, d_out);
+    k_reduce_final<<<1, kRedThreads, 0, s.stream>>>(d_partial, g, 1, d_out);
     return hipGetLastError();
 }
 
@@ -493,15 +487,15 @@ hipError_t launch_inner(const SvDev &a, const SvDev &b, double *d_partial, int b
                                                          d_partial);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    k_reduce_final<<<1, 64, 0, a.stream>>>(d_partial, g, 2, d_out);
+    k_reduce_final<<<2, kRedThreads, 0, a.stream>>>(d_partial, g, 2, d_out);
     return hipGetLastError();
 }
 
 }  // namespace mlx
 
 // ---------------------------------------------------------------------------
-// Norm and <Z_q> without allocating: the block partials of k_reduce_tiles /
-// k_reduce_small live in a fixed device array instead of a state's workspace.
+// Norm and <Z_q> without allocating: the block partials of k_reduce_tiles
+// live in a fixed device array instead of a state's workspace.
 //
 // kNoAllocMaxQubits bounds the array: kMaxRedBlocks blocks x (n + 1) FP64
 // partials for n <= 35 (complex64's limit) is 2048 x 36 x 8 B = 576 KiB per
@@ -541,14 +535,13 @@ hipError_t scratch_on_current_device(double **out)
     return hipSuccess;
 }
 
-__global__ void k_z_from_sums(const double *__restrict__ partial, int blocks, int nvals, double *__restrict__ out)
+__global__ __launch_bounds__(mlx::kRedThreads) void k_z_from_sums(const double *__restrict__ partial, int blocks,
+                                                                  int nvals, double *__restrict__ out)
 {
-    const int v = threadIdx.x;
-    if (v >= nvals) return;
-    double s = 0.0;
-    for (int b = 0; b < blocks; b++) s += partial[(size_t)b * nvals + v];
+    const int v = blockIdx.x;
+    const double s = mlx::column_sum(partial, blocks, nvals, v);
     // 1 - 2 P(1): 2 s is exact, so this rounds once, as 1.0 - 2.0 * s does
-    out[v] = v == 0 ? s : __builtin_fma(-2.0, s, 1.0);
+    if (threadIdx.x == 0) out[v] = v == 0 ? s : __builtin_fma(-2.0, s, 1.0);
 }
 
 }  // namespace
@@ -575,22 +568,9 @@ extern "C" moonlab_hip_status_t moonlab_hip_expect_z_all_noalloc(const void *amp
     const hipStream_t st = (hipStream_t)stream;
     // the same kernels, grid and partial layout as moonlab_hip_expect_z_all,
     // so the sums are bit-identical
-    if (n < kTileBits) {
-        if (precision == MOONLAB_HIP_C64)
-            k_reduce_small<float><<<1, kRedThreads, 0, st>>>((const float2 *)amplitudes, n, partial, nullptr);
-        else
-            k_reduce_small<double><<<1, kRedThreads, 0, st>>>((const double2 *)amplitudes, n, partial, nullptr);
-    } else {
-        if (precision == MOONLAB_HIP_C64)
-            k_reduce_tiles<float><<<blocks, kRedThreads, 0, st>>>((const float2 *)amplitudes, n, ntiles, partial,
-                                                                  nullptr);
-        else
-            k_reduce_tiles<double><<<blocks, kRedThreads, 0, st>>>((const double2 *)amplitudes, n, ntiles,
-                                                                   partial, nullptr);
-    }
-    e = hipGetLastError();
+    e = reduce_tiles(amplitudes, n, precision, ntiles, blocks, partial, nullptr, st);
     if (e == hipSuccess) {
-        k_z_from_sums<<<1, 64, 0, st>>>(partial, blocks, n + 1, out);
+        k_z_from_sums<<<n + 1, kRedThreads, 0, st>>>(partial, blocks, n + 1, out);
         e = hipGetLastError();
     }
     if (e != hipSuccess) return set_last_error(MOONLAB_HIP_ERR_DRIVER, "expect_z_all_noalloc: launch", e);
