@@ -31,6 +31,7 @@
 #include "../../include/moonlab_mi355x.h"
 #include "batch_device.h"
 #include "batch_plan.h"
+#include "frame_plan.h"
 #include "fusion.h"
 #include "sv_internal.h"
 
@@ -39,6 +40,7 @@ namespace mlx {
 hipError_t launch_tile_pass(void *amps, int prec, int n, const BPass &P, const BOp *d_ops, int cus, int threads,
                             int tile_bits, hipStream_t st);
 hipError_t launch_reg_pass(void *amps, int prec, int n, const BPass &P, const BOp *d_ops, int reg_bits, hipStream_t st);
+hipError_t launch_frame_pass(void *amps, int prec, int n, const FPass &P, const FOp *d_prog, hipStream_t st);
 
 hipError_t launch_batch(const BInst *insts, const int32_t *order, int ninst, int *counter, const BPass *passes,
                         const BOp *ops, double2 *scratch, uint64_t slot_amps, double *tile_scratch,
@@ -634,7 +636,8 @@ void plan_passes(const std::vector<GOp> &gops, int n, int tb, int seg_regs, std:
 
 namespace {
 
-// Tile bits and engine of the single-state blocked path: the register-phase
+// Tile bits and engine of the single-state blocked path, where it does not
+// run as rotations (plan_frames below): the register-phase
 // engine for states of at least 12 qubits (16 register values per thread;
 // 12-qubit tiles for complex128, 13-qubit tiles for complex64, unless the
 // tuning fixes them), the LDS op engine otherwise or when selected (11- or
@@ -655,6 +658,40 @@ int blocked_shape(int n, int prec, const GateTuning &t, bool *reg, int *anchor, 
     *anchor = 4;
     const int b = t.blocked_tile_bits == 0 || t.blocked_tile_bits > 12 ? 12 : t.blocked_tile_bits;
     return n < b ? n : b;
+}
+
+// The blocked path's default engine: the gate list as Pauli rotations
+// (frame_plan.h), one pass for states of 4..11 qubits, 12-qubit tiles for
+// complex128 and 13-qubit ones for complex64 (or as tuned) above.  On
+// 30-qubit random layers a pass takes less than half of the register-phase
+// engine's (figures at k_frame_pass).  False where that engine stays: it is
+// selected, the state has under 4 qubits (four register bits), or a
+// parameter is not finite (a rotation would spread it to amplitudes that the
+// gate leaves alone).
+bool plan_frames(const moonlab_hip_gate_t *g, int ng, int n, int prec, const GateTuning &t, std::vector<FPass> &passes,
+                 std::vector<FOp> &prog)
+{
+    if (t.blocked_engine != 0 || n < kFrameRegBits) return false;
+    std::vector<FGate> fg;
+    cd phase;
+    if (!frame_lower(g, ng, n, fg, phase)) return false;
+    const bool c64 = prec == MOONLAB_HIP_C64;
+    const int want = t.blocked_tile_bits ? t.blocked_tile_bits : (c64 ? 13 : 12);
+    frame_plan(fg, phase, n, want >= 13 && n >= 13 ? 13 : 12, c64 ? 4 : 3, c64 ? 8 : 16, t.blocked_lookahead, passes,
+               prog);
+    prog.push_back(FOp{});   // the kernels fetch one unit past the last rotation
+    return true;
+}
+
+// Program units or ops to device memory in stream order; the host copy may
+// go when this returns.
+template <typename T> hipError_t upload(const std::vector<T> &v, T **d, hipStream_t st)
+{
+    *d = nullptr;
+    hipError_t e = hipMallocAsync((void **)d, v.size() * sizeof(T), st);
+    if (e == hipSuccess) e = hipMemcpyAsync(*d, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, st);
+    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    return e;
 }
 
 double now_s()
@@ -1047,19 +1084,34 @@ moonlab_hip_status_t moonlab_hip_apply_gates_blocked(moonlab_hip_state_t *s, con
     if (!s || ng < 0 || (ng > 0 && !g)) return MOONLAB_HIP_ERR_BAD_ARG;
     if (ng == 0) return MOONLAB_HIP_OK;
     const int n = (int)moonlab_hip_state_n_qubits(s);
+    const GateTuning tune = gate_tuning();
+    const int prec = moonlab_hip_state_precision(s);
+    hipStream_t st = (hipStream_t)moonlab_hip_state_stream(s);
+    void *amps = moonlab_hip_state_device_ptr(s);
+    auto status = [](hipError_t e) {
+        if (e == hipErrorOutOfMemory) return MOONLAB_HIP_ERR_OUT_OF_MEMORY;
+        return e == hipSuccess ? MOONLAB_HIP_OK : MOONLAB_HIP_ERR_DRIVER;
+    };
+    std::vector<FPass> fp;
+    std::vector<FOp> prog;
+    if (plan_frames(g, ng, n, prec, tune, fp, prog)) {
+        if (fp.empty()) return MOONLAB_HIP_OK;
+        FOp *d_prog = nullptr;
+        hipError_t e = upload(prog, &d_prog, st);
+        for (size_t i = 0; e == hipSuccess && i < fp.size(); i++) e = launch_frame_pass(amps, prec, n, fp[i], d_prog, st);
+        if (d_prog) hipFreeAsync(d_prog, st);
+        return status(e);
+    }
     std::vector<GOp> gops;
     if (!lower(g, ng, n, gops)) return MOONLAB_HIP_ERR_INVALID_QUBIT;
     std::vector<BPass> passes;
     std::vector<BOp> ops;
-    const GateTuning tune = gate_tuning();
-    const int prec = moonlab_hip_state_precision(s);
     bool reg = false;
     int anchor = 4, reg_bits = kRegBits;
     const int tb = blocked_shape(n, prec, tune, &reg, &anchor, &reg_bits);
     plan_passes(gops, n, tb, reg ? kRegPhases : kSegRegsPass, passes, ops, anchor,
                 prec == MOONLAB_HIP_C64 ? 8 : 16, reg_bits, tune.blocked_lookahead);
     if (ops.empty()) return MOONLAB_HIP_OK;
-    hipStream_t st = (hipStream_t)moonlab_hip_state_stream(s);
     static std::atomic<int> cached_cus{0};   // shared by every launching thread
     int cus = cached_cus.load(std::memory_order_relaxed);
     if (!cus) {
@@ -1074,23 +1126,22 @@ moonlab_hip_status_t moonlab_hip_apply_gates_blocked(moonlab_hip_state_t *s, con
     // keeps that fetch inside the buffer
     if (reg) ops.push_back(BOp{});
     BOp *d_ops = nullptr;
-    hipError_t e = hipMallocAsync((void **)&d_ops, ops.size() * sizeof(BOp), st);
-    if (e == hipSuccess) e = hipMemcpyAsync(d_ops, ops.data(), ops.size() * sizeof(BOp), hipMemcpyHostToDevice, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);   // `ops` is a local vector
-    void *amps = moonlab_hip_state_device_ptr(s);
+    hipError_t e = upload(ops, &d_ops, st);
     const int lds_tile = tune.blocked_tile_bits == 0 || tune.blocked_tile_bits > 12 ? 12 : tune.blocked_tile_bits;
     for (size_t i = 0; e == hipSuccess && i < passes.size(); i++)
         e = reg ? launch_reg_pass(amps, prec, n, passes[i], d_ops, reg_bits, st)
                 : launch_tile_pass(amps, prec, n, passes[i], d_ops, cus, tune.blocked_threads, lds_tile, st);
     if (d_ops) hipFreeAsync(d_ops, st);
-    if (e == hipErrorOutOfMemory) return MOONLAB_HIP_ERR_OUT_OF_MEMORY;
-    return e == hipSuccess ? MOONLAB_HIP_OK : MOONLAB_HIP_ERR_DRIVER;
+    return status(e);
 }
 
 int moonlab_hip_blocked_pass_count(const moonlab_hip_gate_t *g, int ng, int n, int precision)
 {
     if (ng < 0 || (ng > 0 && !g) || n < 1 || n > 40) return MOONLAB_HIP_ERR_BAD_ARG;
     if (precision != MOONLAB_HIP_C128 && precision != MOONLAB_HIP_C64) return MOONLAB_HIP_ERR_BAD_ARG;
+    std::vector<FPass> fp;
+    std::vector<FOp> prog;
+    if (plan_frames(g, ng, n, precision, gate_tuning(), fp, prog)) return (int)fp.size();
     std::vector<GOp> gops;
     if (!lower(g, ng, n, gops)) return MOONLAB_HIP_ERR_INVALID_QUBIT;
     std::vector<BPass> passes;

@@ -1,0 +1,36 @@
+// frame_plan.h -- host planner of the Pauli-rotation engine.
+#pragma once
+
+#include <stdint.h>
+
+#include <complex>
+#include <vector>
+
+#include "../../include/moonlab_hip_statevec.h"
+#include "frame_program.h"
+
+namespace mlx {
+
+enum FGateKind : int8_t { FG_ROT, FG_CX, FG_CZ, FG_SWAP, FG_X, FG_Z };
+
+// A lowered gate: a rotation scale (1 - i t P), P = i^|x&z| X^x Z^z, or a
+// frame gate (CX: control a, target b; CZ, SWAP: a, b; X, Z: a).
+struct FGate {
+    FGateKind kind;
+    int8_t    a, b;
+    uint64_t  x, z;
+    double    t, scale;
+};
+
+// Gate list -> rotations and frame gates, and the global phase they leave
+// out.  False on an invalid gate or qubit or a parameter that is not finite.
+bool frame_lower(const moonlab_hip_gate_t *g, int ng, int n, std::vector<FGate> &out, std::complex<double> &phase);
+
+// Plan passes over tile sets of tb qubits (n <= tb: one pass over max(n, 4)
+// qubits) that keep the lowest anchor_bits qubits.  amp_bytes: 16 or 8.
+// lookahead: seeds per tile set and register basis (0: greedy).  Passes and
+// units are appended.
+void frame_plan(const std::vector<FGate> &gates, std::complex<double> phase, int n, int tb, int anchor_bits,
+                int amp_bytes, int lookahead, std::vector<FPass> &passes, std::vector<FOp> &prog);
+
+}  // namespace mlx
