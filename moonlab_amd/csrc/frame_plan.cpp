@@ -8,6 +8,7 @@
 #include "frame_plan.h"
 
 #include <math.h>
+#include <stddef.h>
 #include <string.h>
 
 #include <algorithm>
@@ -602,6 +603,7 @@ class PassBuilder {
         rest_.resize(rots_.size());
         for (size_t i = 0; i < rest_.size(); i++) rest_[i] = (int)i;
         double grown = 0.0;
+        size_t hpos = 0;   // header of the latest phase
         while (!rest_.empty()) {
             // candidates: the current layout (no exchange through LDS), a
             // basis grown greedily, and bases seeded by the next pending directions
@@ -645,11 +647,19 @@ class PassBuilder {
             set_pivots(L);
             FPhase h{};
             h.relayout = !same(L, cur);
+            for (int j = 0; j < 16; j++) h.from[j] = slot_bytes(reg_index(cur, j), bytes_);
             if (h.relayout) cur = L;
-            for (int i = 0; i < kFrameRegBits; i++) h.pivots |= (uint32_t)cur.piv[i] << (5 * i);
+            for (int i = 0; i < kFrameRegBits; i++) h.nm[i] = 0u - (1u << cur.piv[i]);
             for (int j = 0; j < 16; j++) h.off[j] = slot_bytes(reg_index(cur, j), bytes_);
-            const size_t hpos = prog_.size();
-            prog_.resize(hpos + 3);
+            // in the layout of the phase before (its scan stopped at the
+            // planning bound): its rotations go on
+            const bool join = !h.relayout && P.nphases > 0;
+            if (!join) {
+                hpos = prog_.size();
+                prog_.resize(hpos + kFPhaseUnits);
+                memcpy((void *)&prog_[hpos], &h, sizeof h);
+                P.nphases++;
+            }
             for (int i : best_take_) {
                 const LRot &o = rots_[(size_t)i];
                 prog_.push_back(encode(o, cur));
@@ -662,9 +672,8 @@ class PassBuilder {
                     grown -= floor(grown);
                 }
             }
-            h.nops = (int32_t)(prog_.size() - hpos - 3);
-            memcpy((void *)&prog_[hpos], &h, sizeof h);
-            P.nphases++;
+            const int32_t nops = (int32_t)(prog_.size() - hpos) - kFPhaseUnits;
+            memcpy((char *)&prog_[hpos] + offsetof(FPhase, nops), &nops, sizeof nops);
             rest_.swap(best_def_);
         }
     }
@@ -807,10 +816,11 @@ class PassBuilder {
         };
         FOut o{};
         const uint32_t xb = slot_bytes(col(b0), bytes_);
+        for (int j = 0; j < 16; j++) o.from[j] = slot_bytes(reg_index(cur, j), bytes_);
         for (int j = 0; j < 16; j++) o.off[j] = xb ^ slot_bytes(col((uint32_t)j << tbits), bytes_);
         for (int t = 0; t < tbits; t++) o.col[t] = slot_bytes(col(1u << t), bytes_);
         const size_t at = prog_.size();
-        prog_.resize(at + 4);
+        prog_.resize(at + kFOutUnits);
         memcpy((void *)&prog_[at], &o, sizeof o);
         P.shift = (int32_t)prog_.size();
         for (int i = 0; i < nb; i++)

@@ -51,24 +51,29 @@ static_assert(sizeof(FOp) == 32, "program unit");
 // A phase: a layout of the tile over (register value j, thread t), stored
 // index x = R j + T t, and the rotations that run in it.  R's four columns
 // are the directions the rotations pair values across; T inserts zeros at the
-// four pivot positions.  Followed by `nops` rotations.
+// four pivot positions p, ascending: x + (x & nm), nm = -(1 << p), per pivot.
+// Followed by `nops` >= 1 rotations.  Only a pass's first phase may stay in
+// the layout it is entered in (the IO layout).
 struct FPhase {
     int32_t  nops;
-    int32_t  relayout;      // 0: the layout is the previous one
-    uint32_t pivots;        // 5 bits each, ascending
-    uint32_t pad[5];
-    uint32_t off[16];       // LDS byte offset of register value j: slot(R j)
+    int32_t  relayout;
+    uint32_t nm[4];
+    uint32_t pad[2];
+    uint32_t from[16];      // LDS byte offset of register value j before: slot(R_before j)
+    uint32_t off[16];       // and in this layout: slot(R j)
 };
-static_assert(sizeof(FPhase) == 3 * sizeof(FOp), "phase header units");
+constexpr int kFPhaseUnits = 5;
+static_assert(sizeof(FPhase) == kFPhaseUnits * sizeof(FOp), "phase header units");
 
-// Output layout (after the last phase) when FP_OUT is set, then ncross sign
-// terms and nshift index shifts that depend on qubits outside the tile.
+// Output layout (after the last phase) when FP_OUT is set.
 struct FOut {
-    uint32_t off[16];       // LDS byte offset of output register value j (constant shift included)
+    uint32_t from[16];      // LDS byte offset of register value j in the last layout
+    uint32_t off[16];       // of output register value j (constant shift included)
     uint32_t col[12];       // of thread bit b
     uint32_t pad[4];
 };
-static_assert(sizeof(FOut) == 4 * sizeof(FOp), "output layout units");
+constexpr int kFOutUnits = 6;
+static_assert(sizeof(FOut) == kFOutUnits * sizeof(FOp), "output layout units");
 
 // parity(gmask & base) shifts the stored index: XOR `off` into the LDS byte
 // offset an output value is read from.

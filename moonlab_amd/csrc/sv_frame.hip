@@ -50,13 +50,13 @@ __global__ __launch_bounds__(1 << (TB - 4), WPE) void k_frame_pass(cplx_t<R> *__
     const uint64_t lo = dlo[tid & 63];
     const int hi0 = tid >> 6;
     const FrameThread ft = frame_thread(P, prog, tid, TB - 4, true);
-    cplx_t<R> v[16], pre[16];
+    typename FVec<R>::t v[16], pre[16];
     const TileWalk walk = tile_walk(ntiles);
     uint64_t ti = walk.t;
     if (ti < walk.end) {
         const uint64_t b0 = frame_base<TB>(ti, P) | lo;
 #pragma unroll
-        for (int j = 0; j < 16; j++) pre[j] = ld<NT>(&a[b0 | dhi[hi0 + HSTEP * j]]);
+        for (int j = 0; j < 16; j++) pre[j] = frame_ld<R, NT>(&a[b0 | dhi[hi0 + HSTEP * j]]);
     }
     for (; ti < walk.end; ti += walk.step) {
 #pragma unroll
@@ -65,12 +65,12 @@ __global__ __launch_bounds__(1 << (TB - 4), WPE) void k_frame_pass(cplx_t<R> *__
         if (nti < walk.end) {
             const uint64_t b1 = frame_base<TB>(nti, P) | lo;
 #pragma unroll
-            for (int j = 0; j < 16; j++) pre[j] = ld<NT>(&a[b1 | dhi[hi0 + HSTEP * j]]);
+            for (int j = 0; j < 16; j++) pre[j] = frame_ld<R, NT>(&a[b1 | dhi[hi0 + HSTEP * j]]);
         }
         const uint64_t base = frame_base<TB>(ti, P);
-        frame_tile<R, true>(t, v, P, prog, ft, base, tid, TB, true);
+        frame_tile<R>(t, v, P, prog, ft, base, tid, TB);
 #pragma unroll
-        for (int j = 0; j < 16; j++) st<NT>(&a[(base | lo) | dhi[hi0 + HSTEP * j]], v[j]);
+        for (int j = 0; j < 16; j++) frame_st<R, NT>(&a[(base | lo) | dhi[hi0 + HSTEP * j]], v[j]);
     }
 }
 
@@ -83,13 +83,13 @@ __global__ __launch_bounds__(128) void k_frame_small(cplx_t<R> *__restrict__ a, 
     const int tid = threadIdx.x, threads = 1 << (P.nbits - kFrameRegBits);
     const bool active = tid < threads;
     const FrameThread ft = frame_thread(P, prog, tid, P.nbits - kFrameRegBits, active);
-    cplx_t<R> v[16];
+    typename FVec<R>::t v[16];
 #pragma unroll
-    for (int j = 0; j < 16; j++) v[j] = active ? a[tid + threads * j] : cplx_t<R>{R(0), R(0)};
-    frame_tile<R, false>(t, v, P, prog, ft, 0, tid, P.nbits, active);
+    for (int j = 0; j < 16; j++) v[j] = active ? frame_ld<R, false>(&a[tid + threads * j]) : typename FVec<R>::t{R(0), R(0)};
+    frame_tile<R>(t, v, P, prog, ft, 0, tid, P.nbits);
 #pragma unroll
     for (int j = 0; j < 16; j++)
-        if (active) a[tid + threads * j] = v[j];
+        if (active) frame_st<R, false>(&a[tid + threads * j], v[j]);
 }
 
 // Tiles per workgroup: short-lived workgroups that the dispatcher keeps
@@ -101,7 +101,7 @@ hipError_t run_frame_pass(void *amps, const FPass &P, const FOp *d_prog, uint64_
 {
     // complex64: two 512-thread workgroups fit a CU's LDS, 4 waves per SIMD
     // (at most 128 registers); complex128 has 2 waves per SIMD by its LDS
-    constexpr int WPE = (sizeof(R) == 4 && TB == 13) ? 4 : 1;
+    constexpr int WPE = sizeof(R) == 4 ? 4 : 2;
     const unsigned grid = (unsigned)(ntiles >= kTilesPerGroup ? ntiles / kTilesPerGroup : 1);
     k_frame_pass<R, NT, TB, WPE><<<grid, 1 << (TB - 4), 0, st>>>((cplx_t<R> *)amps, P, d_prog, ntiles);
     return hipGetLastError();

@@ -36,13 +36,15 @@ static void run_tile(std::vector<cd> &tile, const FPass &P, const std::vector<FO
     };
     size_t p = (size_t)P.first;
     for (int ph = 0; ph < P.nphases; ph++) {
-        FPhase h; memcpy(&h, &prog[p], sizeof h); p += 3;
+        FPhase h; memcpy(&h, &prog[p], sizeof h); p += kFPhaseUnits;
+        if (!h.relayout && ph) die("a later phase without a layout change");
+        if (memcmp(h.from, off, sizeof off)) die("header does not start from the layout before");
         g_phases++;
         if (h.nops < 1) die("empty phase");
         if (h.relayout) {
             g_relayouts++;
             std::vector<uint32_t> ns(TH);
-            for (int t = 0; t < TH; t++) { int x = t; for (int i = 0; i < 4; i++) x = (int)ins0((uint64_t)x, (h.pivots >> (5 * i)) & 31); ns[t] = slot(x); }
+            for (int t = 0; t < TH; t++) { int x = t; for (int i = 0; i < 4; i++) x += x & (int)h.nm[i]; ns[t] = slot(x); }
             change(ns, h.off); memcpy(off, h.off, sizeof off); sl = ns;
         }
         for (int q = 0; q < h.nops; q++, p++) {
@@ -79,6 +81,7 @@ static void run_tile(std::vector<cd> &tile, const FPass &P, const std::vector<FO
         }
     if (P.flags & FP_OUT) {
         FOut o; memcpy(&o, &prog[(size_t)P.out], sizeof o);
+        if (memcmp(o.from, off, sizeof off)) die("output does not start from the last layout");
         uint32_t sh = 0;
         for (int c = 0; c < P.nshift; c++) { FShift x; memcpy(&x, &prog[(size_t)(P.shift + c)], sizeof x); g_shift++; if (par(x.gmask & base)) sh ^= x.off; }
         std::vector<uint32_t> ns(TH);
