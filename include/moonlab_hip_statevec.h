@@ -179,7 +179,7 @@ MOONLAB_API moonlab_hip_status_t moonlab_hip_apply_gates_blocked(moonlab_hip_sta
  * only, no device needed), or a negative moonlab_hip_status_t value. */
 MOONLAB_API int moonlab_hip_blocked_pass_count(const moonlab_hip_gate_t *gates, int num_gates, int n,
                                                int precision);
-/* Addition: tile (11, 12 or 13 qubits; the register-phase engine uses 12 or
+/* Addition: tile (11, 12 or 13 qubits; the register engines use 12 or
  * 13 -- by default 12 for complex128 and 13 for complex64 -- the LDS op engine
  * 11 or 12) and the LDS op engine's workgroup size (256 or 512) of the
  * blocked path; 0 keeps a value, tile_bits -1 restores the default by
@@ -187,12 +187,14 @@ MOONLAB_API int moonlab_hip_blocked_pass_count(const moonlab_hip_gate_t *gates, 
  * reorder commuting gates, so results agree to rounding; one setting gives
  * the same result on every call. */
 MOONLAB_API moonlab_hip_status_t moonlab_hip_set_blocked_tuning(int tile_bits, int threads);
-/* Addition: engine of the blocked path for states of at least 12 qubits:
- * 0 = register phases (default: each thread keeps 16 tile amplitudes in
- * registers, LDS only changes which tile qubits those are), 1 = LDS ops (one
- * LDS sweep per op or register segment), 2 = register phases (same as 0),
- * 3 = register phases with 8 amplitudes per thread (twice the waves, three
- * register qubits per phase).  Smaller states use the LDS engine. */
+/* Addition: engine of the blocked path: 0 = Pauli rotations (default; states
+ * of at least 4 qubits: Clifford gates move a frame, the rest are rotations on
+ * 16 amplitudes per thread; lists with a parameter that is not finite take
+ * engine 2), 1 = LDS ops (one LDS sweep per op or register segment), 2 =
+ * register phases (one op per gate, each thread keeps 16 tile amplitudes in
+ * registers), 3 = register phases with 8 amplitudes per thread (twice the
+ * waves, three register qubits per phase).  The register phases need 12
+ * qubits; smaller states use the LDS ops there. */
 MOONLAB_API moonlab_hip_status_t moonlab_hip_set_blocked_engine(int engine);
 
 /* Addition: how the blocked path's planner picks each pass's tile set and

@@ -1,7 +1,11 @@
-// batch.cpp -- host planner and C ABI of the persistent batch engine.
+// batch.cpp -- host side and C ABI of the persistent batch engine, and the
+// cache-blocked path of one state.
 //
-// Planning per circuit (independent of the rest of the batch, so a
-// circuit's results are the same alone and in any mix):
+// Circuits are planned as Pauli rotations (frame_plan.h), each independently
+// of the rest of the batch, so its results are the same alone and in any mix.
+//
+// The op planner below serves the blocked path's selectable op engines
+// (sv_regpass.hip, batch.hip: k_tile_pass):
 //   1. single-qubit gates fold into one FP64 2x2 per qubit until a
 //      multi-qubit gate touches that qubit (the reference's run-length 1q
 //      fusion, src/optimization/fusion/fusion.c:247-292); a folded diagonal
@@ -40,10 +44,11 @@ namespace mlx {
 hipError_t launch_tile_pass(void *amps, int prec, int n, const BPass &P, const BOp *d_ops, int cus, int threads,
                             int tile_bits, hipStream_t st);
 hipError_t launch_reg_pass(void *amps, int prec, int n, const BPass &P, const BOp *d_ops, int reg_bits, hipStream_t st);
-hipError_t launch_frame_pass(void *amps, int prec, int n, const FPass &P, const FOp *d_prog, hipStream_t st);
+hipError_t launch_frame_pass(void *amps, int prec, int n, const FPass &P, const FPass *d_pass, const FOp *d_prog,
+                             hipStream_t st);
 
-hipError_t launch_batch(const BInst *insts, const int32_t *order, int ninst, int *counter, const BPass *passes,
-                        const BOp *ops, double2 *scratch, uint64_t slot_amps, double *tile_scratch,
+hipError_t launch_batch(const BInst *insts, const int32_t *order, int n128, int n64, int *counter, const FPass *passes,
+                        const FOp *prog, double2 *scratch, uint64_t slot_amps, double *tile_scratch,
                         uint64_t tile_slot, const double *draws, double *obs, uint64_t *outcomes,
                         const PauliT *terms, void *state_out, int grid, hipStream_t st);
 
@@ -729,6 +734,10 @@ struct moonlab_mi355x_batch {
     hipGraphExec_t  gexec = nullptr;
     std::vector<uint64_t> gkey;       // shape of gexec
     std::vector<uint64_t> last_key;   // shape of the previous run
+    // room for passes and program units in the arena: they depend on the
+    // angles a little (a rotation past pi/2 leaves a Pauli to the frame), and
+    // a fixed room keeps the shape, so that new angles replay the graph
+    size_t      room_passes = 0, room_ops = 0;
     // state and overlap buffers of the geometric-tensor calls (vqe.cpp)
     void       *d_states = nullptr;
     size_t      states_cap = 0;
@@ -777,10 +786,15 @@ void on_threads(int nthreads, F &&fn)
     for (std::thread &x : th) x.join();
 }
 
-int host_threads(int work_items)
+// Host threads for `gates` gates to build or plan in at most `parts` parts:
+// starting a thread costs 10-20 us, planning a gate about 0.2 us, so one per
+// 1000 gates (193 circuits of 140 gates on 16 threads spent most of a
+// millisecond starting them three times over).
+int host_threads(size_t gates, int parts)
 {
     const unsigned hw = std::thread::hardware_concurrency();
-    return work_items < 64 ? 1 : (int)std::min<unsigned>(16u, hw ? hw : 1u);
+    const size_t most = std::min<size_t>({16u, hw ? hw : 1u, (size_t)std::max(parts, 1)});
+    return (int)std::min(most, 1 + gates / 1000);
 }
 
 int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int count,
@@ -805,15 +819,17 @@ int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int
     // which are then concatenated in circuit order with their offsets shifted.
     struct Chunk {
         int                lo = 0, hi = 0;
-        std::vector<BPass> passes;
-        std::vector<BOp>   ops;
+        std::vector<FPass> passes;
+        std::vector<FOp>   ops;
         bool               bad = false;
-        bool               internal = false;
     };
-    const int nthreads = host_threads(count);
+    size_t total_gates = 0;
+    for (int i = 0; i < count; i++) total_gates += items[i].num_gates > 0 ? (size_t)items[i].num_gates : 0;
+    const int nthreads = host_threads(total_gates, count);
     std::vector<Chunk> chunks((size_t)nthreads);
     auto plan_chunk = [&](Chunk &c) {
-        std::vector<GOp> gops;
+        std::vector<FGate> gates;
+        cd phase;
         for (int i = c.lo; i < c.hi; i++) {
             const moonlab_mi355x_batch_item_t &it = items[i];
             const int n = it.num_qubits;
@@ -823,27 +839,21 @@ int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int
                 c.bad = true;
                 return;
             }
-            gops.clear();
-            if (!lower(it.gates, it.num_gates, n, gops)) {
+            gates.clear();
+            if (!frame_lower(it.gates, it.num_gates, n, gates, phase, true)) {
                 c.bad = true;
                 return;
             }
             BInst &I = insts[(size_t)i];
             I.n = n;
             I.prec = it.precision;
-            I.tile_bits = n < tbmax ? n : tbmax;
-            I.first_pass = (int)c.passes.size();   // chunk-local (passes and ops) until placed
-            plan_passes(gops, n, I.tile_bits, kSegRegsBatch, c.passes, c.ops);
+            I.tile_bits = std::max(n < tbmax ? n : tbmax, kFrameRegBits);
+            I.first_pass = (int)c.passes.size();   // chunk-local (passes and units) until placed
+            frame_plan(gates, phase, n, tbmax, 4, it.precision == MOONLAB_HIP_C64 ? 8 : 16, kBatchLookahead, c.passes,
+                       c.ops);
             I.num_passes = (int)c.passes.size() - I.first_pass;
-            for (int p = I.first_pass; p < I.first_pass + I.num_passes; p++) {
-                const BPass &P = c.passes[(size_t)p];
-                if (!segments_fit_staging(c.ops.data() + P.first_op, P.num_ops)) {
-                    c.internal = true;   // a planner bug: the staged op loop could not advance
-                    return;
-                }
-            }
             // longest first: sweeps x amplitudes (resident circuits: ops x tile)
-            const double sweeps = n > I.tile_bits ? (double)(I.num_passes + 2) * 4.0 : 0.2 * (double)gops.size();
+            const double sweeps = n > I.tile_bits ? (double)(I.num_passes + 2) * 4.0 : 0.2 * (double)gates.size();
             cost[(size_t)i] = {-(sweeps * (double)(1ull << n)), i};
         }
     };
@@ -859,7 +869,6 @@ int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int
     for (int t = 0; t < nthreads; t++) {
         const Chunk &c = chunks[(size_t)t];
         if (c.bad) return MOONLAB_SCHED_BAD_ARG;
-        if (c.internal) return MOONLAB_SCHED_INTERNAL;
         pass_base[(size_t)t] = total_passes;
         op_base[(size_t)t] = total_ops;
         total_passes += c.passes.size();
@@ -893,8 +902,14 @@ int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int
         if (n > I.tile_bits && n > max_big) max_big = n;
     }
     std::stable_sort(cost.begin(), cost.end());
-    std::vector<int32_t> order((size_t)count);
-    for (int i = 0; i < count; i++) order[(size_t)i] = cost[(size_t)i].second;
+    std::vector<int32_t> order;   // complex128 circuits, then complex64 ones, each longest first
+    order.reserve((size_t)count);
+    int n128 = 0;
+    for (const int prec : {MOONLAB_HIP_C128, MOONLAB_HIP_C64}) {
+        for (int i = 0; i < count; i++)
+            if (insts[(size_t)cost[(size_t)i].second].prec == prec) order.push_back(cost[(size_t)i].second);
+        if (prec == MOONLAB_HIP_C128) n128 = (int)order.size();
+    }
 
     // grid: as many workgroups as fit, bounded by the HBM slots large circuits need
     int grid = b->num_cus * b->wg_per_cu;
@@ -914,13 +929,17 @@ int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int
     const size_t scratch_bytes = (size_t)grid * (slot_amps * 16 + tile_slot * 8) + 256;
     if (grow_dev(&b->d_scratch, &b->scratch_cap, scratch_bytes)) return MOONLAB_SCHED_OOM;
 
-    // program arena layout
+    auto room = [](size_t need, size_t &have) {
+        if (need > have || 2 * need + 128 < have) have = need + need / 8 + 64;
+        return have;
+    };
+    // program arena layout; a spare unit: the kernel fetches one ahead
     size_t off = 0;
     auto place = [&](size_t bytes) { const size_t o = off; off = (off + bytes + 255) / 256 * 256; return o; };
     const size_t o_inst = place(insts.size() * sizeof(BInst));
     const size_t o_order = place(order.size() * sizeof(int32_t));
-    const size_t o_pass = place((total_passes + 1) * sizeof(BPass));
-    const size_t o_ops = place((total_ops + 1) * sizeof(BOp));
+    const size_t o_pass = place(room(total_passes, b->room_passes) * sizeof(FPass));
+    const size_t o_ops = place(room(total_ops + 1, b->room_ops) * sizeof(FOp));
     const size_t o_draw = place((draws.size() + 1) * sizeof(double));
     const size_t o_pauli = place((pauli.size() + 1) * sizeof(PauliT));
     const size_t prog_bytes = off;
@@ -935,18 +954,24 @@ int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int
     memcpy(hp + o_inst, insts.data(), insts.size() * sizeof(BInst));
     memcpy(hp + o_order, order.data(), order.size() * sizeof(int32_t));
     {
-        BPass *hpass = (BPass *)(hp + o_pass);
-        BOp *hops = (BOp *)(hp + o_ops);
+        FPass *hpass = (FPass *)(hp + o_pass);
+        FOp *hops = (FOp *)(hp + o_ops);
         auto place_chunk = [&](int t) {
             const Chunk &c = chunks[(size_t)t];
-            BPass *dst = hpass + pass_base[(size_t)t];
+            FPass *dst = hpass + pass_base[(size_t)t];
+            const int32_t at = (int32_t)op_base[(size_t)t];
             for (size_t k = 0; k < c.passes.size(); k++) {
                 dst[k] = c.passes[k];
-                dst[k].first_op += (int32_t)op_base[(size_t)t];
+                for (int32_t *u : {&dst[k].first, &dst[k].out, &dst[k].cross, &dst[k].shift, &dst[k].table})
+                    if (*u >= 0) *u += at;
             }
-            if (!c.ops.empty()) memcpy(hops + op_base[(size_t)t], c.ops.data(), c.ops.size() * sizeof(BOp));
+            if (!c.ops.empty()) memcpy((void *)(hops + op_base[(size_t)t]), c.ops.data(), c.ops.size() * sizeof(FOp));
         };
-        on_threads(nthreads, place_chunk);
+        if (total_ops > 65536) {
+            on_threads(nthreads, place_chunk);
+        } else {   // 2 MiB or less: copied sooner than threads start
+            for (int t = 0; t < nthreads; t++) place_chunk(t);
+        }
     }
     if (!draws.empty()) memcpy(hp + o_draw, draws.data(), draws.size() * sizeof(double));
     if (!pauli.empty()) memcpy(hp + o_pauli, pauli.data(), pauli.size() * sizeof(PauliT));
@@ -960,8 +985,8 @@ int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int
     auto step = [&]() -> hipError_t {
         hipError_t r = hipMemcpyAsync(dp, hp, prog_bytes, hipMemcpyHostToDevice, b->stream);
         if (r == hipSuccess)
-            r = launch_batch((const BInst *)(dp + o_inst), (const int32_t *)(dp + o_order), count, b->d_counter,
-                             (const BPass *)(dp + o_pass), (const BOp *)(dp + o_ops), scratch, slot_amps,
+            r = launch_batch((const BInst *)(dp + o_inst), (const int32_t *)(dp + o_order), n128, count - n128, b->d_counter,
+                             (const FPass *)(dp + o_pass), (const FOp *)(dp + o_ops), scratch, slot_amps,
                              tile_scratch, tile_slot, (const double *)(dp + o_draw), (double *)(dr + r_obs),
                              (uint64_t *)(dr + r_out), (const PauliT *)(dp + o_pauli), d_state, grid, b->stream);
         if (r == hipSuccess) r = hipMemcpyAsync(b->h_res, dr, res_bytes, hipMemcpyDeviceToHost, b->stream);
@@ -972,7 +997,7 @@ int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int
                                        (uint64_t)(uintptr_t)hp, (uint64_t)(uintptr_t)b->h_res,
                                        (uint64_t)(uintptr_t)b->d_scratch, prog_bytes, res_bytes, o_inst, o_order,
                                        o_pass, o_ops, o_draw, r_obs, r_out, (uint64_t)count, (uint64_t)grid,
-                                       slot_amps, tile_slot, o_pauli, (uint64_t)(uintptr_t)d_state};
+                                       slot_amps, tile_slot, o_pauli, (uint64_t)(uintptr_t)d_state, (uint64_t)n128};
     // A shape seen for the first time runs eagerly; its second run is captured
     // and launched as a graph; later runs of it replay that graph.
     bool replayed = false;
@@ -1096,9 +1121,15 @@ moonlab_hip_status_t moonlab_hip_apply_gates_blocked(moonlab_hip_state_t *s, con
     std::vector<FOp> prog;
     if (plan_frames(g, ng, n, prec, tune, fp, prog)) {
         if (fp.empty()) return MOONLAB_HIP_OK;
+        // program and passes in one upload
+        const size_t units = prog.size(), tail = (fp.size() * sizeof(FPass) + sizeof(FOp) - 1) / sizeof(FOp);
+        prog.resize(units + tail);
+        memcpy((void *)&prog[units], fp.data(), fp.size() * sizeof(FPass));
         FOp *d_prog = nullptr;
         hipError_t e = upload(prog, &d_prog, st);
-        for (size_t i = 0; e == hipSuccess && i < fp.size(); i++) e = launch_frame_pass(amps, prec, n, fp[i], d_prog, st);
+        const FPass *d_pass = (const FPass *)(d_prog + units);
+        for (size_t i = 0; e == hipSuccess && i < fp.size(); i++)
+            e = launch_frame_pass(amps, prec, n, fp[i], d_pass + i, d_prog, st);
         if (d_prog) hipFreeAsync(d_prog, st);
         return status(e);
     }
@@ -1275,8 +1306,11 @@ int moonlab_mi355x_hea_tfim_energies(moonlab_mi355x_batch_t *b, const moonlab_mi
         zoff += (size_t)(n > 1 ? n - 1 : 1);
         xoff += (size_t)n;
     }
-    // the ansatz gate lists (vqe.c:764-781 layer order), built on host threads
-    const int nthreads = host_threads(count);
+    // the ansatz gate lists (vqe.c:764-781 layer order), built on host
+    // threads when there are many (building a gate costs a hundredth of planning it)
+    size_t total = 0;
+    for (int i = 0; i < count; i++) total += (size_t)inst[i].num_layers * (size_t)(3 * inst[i].num_qubits);
+    const int nthreads = host_threads(total / 64, count);
     on_threads(nthreads, [&](int t) {
         const int lo = (int)((int64_t)count * t / nthreads), hi = (int)((int64_t)count * (t + 1) / nthreads);
         for (int i = lo; i < hi; i++) {

@@ -1,16 +1,24 @@
 // batch.hip -- one persistent launch that simulates thousands of small,
 // uneven circuits.
 //
-// Each 1024-thread workgroup takes the next circuit from an atomic work queue
-// (the host orders it longest-first) and runs it start to finish:
-//   * n <= tile bits (12): the whole state lives in LDS (64 KiB at
-//     complex128); gates are LDS sweeps; observables and shots are computed
-//     from LDS.  HBM sees only the program and the results.
+// Each 256-thread workgroup takes the next circuit from an atomic work queue
+// (the host orders it longest-first) and runs it start to finish as passes of
+// the Pauli-rotation engine (frame_device.h: 16 tile amplitudes per thread in
+// registers, LDS only for layout changes):
+//   * n <= tile bits (12): the whole state is one tile that never leaves the
+//     registers; HBM sees only the program and the results.
 //   * n > 12: the state lives in the workgroup's HBM slot and every pass
-//     streams it through LDS in 2^12-amplitude tiles (cache blocking): the
-//     host planner packs each run of gates whose non-diagonal qubits fit in a
-//     12-qubit tile set into one pass, so a circuit costs a few HBM sweeps
-//     per layer instead of one per gate.
+//     streams it in 2^12-amplitude tiles, the next tile's loads issued before
+//     the current tile's rotations.
+// Observables are read from the registers and accumulated per thread over all
+// tiles of a circuit; one block reduction at its end.
+//
+// Bound: at two workgroups per CU (64 KiB of LDS each) the rotations' FP64
+// FMAs and LDS exchanges for small circuits, slot traffic for large ones.
+// The engine before it (1024 threads, one LDS sweep and barrier per op or
+// pair of qubits, observables eight at a time) took 83 ms for 4096 ansatz
+// instances of 8..18 qubits and 178 us for 193 of 12 qubits; this one takes
+// 9.6 ms and 53 us.
 // Workgroups never wait on each other; every workgroup exits when the queue
 // is empty, so the grid always drains.
 //
@@ -24,6 +32,7 @@
 #include <atomic>
 
 #include "batch_device.h"
+#include "frame_device.h"
 #include "sv_device.h"
 #include "sv_internal.h"
 
@@ -41,21 +50,19 @@ __device__ __forceinline__ double wsum(double v)
     return v;
 }
 
+// The tile's LDS: layout changes and pair reads of amplitudes, later the CDF
+// of a tile (one padding double per 16).
 struct Shared {
-    double2  tile[1 << kBatchMaxTileBits];   // 64 KiB: state tile, later the CDF
-    uint64_t dlo[64], dhi[64];               // deposit tables of the current tile set
+    double2  tile[1 << kBatchMaxTileBits];   // 64 KiB
     double   red[NW][kMaxObs];               // per-wave partials
-    double   acc[kMaxObs];                   // per-circuit accumulators
     double   res[8];                         // block_reduce results
-    BOp      opbuf[kOpBuf];                  // op descriptors of the current chunk
     int      next;
-    int      flag;
     int      last_nz;
 };
 
 // Block reduction of v[0..nv): wave butterflies, then waves summed in order.
 // Result j lands in out[j] (for j < nv) on every thread after the call.
-__device__ void block_reduce(Shared &sh, double *v, int nv, double *out)
+__device__ __forceinline__ void block_reduce(Shared &sh, double *v, int nv, double *out)
 {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (int j = 0; j < nv; j++) {
@@ -85,7 +92,7 @@ __device__ __forceinline__ int bit_of(int32_t code, int l, uint64_t base)
     return code >= 0 ? (l >> code) & 1 : (int)((base >> (-1 - code)) & 1ull);
 }
 
-template <typename R, int STRIDE = NT>
+template <typename R, int STRIDE>
 __device__ void apply_op(cplx_t<R> *t, int T, const BOp &op, uint64_t base)
 {
     if ((base & op.cg) != op.cg) return;          // a global control is 0 for this whole tile
@@ -272,145 +279,176 @@ __device__ __forceinline__ void run_pass_ops(cplx_t<R> *t, int T, const BOp *ops
     }
 }
 
-// run_pass_ops for the batch kernel: a circuit's op descriptors are read
-// once per tile, and a read straight from device memory would expose a full
-// memory latency per op, so they are staged in LDS kOpBuf at a time (one
-// cooperative 16-byte-per-thread copy, one barrier) and applied from there.
-template <typename R, int NR>
-__device__ void run_pass_ops_staged(Shared &sh, cplx_t<R> *t, int T, const BOp *ops, int nops, uint64_t base)
-{
-    constexpr int kWords = (int)(sizeof(BOp) / sizeof(uint4));
-    static_assert(sizeof(BOp) % sizeof(uint4) == 0, "BOp is copied as 16-byte words");
-    for (int k = 0; k < nops;) {
-        const int cnt = nops - k < kOpBuf ? nops - k : kOpBuf;
-        const uint4 *src = (const uint4 *)(ops + k);
-        uint4 *dst = (uint4 *)sh.opbuf;
-        for (int w = threadIdx.x; w < cnt * kWords; w += NT) dst[w] = src[w];
-        __syncthreads();
-        int j = 0;
-        while (j < cnt) {
-            const BOp &op = sh.opbuf[j];
-            if (op.kind == BOP_SEG) {
-                if (j + 1 + op.lq > cnt) break;   // the segment runs past this chunk: restage from it
-                apply_segment<R, NT, NR>(t, T, &sh.opbuf[j + 1], op.lq, op.cl, base);
-                j += 1 + op.lq;
-            } else {
-                apply_op<R, NT>(t, T, op, base);
-                j++;
-            }
-            __syncthreads();
-        }
-        // every thread has passed the last barrier: opbuf may be overwritten.
-        // The host refuses plans whose segments do not fit one chunk
-        // (segments_fit_staging), so j > 0 here; should one ever reach the
-        // device, its segment is skipped rather than restaged forever.
-        k += j ? j : 1 + sh.opbuf[0].lq;
-    }
-}
-
-__device__ void build_deposit(Shared &sh, const BPass &p)
-{
-    const int tid = threadIdx.x;
-    if (tid < 128) {
-        const int j = tid & 63, hi = tid >> 6;
-        uint64_t o = 0;
-        for (int b = 0; b < 6; b++) {
-            const int qi = hi * 6 + b;
-            if (qi < p.nbits && ((j >> b) & 1)) o |= 1ull << p.qubits[qi];
-        }
-        if (hi) sh.dhi[j] = o;
-        else sh.dlo[j] = o;
-    }
-}
-
 __device__ __forceinline__ uint64_t tile_base(uint64_t t, const BPass &p)
 {
     for (int b = 0; b < p.nbits; b++) t = ins0(t, p.qubits[b]);
     return t;
 }
 
-// Observables of one tile, added into sh.acc (value layout of obs_size()).
-// Measurement pass 0 uses the low `tb` qubits as the tile (tiles in index
-// order: norm, P(1), ZZ and X on the low qubits); pass 1 uses the top `tb`
-// qubits (X on the qubits pass 0 could not pair).  Values are reduced eight
-// at a time to bound register use; the order of every sum is fixed.
+// A tile as the batch kernel walks it: the thread holds tile indices tid +
+// 2^(nb-4) j (IO layout); byte offsets into the circuit's slot (2^24
+// amplitudes at most, so 32 bits hold them).
+struct BatchTile {
+    uint32_t tid;        // of the thread's index bits
+    uint32_t reg[4];     // of register bit i (tile bit nb - 4 + i)
+};
+
 template <typename R>
-__device__ void measure_tile(Shared &sh, const cplx_t<R> *t, int T, int tb, int n, uint64_t base,
-                             int flags, int mpass, double *tile_total)
+__device__ __forceinline__ BatchTile batch_tile(uint64_t mask, int nb, int tid)
 {
-    const int tid = threadIdx.x;
-    const int nzz = n > 1 ? n - 1 : 0;
-    const int xb = 1 + n + nzz;               // first X slot
-    const int nv = xb + n;
-    const int qoff = mpass == 0 ? 0 : n - tb;  // global qubit of local bit 0
-    const int half = T >> 1;
-    for (int c0 = 0; c0 < nv; c0 += 8) {
-        double v[8];
+    constexpr uint32_t B = (uint32_t)sizeof(cplx_t<R>);
+    BatchTile t;
+    t.tid = (uint32_t)frame_deposit((uint64_t)tid & ((1ull << (nb - 4)) - 1ull), mask) * B;
 #pragma unroll
-        for (int j = 0; j < 8; j++) v[j] = 0.0;
-        bool any = false;
-        for (int j = 0; j < 8 && c0 + j < nv; j++) {
-            const int vi = c0 + j;
-            if (vi == 0) any = any || mpass == 0;
-            else if (vi < 1 + n) any = any || (mpass == 0 && (flags & BF_Z));
-            else if (vi < xb) any = any || (mpass == 0 && (flags & BF_ZZ));
-            else any = any || (flags & BF_X);
-        }
-        if (!any) continue;   // uniform across the block
-        if (mpass == 0 && c0 < xb) {
-            for (int l = tid; l < T; l += NT) {
-                const double p = p2<R>(t[l]);
-                const uint64_t full = base | (uint64_t)l;
+    for (int i = 0; i < 4; i++) t.reg[i] = (uint32_t)frame_uniform(frame_deposit(1ull << (nb - 4 + i), mask)) * B;
+    return t;
+}
+
+// byte offset of register value j; base: the tile's, uniform.  The thread's
+// part is made opaque per use: hoisted out of the tile loop, the sixteen sums
+// would hold sixteen registers through the interpreter, which has none to spare.
+__device__ __forceinline__ uint32_t batch_thread(const BatchTile &t)
+{
+    uint32_t x = t.tid;
+    asm volatile("" : "+v"(x));
+    return x;
+}
+__device__ __forceinline__ uint32_t batch_reg(const BatchTile &t, uint32_t base, int j)
+{
+    uint32_t o = base;
 #pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    const int vi = c0 + j;
-                    if (vi == 0) {
-                        v[j] += p;
-                    } else if (vi < 1 + n) {
-                        if ((flags & BF_Z) && ((full >> (vi - 1)) & 1ull)) v[j] += p;
-                    } else if (vi < xb) {
-                        const int q = vi - 1 - n;
-                        if (flags & BF_ZZ) v[j] += (((full >> q) ^ (full >> (q + 1))) & 1ull) ? -p : p;
-                    }
-                }
-            }
-        }
-        if (flags & BF_X) {
+    for (int i = 0; i < 4; i++)
+        if ((j >> i) & 1) o |= t.reg[i];
+    return o;
+}
+template <typename R>
+__device__ __forceinline__ void batch_load(const cplx_t<R> *slot, const BatchTile &t, uint32_t base,
+                                           typename FVec<R>::t (&v)[16])
+{
+    const uint32_t x = batch_thread(t);
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const int vi = c0 + j;
-                if (vi < xb || vi >= nv) continue;
-                const int q = vi - xb, lb = q - qoff;
-                if (lb < 0 || lb >= tb || (mpass == 1 && q < tb)) continue;
-                double s2 = 0.0;
-                for (int pp = tid; pp < half; pp += NT) {
-                    const int i0 = (int)ins0((uint64_t)pp, lb), i1 = i0 | (1 << lb);
-                    s2 += fmar((double)t[i0].x, (double)t[i1].x, (double)t[i0].y * (double)t[i1].y);
-                }
-                v[j] += s2 + s2;
-            }
+    for (int j = 0; j < 16; j++)
+        v[j] = frame_ld<R, false>((const cplx_t<R> *)((const char *)slot + batch_reg(t, base, j) + x));
+}
+template <typename R>
+__device__ __forceinline__ void batch_store(cplx_t<R> *slot, const BatchTile &t, uint32_t base,
+                                            const typename FVec<R>::t (&v)[16])
+{
+    const uint32_t x = batch_thread(t);
+#pragma unroll
+    for (int j = 0; j < 16; j++) frame_st<R, false>((cplx_t<R> *)((char *)slot + batch_reg(t, base, j) + x), v[j]);
+}
+
+// What a thread accumulates over the tiles of the low nb qubits.  Tile-index
+// bits of the thread (0 .. nb-5) enter only through signs, so one total per
+// thread serves every qubit among them; the qubits above the tile take the
+// tile's sums (block_reduce), one qubit per thread.
+struct ObsAcc {
+    double tot = 0.0;
+    double reg[4] = {};         // P(1) of the register bits
+    double rzz[3] = {};         // <ZZ> of neighbouring register bits
+    double link = 0.0;          // Z of register bit 0 (ZZ with the highest thread bit)
+};
+
+template <typename V>
+__device__ __forceinline__ double pr(const V &x)
+{
+    const double r = (double)x.x, i = (double)x.y;
+    return fmar(r, r, i * i);
+}
+
+// norm, P(1) and neighbour <ZZ> sums of one tile into the accumulators; s[0]:
+// the tile's mass, s[1]: its Z of the top register bit
+template <typename V>
+__device__ __forceinline__ void observe_z(const V (&v)[16], ObsAcc &a, bool zz, double (&s)[2])
+{
+    double t = 0.0, r[4] = {}, z3 = 0.0, q[3] = {}, z0 = 0.0;
+#pragma unroll
+    for (int j = 0; j < 16; j++) {
+        const double p = pr(v[j]);
+        t += p;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if ((j >> i) & 1) r[i] += p;
+        if (zz) {
+#pragma unroll
+            for (int i = 0; i < 3; i++) q[i] += (((j >> i) ^ (j >> (i + 1))) & 1) ? -p : p;
+            z0 += (j & 1) ? -p : p;
+            z3 += (j & 8) ? -p : p;
         }
-        const int cnt = nv - c0 < 8 ? nv - c0 : 8;
-        block_reduce(sh, v, cnt, sh.res);
-        if (tid < cnt) sh.acc[c0 + tid] += sh.res[tid];
-        if (c0 == 0 && tile_total && tid == 0) *tile_total = sh.res[0];
-        __syncthreads();
+    }
+    a.tot += t;
+#pragma unroll
+    for (int i = 0; i < 4; i++) a.reg[i] += r[i];
+    if (zz) {
+#pragma unroll
+        for (int i = 0; i < 3; i++) a.rzz[i] += q[i];
+        a.link += z0;
+    }
+    s[0] = t;
+    s[1] = z3;
+}
+
+// 2 Re sum conj(a) b over the pairs across each register bit
+template <typename V>
+__device__ __forceinline__ void observe_x(const V (&v)[16], double (&x)[4])
+{
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        double s = 0.0;
+#pragma unroll
+        for (int j = 0; j < 16; j++) {
+            if ((j >> i) & 1) continue;
+            const V a = v[j], b = v[j | (1 << i)];
+            s += fmar((double)a.x, (double)b.x, (double)a.y * (double)b.y);
+        }
+        x[i] += s + s;
     }
 }
 
-// Pauli strings over one tile of the low tb qubits (tiles in index order):
-// term k adds sum_l Re[conj(a_(i^x)) a_i i^ny (-1)^popcount(i & z)], i =
-// base | l, into out[k].  The partner i ^ x is in the tile when x has no bit
-// at or above tb; otherwise it is read from the circuit's HBM slot (the
-// final state, which measurement does not modify).  Terms are reduced eight
-// at a time; every sum runs in a fixed order, and out[k] is updated by one
-// thread, tile after tile.
+// the thread's values with tile bits b .. b+3 as register bits
 template <typename R>
-__device__ void measure_pauli_tile(Shared &sh, const cplx_t<R> *t, int T, uint64_t base, const cplx_t<R> *slot,
+__device__ __forceinline__ void tile_read(const cplx_t<R> *t, typename FVec<R>::t (&v)[16], int tid, int b)
+{
+    constexpr int B = (int)sizeof(cplx_t<R>);
+    const int lo = tid & ((1 << b) - 1), x0 = lo | ((tid >> b) << (b + 4));
+    const int s0 = lds_slot<B>(x0);
+#pragma unroll
+    for (int j = 0; j < 16; j++) {
+        const cplx_t<R> x = t[s0 ^ lds_slot<B>(j << b)];
+        v[j].x = x.x;
+        v[j].y = x.y;
+    }
+}
+
+template <typename R>
+__device__ __forceinline__ void tile_write(cplx_t<R> *t, const typename FVec<R>::t (&v)[16], int tid, int nb)
+{
+    constexpr int B = (int)sizeof(cplx_t<R>);
+    const int s0 = lds_slot<B>(tid);
+#pragma unroll
+    for (int j = 0; j < 16; j++) t[s0 ^ lds_slot<B>(j << (nb - 4))] = cplx_t<R>{v[j].x, v[j].y};
+}
+
+// Pauli strings over one tile of the low tb qubits (tiles in index order, the
+// tile's amplitudes in LDS): term k adds sum_l Re[conj(a_(i^x)) a_i i^ny
+// (-1)^popcount(i & z)], i = base | l, into out[k].  The partner i ^ x is in
+// the tile when x has no bit at or above tb; otherwise it is read from the
+// circuit's HBM slot (the final state, which measurement does not modify).
+// Terms are reduced eight at a time; every sum runs in a fixed order, and
+// out[k] is updated by one thread, tile after tile.
+template <typename R>
+__device__ __forceinline__ void measure_pauli_tile(Shared &sh, uint32_t lds, int T, uint64_t base, const cplx_t<R> *slot,
                                    const PauliT *terms, int nterms, double *out)
 {
+    using V = typename FVec<R>::t;
+    using SharedV = const __attribute__((address_space(3))) V;
+    constexpr int B = (int)sizeof(V);
     const int tid = threadIdx.x;
     const uint64_t lowmask = (uint64_t)T - 1ull;
+    // an LDS pointer of its own address space: a choice between it and the
+    // slot stays two loads instead of a flat one
+    auto in_tile = [&](int l) { return *(SharedV *)(uintptr_t)(lds + (uint32_t)(lds_slot<B>(l) * B)); };
     for (int c0 = 0; c0 < nterms; c0 += 8) {
         const int cnt = nterms - c0 < 8 ? nterms - c0 : 8;
         double v[8];
@@ -423,8 +461,9 @@ __device__ void measure_pauli_tile(Shared &sh, const cplx_t<R> *t, int T, uint64
             const uint64_t xl = x & lowmask, xh = x & ~lowmask;
             double s = 0.0;
             for (int l = tid; l < T; l += NT) {
-                const cplx_t<R> a = t[l];
-                const cplx_t<R> b = xh == 0 ? t[(uint64_t)l ^ xl] : slot[(base ^ xh) | ((uint64_t)l ^ xl)];
+                const V a = in_tile(l);
+                const V b = xh == 0 ? in_tile(l ^ (int)xl)
+                                    : frame_ld<R, false>(&slot[(base ^ xh) | ((uint64_t)l ^ xl)]);
                 const double br = (double)b.x, bi = (double)b.y, ar = (double)a.x, ai = (double)a.y;
                 const double re = fmar(br, ar, bi * ai);     // Re conj(b) a
                 const double im = fmar(br, ai, -(bi * ar));  // Im conj(b) a
@@ -439,15 +478,17 @@ __device__ void measure_pauli_tile(Shared &sh, const cplx_t<R> *t, int T, uint64
     }
 }
 
-// Inclusive scan of p over T entries in LDS (as doubles), index order.
-__device__ void lds_scan(Shared &sh, double *cdf, int T, double offset)
+__device__ __forceinline__ int cdf_at(int l) { return l + (l >> 4); }
+
+// Inclusive scan of p over T entries in LDS (as doubles, at cdf_at), index order.
+__device__ __forceinline__ void lds_scan(Shared &sh, double *cdf, int T, double offset)
 {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int per = T >= NT ? T / NT : 1;
     const int lo = tid * per;
     double s = 0.0;
     if (lo < T)
-        for (int e = 0; e < per; e++) s += cdf[lo + e];
+        for (int e = 0; e < per; e++) s += cdf[cdf_at(lo + e)];
     double x = s;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
@@ -462,132 +503,302 @@ __device__ void lds_scan(Shared &sh, double *cdf, int T, double offset)
     __syncthreads();
     if (lo < T)
         for (int e = 0; e < per; e++) {
-            run += cdf[lo + e];
-            cdf[lo + e] = run;
+            run += cdf[cdf_at(lo + e)];
+            cdf[cdf_at(lo + e)] = run;
         }
     __syncthreads();
 }
 
-template <typename R>
-__device__ void run_circuit(Shared &sh, const BInst &I, const BPass *passes, const BOp *ops,
-                            double2 *slot_raw, double *tile_sums, const double *draws, double *obs,
-                            uint64_t *outcomes, const PauliT *terms, void *state_out)
+// first l with u < cdf_l, T when there is none
+__device__ __forceinline__ int cdf_find(const double *cdf, int T, double u)
 {
+    int lo = 0, hi = T;
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (u < cdf[cdf_at(mid)]) hi = mid;
+        else lo = mid + 1;
+    }
+    return lo;
+}
+
+template <typename R>
+__device__ __forceinline__ void run_circuit(Shared &sh, uint32_t lds, const BInst &I, const FPass *passes, const FOp *prog, double2 *slot_raw,
+                            double *tile_sums, const double *draws, double *obs, uint64_t *outcomes,
+                            const PauliT *terms, void *state_out)
+{
+    using V = typename FVec<R>::t;
     const int tid = threadIdx.x;
-    const int n = I.n, tb = I.tile_bits, T = 1 << tb;
+    const int n = I.n, nb = I.tile_bits;              // tile bits: 4 at least, above n for tiny circuits
+    const bool resident = n <= nb;
+    const uint64_t ntiles = resident ? 1 : 1ull << (n - nb);
+    const int threads = 1 << (nb - kFrameRegBits);    // that hold amplitudes
+    const bool active = tid < threads;
     cplx_t<R> *t = (cplx_t<R> *)sh.tile;
     cplx_t<R> *slot = (cplx_t<R> *)slot_raw;
-    const uint64_t ntiles = 1ull << (n - tb);
-    const bool resident = n == tb;
-    for (int j = tid; j < kMaxObs; j += NT) sh.acc[j] = 0.0;
 
     // ---- gate passes ----
     for (int pi = 0; pi < I.num_passes; pi++) {
-        const BPass P = passes[I.first_pass + pi];
-        if (!resident) build_deposit(sh, P);
-        __syncthreads();
+        const FConst<FPass> P = (FConst<FPass>)(uintptr_t)(passes + I.first_pass + pi);
+        const uint64_t mask = P->mask;
+        const FrameThread ft = frame_thread(P, prog, tid, nb - kFrameRegBits, active);
+        const BatchTile bt = batch_tile<R>(mask, nb, tid);
+        // threads past the tile's load what thread tid mod threads loads and store nothing
+        const bool load = pi > 0 && !resident, store = !resident && active;
+        V pre[16];
+        uint64_t base = 0;
+        constexpr uint32_t B = (uint32_t)sizeof(cplx_t<R>);
+        if (load) batch_load<R>(slot, bt, 0u, pre);
         for (uint64_t ti = 0; ti < ntiles; ti++) {
-            const uint64_t base = resident ? 0 : tile_base(ti, P);
-            if (pi == 0) {
-                for (int l = tid; l < T; l += NT) t[l] = cplx_t<R>{(base | l) == 0 ? R(1) : R(0), R(0)};
-            } else if (!resident) {
-                for (int l = tid; l < T; l += NT) t[l] = slot[base | sh.dlo[l & 63] | sh.dhi[l >> 6]];
+            // the values live from here to the stores only (a resident
+            // circuit has one pass): kept across passes they cost the
+            // interpreter's fixed registers a second copy, and spills
+            V v[16];
+            const uint64_t next = frame_uniform(frame_step(base, frame_uniform((~mask) & (mask + 1)), mask));
+            if (load) {
+#pragma unroll
+                for (int j = 0; j < 16; j++) v[j] = pre[j];
+                if (ti + 1 < ntiles) batch_load<R>(slot, bt, (uint32_t)next * B, pre);
+            } else {   // the first pass starts from |0..0>
+#pragma unroll
+                for (int j = 0; j < 16; j++) v[j] = V{R(j == 0 && tid == 0 && base == 0), R(0)};
             }
-            __syncthreads();
-            run_pass_ops_staged<R, kSegRegsBatch>(sh, t, T, ops + P.first_op, P.num_ops, base);
-            if (!resident) {
-                for (int l = tid; l < T; l += NT) slot[base | sh.dlo[l & 63] | sh.dhi[l >> 6]] = t[l];
-                __syncthreads();
+            frame_tile<R>(lds, v, P, prog, ft, base, tid, nb);
+            if (store) batch_store<R>(slot, bt, (uint32_t)base * B, v);
+            if (resident) {
+                __syncthreads();   // a layout change may still be read
+                if (active) tile_write<R>(t, v, tid, nb);
             }
+            base = next;
         }
+        __syncthreads();   // the slot's stores are visible to the workgroup
     }
     if (I.num_passes == 0) {   // empty circuit: |0..0>
-        for (uint64_t ti = 0; ti < (resident ? 1 : ntiles); ti++) {
-            for (int l = tid; l < T; l += NT)
-                t[l] = cplx_t<R>{(ti == 0 && l == 0) ? R(1) : R(0), R(0)};
-            __syncthreads();
-            if (!resident)
-                for (int l = tid; l < T; l += NT) slot[(ti << tb) | l] = t[l];
-            __syncthreads();
+        if (resident) {
+            V v[16];
+#pragma unroll
+            for (int j = 0; j < 16; j++) v[j] = V{R(j == 0 && tid == 0), R(0)};
+            if (active) tile_write<R>(t, v, tid, nb);
+        } else {
+            const uint64_t dim = 1ull << n;
+            for (uint64_t i = tid; i < dim; i += NT) slot[i] = cplx_t<R>{R(i == 0), R(0)};
         }
+        __syncthreads();
     }
 
     // ---- the final state, when asked for (geometric-tensor overlaps) ----
     if (I.state_offset >= 0) {
         cplx_t<R> *so = (cplx_t<R> *)state_out + I.state_offset;
+        const uint64_t dim = 1ull << n;
         if (resident) {
-            for (int l = tid; l < T; l += NT) so[l] = t[l];
+            for (uint64_t i = tid; i < dim; i += NT) so[i] = t[lds_slot<(int)sizeof(V)>((int)i)];
         } else {
-            const uint64_t dim = 1ull << n;
             for (uint64_t i = tid; i < dim; i += NT) so[i] = slot[i];
         }
-        __syncthreads();
     }
 
-    // ---- measurement pass 0: tiles of the low tb qubits, index order ----
-    const bool want_shots = I.num_shots > 0;
+    // ---- tiles of the low nb qubits, index order: norm, P(1), <ZZ>, <X> of
+    // those qubits, Pauli strings, tile sums for the shots ----
+    const bool want_shots = I.num_shots > 0, zz = (I.flags & BF_ZZ) != 0, want_x = (I.flags & BF_X) != 0;
+    const int nhigh = resident ? 0 : n - nb, tb = nb - kFrameRegBits;
+    const int nzz = n > 1 ? n - 1 : 0;
     double *pauli_out = obs + I.obs_offset + obs_size(n);
     for (int k = tid; k < I.num_pauli; k += NT) pauli_out[k] = 0.0;
+    ObsAcc acc;
+    double hi = 0.0, hzz = 0.0;   // thread i: P(1) of qubit nb + i; thread 64 + i: <ZZ> of (nb - 1 + i, nb + i)
+    double xs[3][4] = {};         // <X> of the register bits, of tile bits 0..3 and of the four below the register bits
+    const bool lds_tile = want_x || I.num_pauli > 0;
     __syncthreads();
     for (uint64_t ti = 0; ti < ntiles; ti++) {
-        const uint64_t base = ti << tb;
+        V v[16];
+        if (resident) tile_read<R>(t, v, tid & (threads - 1), tb);
+        else
+#pragma unroll
+            for (int j = 0; j < 16; j++)
+                v[j] = frame_ld<R, false>(&slot[(ti << nb) | (uint64_t)((tid & (threads - 1)) + threads * j)]);
+        double s2[2] = {0.0, 0.0};
+        if (active) {
+            observe_z<V>(v, acc, zz, s2);
+            if (want_x) observe_x<V>(v, xs[0]);
+        }
         if (!resident) {
-            for (int l = tid; l < T; l += NT) t[l] = slot[base | l];
+            block_reduce(sh, s2, 2, sh.res);
+            const int i = tid & 63;
+            if (tid < 64 && i < nhigh && ((ti >> i) & 1ull)) hi += sh.res[0];
+            if (tid >= 64 && tid < 128 && i < nhigh) {
+                // the tile's top register bit is the qubit below the first high one
+                const bool flip = (((ti >> i) ^ (i ? ti >> (i - 1) : 0)) & 1ull) != 0;
+                const double x = i ? sh.res[0] : sh.res[1];
+                hzz += flip ? -x : x;
+            }
+            if (want_shots && tid == 0) tile_sums[ti] = sh.res[0];
+        }
+        if (lds_tile) {
+            if (!resident) {
+                if (active) tile_write<R>(t, v, tid, nb);
+                __syncthreads();
+            }
+            if (want_x && active) {
+                // the thread bits' qubits, four at a time; a last set that
+                // overlaps counts its new bits only
+#pragma unroll
+                for (int s = 0; s < 2; s++) {
+                    const int b = 4 * s < tb - 4 ? 4 * s : tb - 4;
+                    if (4 * s >= tb || b < 0) continue;
+                    V w[16];
+                    tile_read<R>(t, w, tid, b);
+                    observe_x<V>(w, xs[1 + s]);
+                }
+                if (tb > 0 && tb < 4) {   // fewer than four thread bits: pairs straight from LDS
+#pragma unroll
+                    for (int q = 0; q < 3; q++) {
+                        if (q >= tb) break;
+                        double s = 0.0;
+                        for (int j = 0; j < 16; j++) {
+                            const int l = tid + threads * j;
+                            if ((l >> q) & 1) continue;
+                            const cplx_t<R> a = t[lds_slot<(int)sizeof(V)>(l)], b = t[lds_slot<(int)sizeof(V)>(l | (1 << q))];
+                            s += fmar((double)a.x, (double)b.x, (double)a.y * (double)b.y);
+                        }
+                        xs[1][q] += s + s;
+                    }
+                }
+            }
+            if (I.num_pauli > 0)
+                measure_pauli_tile<R>(sh, lds, resident ? 1 << n : 1 << nb, ti << nb, slot, terms + I.pauli_offset,
+                                      I.num_pauli, pauli_out);
+            __syncthreads();   // before the next tile is written
+        }
+    }
+    // values of the circuit as per-thread terms, reduced over the block
+    {
+        const int xb = 1 + n + nzz, nv = xb + n;
+        const int lane = tid & 63, wave = tid >> 6;
+        auto put = [&](int k, double x) {
+            const double s = wsum(x);
+            if (lane == 0) sh.red[wave][k] = s;
+        };
+        put(0, acc.tot);
+        for (int q = 0; q < n && q < nb; q++) {
+            if (!(I.flags & BF_Z)) break;
+            double x = 0.0;
+            if (q < tb) x = ((tid >> q) & 1) ? acc.tot : 0.0;
+            else
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    if (q - tb == i) x = acc.reg[i];
+            put(1 + q, x);
+        }
+        if (zz)
+            for (int q = 0; q + 1 < n && q + 1 < nb; q++) {
+                double x = 0.0;
+                if (q + 1 < tb) x = (((tid >> q) ^ (tid >> (q + 1))) & 1) ? -acc.tot : acc.tot;
+                else if (q + 1 == tb) x = ((tid >> q) & 1) ? -acc.link : acc.link;
+                else
+#pragma unroll
+                    for (int i = 0; i < 3; i++)
+                        if (q - tb == i) x = acc.rzz[i];
+                put(1 + n + q, x);
+            }
+        // already block sums, one per thread: three of the four rows hold 0
+        if (tid < nhigh)
+            for (int w = 0; w < NW; w++) sh.red[w][1 + nb + tid] = w ? 0.0 : hi;
+        if (tid >= 64 && tid < 64 + nhigh)
+            for (int w = 0; w < NW; w++) sh.red[w][1 + n + nb - 1 + (tid - 64)] = w ? 0.0 : hzz;
+        if (want_x) {
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (tb + i < n) put(xb + tb + i, xs[0][i]);
+            const int b1 = tb > 4 ? tb - 4 : 0;   // first bit of the second set
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                if (i < tb && i < n) put(xb + i, xs[1][i]);
+                if (tb > 4 && b1 + i >= 4 && b1 + i < n) put(xb + b1 + i, xs[2][i]);
+            }
+        }
+        __syncthreads();
+        // slots that no flag asked for hold 0
+        const int nvis = nhigh && want_x ? xb + nb : nv;   // <X> above the tile follows
+        for (int k = tid; k < nvis; k += NT) {
+            const bool on = k == 0 || (k < 1 + n ? (I.flags & BF_Z) != 0 : k < xb ? zz : want_x);
+            double s = 0.0;
+            if (on)
+                for (int w = 0; w < NW; w++) s += sh.red[w][k];
+            obs[I.obs_offset + k] = s;
+        }
+        __syncthreads();
+    }
+    // ---- <X> of the qubits above the low tile: tiles that keep the lowest
+    // four qubits (runs of 64 bytes or more) and take nb - 4 of the others ----
+    if (want_x && nhigh) {
+        const int xb = 1 + n + nzz, step = nb - 4;
+        for (int q0 = nb; q0 < n; q0 += step) {
+            const int top = q0 + step <= n ? q0 : n - step;   // the set's first qubit after the lowest four
+            BatchTile bt;
+            constexpr uint32_t B = (uint32_t)sizeof(cplx_t<R>);
+            bt.tid = ((uint32_t)(tid & 15) | ((uint32_t)((tid & (threads - 1)) >> 4) << top)) * B;
+#pragma unroll
+            for (int i = 0; i < 4; i++) bt.reg[i] = B << (top + nb - 8 + i);
+            double x0[4] = {}, x1[4] = {};
+            for (uint64_t ti = 0; ti < ntiles; ti++) {
+                const uint64_t base = ((ti & ((1ull << (top - 4)) - 1)) << 4) | ((ti >> (top - 4)) << (top + step));
+                V v[16];
+                batch_load<R>(slot, bt, (uint32_t)base * B, v);
+                if (active) observe_x<V>(v, x0);       // tile bits nb-4 .. nb-1
+                if (nb >= 9) {                         // tile bits nb-8 .. nb-5 (those above the lowest four count)
+                    if (active) tile_write<R>(t, v, tid, nb);
+                    __syncthreads();
+                    if (active) {
+                        V w[16];
+                        tile_read<R>(t, w, tid, nb - 8);
+                        observe_x<V>(w, x1);
+                    }
+                    __syncthreads();
+                }
+            }
+            double x8[8];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                x8[i] = x0[i];
+                x8[4 + i] = x1[i];
+            }
+            block_reduce(sh, x8, 8, sh.res);
+            if (tid < 8) {
+                const int b = tid < 4 ? nb - 4 + tid : nb - 8 + (tid - 4);   // tile bit
+                const int qq = top + b - 4;                                    // its qubit
+                if (b >= 4 && qq >= q0 && (tid < 4 || nb >= 9)) obs[I.obs_offset + xb + qq] = sh.res[tid];
+            }
             __syncthreads();
         }
-        double tt = 0.0;
-        measure_tile<R>(sh, t, T, tb, n, base, I.flags, 0, &tt);
-        if (!resident && tid == 0 && want_shots) tile_sums[ti] = tt;
-        __syncthreads();
-        if (I.num_pauli > 0)
-            measure_pauli_tile<R>(sh, t, T, base, slot, terms + I.pauli_offset, I.num_pauli, pauli_out);
     }
-    // ---- measurement pass 1: X on the qubits above the low tile ----
-    if ((I.flags & BF_X) && !resident) {
-        BPass P;
-        P.nbits = tb;
-        for (int b = 0; b < tb; b++) P.qubits[b] = (int8_t)(n - tb + b);
-        build_deposit(sh, P);
-        __syncthreads();
-        for (uint64_t ti = 0; ti < ntiles; ti++) {
-            const uint64_t base = tile_base(ti, P);
-            for (int l = tid; l < T; l += NT) t[l] = slot[base | sh.dlo[l & 63] | sh.dhi[l >> 6]];
-            __syncthreads();
-            measure_tile<R>(sh, t, T, tb, n, base, BF_X, 1, nullptr);
-        }
-    }
-    const int nv = 1 + n + (n > 1 ? n - 1 : 0) + n;
-    for (int j = tid; j < nv; j += NT) obs[I.obs_offset + j] = sh.acc[j];
 
     // ---- shots: first index with u < cdf_i, else the last nonzero ----
     if (!want_shots) return;
     double *cdf = (double *)sh.tile;
+    const int T = resident ? 1 << n : 1 << nb;
     if (resident) {
-        double pv[(1 << kBatchMaxTileBits) / NT > 0 ? (1 << kBatchMaxTileBits) / NT : 1];
-        int k = 0;
-        for (int l = tid; l < T; l += NT) pv[k++] = p2<R>(t[l]);
+        double pv[16];
+#pragma unroll
+        for (int j = 0; j < 16; j++) {
+            const int l = tid + threads * j;
+            pv[j] = active && l < T ? p2<R>(t[lds_slot<(int)sizeof(V)>(l)]) : 0.0;
+        }
         if (tid == 0) sh.last_nz = -1;
-        __syncthreads();
-        k = 0;
+        __syncthreads();   // the amplitudes are read before the CDF takes their place
         int mylast = -1;
-        for (int l = tid; l < T; l += NT) {
-            cdf[l] = pv[k];
-            if (pv[k] > 0.0) mylast = l;
-            k++;
+#pragma unroll
+        for (int j = 0; j < 16; j++) {
+            const int l = tid + threads * j;
+            if (!active || l >= T) continue;
+            cdf[cdf_at(l)] = pv[j];
+            if (pv[j] > 0.0) mylast = l;
         }
         if (mylast >= 0) atomicMax(&sh.last_nz, mylast);
         __syncthreads();
         lds_scan(sh, cdf, T, 0.0);
         const int fallback = sh.last_nz < 0 ? 0 : sh.last_nz;
         for (int s = tid; s < I.num_shots; s += NT) {
-            const double u = draws[I.draw_offset + s];
-            int lo = 0, hi = T;
-            while (lo < hi) {
-                const int mid = (lo + hi) >> 1;
-                if (u < cdf[mid]) hi = mid;
-                else lo = mid + 1;
-            }
-            outcomes[I.out_offset + s] = (uint64_t)(lo < T ? lo : fallback);
+            const int l = cdf_find(cdf, T, draws[I.draw_offset + s]);
+            outcomes[I.out_offset + s] = (uint64_t)(l < T ? l : fallback);
         }
         __syncthreads();
         return;
@@ -602,75 +813,65 @@ __device__ void run_circuit(Shared &sh, const BInst &I, const BPass *passes, con
         }
     }
     __syncthreads();
-    // each shot's starting tile
-    const int per_thread = (I.num_shots + NT - 1) / NT;
-    for (int rep = 0; rep < per_thread; rep++) {
-        const int s = tid + rep * NT;
-        uint64_t tile = ntiles;
-        double u = 2.0;
-        if (s < I.num_shots) {
-            u = draws[I.draw_offset + s];
-            uint64_t lo = 0, hi = ntiles;
-            while (lo < hi) {
-                const uint64_t mid = (lo + hi) >> 1;
-                if (u < incl[mid]) hi = mid;
-                else lo = mid + 1;
-            }
-            tile = lo;
+    // Each shot's slot holds, until it is resolved, a mark and the tile it is
+    // looked for in: first the one the prefix names, the next one when
+    // rounding leaves its draw past that tile's own sums.
+    constexpr uint64_t kMark = 1ull << 63;
+    uint64_t *oc = outcomes + I.out_offset;
+    for (int s = tid; s < I.num_shots; s += NT) {
+        const double u = draws[I.draw_offset + s];
+        uint64_t lo = 0, hi = ntiles;
+        while (lo < hi) {
+            const uint64_t mid = (lo + hi) >> 1;
+            if (u < incl[mid]) hi = mid;
+            else lo = mid + 1;
         }
-        uint64_t result = UINT64_MAX;
-        // walk tiles in order; every thread joins every step so barriers match
-        for (uint64_t ti = 0; ti < ntiles; ti++) {
-            if (tid == 0) sh.flag = 0;
-            __syncthreads();
-            if (tile == ti && result == UINT64_MAX) sh.flag = 1;
-            __syncthreads();
-            const int need = sh.flag;
-            __syncthreads();   // every thread has read the flag before thread 0 clears it again
-            if (!need) continue;
-            for (int l = tid; l < T; l += NT) cdf[l] = p2<R>(slot[(ti << tb) | l]);
-            __syncthreads();
-            lds_scan(sh, cdf, T, ti ? incl[ti - 1] : 0.0);
-            if (tile == ti && result == UINT64_MAX) {
-                int lo = 0, hi = T;
-                while (lo < hi) {
-                    const int mid = (lo + hi) >> 1;
-                    if (u < cdf[mid]) hi = mid;
-                    else lo = mid + 1;
-                }
-                if (lo < T) result = (ti << tb) | (uint64_t)lo;
-                else tile = ti + 1;   // rounding left u past this tile: continue in the next
-            }
-            __syncthreads();
+        oc[s] = kMark | lo;
+    }
+    for (uint64_t ti = 0; ti < ntiles; ti++) {
+        int mine = 0;
+        for (int s = tid; s < I.num_shots; s += NT) mine |= oc[s] == (kMark | ti);
+        if (!__syncthreads_or(mine)) continue;
+        for (int l = tid; l < T; l += NT) cdf[cdf_at(l)] = p2<R>(slot[(ti << nb) | (uint64_t)l]);
+        __syncthreads();
+        lds_scan(sh, cdf, T, ti ? incl[ti - 1] : 0.0);
+        for (int s = tid; s < I.num_shots; s += NT) {
+            if (oc[s] != (kMark | ti)) continue;
+            const int l = cdf_find(cdf, T, draws[I.draw_offset + s]);
+            oc[s] = l < T ? (ti << nb) | (uint64_t)l : kMark | (ti + 1);
         }
-        if (s < I.num_shots && result == UINT64_MAX) {
-            // u >= total mass: the last index with nonzero probability
-            uint64_t last = 0;
-            for (uint64_t ti = ntiles; ti-- > 0;) {
-                if (tile_sums[ti] > 0.0) {
-                    for (int l = T - 1; l >= 0; l--)
-                        if (p2<R>(slot[(ti << tb) | l]) > 0.0) {
-                            last = (ti << tb) | (uint64_t)l;
-                            break;
-                        }
-                    break;
-                }
-            }
-            result = last;
-        }
-        if (s < I.num_shots) outcomes[I.out_offset + s] = result;
         __syncthreads();
     }
+    for (int s = tid; s < I.num_shots; s += NT) {
+        if (!(oc[s] & kMark)) continue;
+        // u >= total mass: the last index with nonzero probability
+        uint64_t last = 0;
+        for (uint64_t ti = ntiles; ti-- > 0;) {
+            if (tile_sums[ti] > 0.0) {
+                for (int l = T - 1; l >= 0; l--)
+                    if (p2<R>(slot[(ti << nb) | (uint64_t)l]) > 0.0) {
+                        last = (ti << nb) | (uint64_t)l;
+                        break;
+                    }
+                break;
+            }
+        }
+        oc[s] = last;
+    }
+    __syncthreads();
 }
 
-__global__ __launch_bounds__(NT) void k_batch(const BInst *__restrict__ insts,
-                                              const int32_t *__restrict__ order, int ninst,
-                                              int *__restrict__ counter, const BPass *__restrict__ passes,
-                                              const BOp *__restrict__ ops, double2 *__restrict__ scratch,
-                                              uint64_t slot_amps, double *__restrict__ tile_scratch,
-                                              uint64_t tile_slot, const double *__restrict__ draws,
-                                              double *__restrict__ obs, uint64_t *__restrict__ outcomes,
-                                              const PauliT *__restrict__ terms, void *__restrict__ state_out)
+// One precision per launch: a kernel with both interpreters (42 KiB each)
+// would put the ends of the queue loop further apart than a branch reaches.
+template <typename R>
+__global__ __launch_bounds__(NT, 2) void k_batch(const BInst *__restrict__ insts, const int32_t *__restrict__ order,
+                                                 int ninst, int *__restrict__ counter,
+                                                 const FPass *__restrict__ passes, const FOp *__restrict__ prog,
+                                                 double2 *__restrict__ scratch, uint64_t slot_amps,
+                                                 double *__restrict__ tile_scratch, uint64_t tile_slot,
+                                                 const double *__restrict__ draws, double *__restrict__ obs,
+                                                 uint64_t *__restrict__ outcomes, const PauliT *__restrict__ terms,
+                                                 void *__restrict__ state_out)
 {
     __shared__ Shared sh;
     double2 *slot = scratch + (uint64_t)blockIdx.x * slot_amps;
@@ -679,21 +880,20 @@ __global__ __launch_bounds__(NT) void k_batch(const BInst *__restrict__ insts,
         if (threadIdx.x == 0) sh.next = atomicAdd(counter, 1);
         __syncthreads();
         // every lane read the same queue slot: make that explicit, so the
-        // instance, its passes and every op descriptor below are fetched with
-        // scalar (wave-uniform) loads instead of one vector load per lane
+        // instance and its passes are fetched with scalar (wave-uniform) loads
         const int k = __builtin_amdgcn_readfirstlane(sh.next);
         __syncthreads();
         if (k >= ninst) break;
-        const BInst I = insts[order[k]];
-        if (I.prec == 1)
-            run_circuit<float>(sh, I, passes, ops, slot, ts, draws, obs, outcomes, terms, state_out);
-        else
-            run_circuit<double>(sh, I, passes, ops, slot, ts, draws, obs, outcomes, terms, state_out);
+        BInst I;
+        const FConst<uint32_t> src = (FConst<uint32_t>)(uintptr_t)(insts + *(FConst<int32_t>)(uintptr_t)(order + k));
+#pragma unroll
+        for (int w = 0; w < (int)(sizeof I / sizeof(uint32_t)); w++) ((uint32_t *)&I)[w] = src[w];
+        run_circuit<R>(sh, MLX_FRAME_LDS(sh.tile), I, passes, prog, slot, ts, draws, obs, outcomes, terms, state_out);
         __syncthreads();
     }
 }
 
-__global__ void k_reset_counter(int *c) { *c = 0; }
+__global__ void k_reset_counter(int *c) { c[threadIdx.x] = 0; }
 
 // One cache-blocked pass over a large state: each workgroup streams tiles of
 // 2^P.nbits amplitudes through LDS and applies the pass's ops there.  The
@@ -802,14 +1002,23 @@ hipError_t launch_tile_pass(void *amps, int prec, int n, const BPass &P, const B
               : tile_pass_shape<double, false>(amps, P, d_ops, ntiles, cus, threads, tile_bits, st);
 }
 
-hipError_t launch_batch(const BInst *insts, const int32_t *order, int ninst, int *counter, const BPass *passes,
-                        const BOp *ops, double2 *scratch, uint64_t slot_amps, double *tile_scratch,
+// order: the n128 complex128 circuits, then the n64 complex64 ones; counter:
+// two queue heads; grid: workgroups at most (the two launches follow each
+// other and share the slots).
+hipError_t launch_batch(const BInst *insts, const int32_t *order, int n128, int n64, int *counter, const FPass *passes,
+                        const FOp *prog, double2 *scratch, uint64_t slot_amps, double *tile_scratch,
                         uint64_t tile_slot, const double *draws, double *obs, uint64_t *outcomes,
                         const PauliT *terms, void *state_out, int grid, hipStream_t st)
 {
-    k_reset_counter<<<1, 1, 0, st>>>(counter);
-    k_batch<<<grid, NT, 0, st>>>(insts, order, ninst, counter, passes, ops, scratch, slot_amps, tile_scratch,
-                                 tile_slot, draws, obs, outcomes, terms, state_out);
+    k_reset_counter<<<1, 2, 0, st>>>(counter);
+    if (n128 > 0)
+        k_batch<double><<<n128 < grid ? n128 : grid, NT, 0, st>>>(insts, order, n128, counter, passes, prog, scratch,
+                                                                  slot_amps, tile_scratch, tile_slot, draws, obs,
+                                                                  outcomes, terms, state_out);
+    if (n64 > 0)
+        k_batch<float><<<n64 < grid ? n64 : grid, NT, 0, st>>>(insts, order + n128, n64, counter + 1, passes, prog,
+                                                               scratch, slot_amps, tile_scratch, tile_slot, draws, obs,
+                                                               outcomes, terms, state_out);
     return hipGetLastError();
 }
 

@@ -114,10 +114,8 @@ __host__ __device__ inline int lds_slot(int x)
     return x ^ ((x >> 4 ^ x >> 8 ^ x >> 12) & 15);
 }
 
-// Register bits of a segment: the single-state tile pass holds 8 amplitudes
-// per thread; the batch kernel, which also carries measurement state, 4.
-// Op descriptors the batch kernel stages in LDS at a time; a register
-// segment (header + its ops) never exceeds it.
+// A register segment of the LDS op engine (header + its ops) holds at most
+// kOpBuf descriptors, on 2 register bits: 4 amplitudes per thread.
 constexpr int kOpBuf = 32;
 constexpr int kSegRegsPass = 2;
 constexpr int kSegRegsBatch = 2;
@@ -146,7 +144,7 @@ struct BPass {
 struct BInst {
     int32_t  n;
     int32_t  prec;          // 0 = complex128, 1 = complex64
-    int32_t  tile_bits;     // min(n, max tile bits)
+    int32_t  tile_bits;     // tile bits of its passes: max(min(n, tile bits of the batch), 4)
     int32_t  first_pass;
     int32_t  num_passes;    // gate passes
     int32_t  num_mpasses;   // measurement passes (follow the gate passes)
@@ -181,7 +179,7 @@ enum : int32_t {
 __host__ __device__ inline int64_t obs_size(int n) { return 1 + n + (n > 1 ? n - 1 : 0) + n; }
 
 constexpr int kBatchMaxTileBits = 12;
-constexpr int kBatchThreads = 1024;
+constexpr int kBatchThreads = 256;
 constexpr int kBatchMaxQubits = 24;
 
 }  // namespace mlx

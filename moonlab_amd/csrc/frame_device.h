@@ -332,6 +332,21 @@ template <typename T> __device__ __forceinline__ FConst<T> frame_const(const FOp
     return (FConst<T>)(uintptr_t)p;
 }
 
+// The lowest bits of x spread over the set bits of mask, lowest first.
+__device__ __forceinline__ uint64_t frame_deposit(uint64_t x, uint64_t mask)
+{
+    uint64_t o = 0;
+    for (; mask && x; mask &= mask - 1, x >>= 1)
+        if (x & 1ull) o |= mask & (0ull - mask);
+    return o;
+}
+
+// a + b where both are numbers spread over the clear bits of mask
+__device__ __forceinline__ uint64_t frame_step(uint64_t a, uint64_t b, uint64_t mask)
+{
+    return ((a | mask) + b) & ~mask;
+}
+
 // What a thread keeps over the tiles of a pass: the output layout's LDS
 // address and its word of the sign table.
 struct FrameThread {
@@ -339,72 +354,87 @@ struct FrameThread {
     uint32_t sign;
 };
 
-__device__ __forceinline__ FrameThread frame_thread(const FPass &P, const FOp *prog, int tid, int tbits, bool active)
+__device__ __forceinline__ FrameThread frame_thread(FConst<FPass> P, const FOp *prog, int tid, int tbits, bool active)
 {
     FrameThread f{0, 0};
-    if (P.flags & FP_OUT) {
-        const FConst<FOut> o = frame_const<FOut>(prog + P.out);
+    if (P->flags & FP_OUT) {
+        const FConst<FOut> o = frame_const<FOut>(prog + P->out);
         for (int b = 0; b < tbits; b++) f.out_slot ^= ((tid >> b) & 1) ? o->col[b] : 0u;
     }
-    if (P.table >= 0 && active) f.sign = ((const uint16_t *)(prog + P.table))[tid];
+    if (P->table >= 0 && active) f.sign = ((const uint16_t *)(prog + P->table))[tid];
     return f;
+}
+
+// byte address of a __shared__ variable
+#define MLX_FRAME_LDS(var) ((uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)&(var))
+
+// x, known to be the same on every lane, in scalar registers
+__device__ __forceinline__ uint64_t frame_uniform(uint64_t x)
+{
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)x);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(x >> 32));
+    return ((uint64_t)hi << 32) | lo;
 }
 
 // The phases of a pass on one tile, then the signs, the scale and the output
 // layout: v enters and leaves in the IO layout (register bits = top four tile
-// bits).  Every thread of the workgroup calls it (barriers); the LDS holds 16
-// amplitudes per thread of the workgroup, whatever the tile's size.
+// bits).  Every thread of the workgroup calls it (barriers); lds: byte address
+// (MLX_FRAME_LDS) of 16 amplitudes per thread of the workgroup, whatever the
+// tile's size.
 template <typename R>
-__device__ __forceinline__ void frame_tile(cplx_t<R> *tile, typename FVec<R>::t (&v)[16], const FPass &P,
+__device__ __forceinline__ void frame_tile(uint32_t lds, typename FVec<R>::t (&v)[16], FConst<FPass> P,
                                            const FOp *prog, const FrameThread &ft, uint64_t base, int tid,
                                            int nbits)
 {
     using V = typename FVec<R>::t;
-    using Shared = __attribute__((address_space(3))) char;
-    Shared *lb = (Shared *)tile;
     // the thread's slot in the current layout; thread bits past the tile's
     // go above its index
     const int x0 = tid + 15 * (tid & -(1 << (nbits - kFrameRegBits)));
     uint32_t slot = (uint32_t)lds_slot<(int)sizeof(V)>(x0) * (uint32_t)sizeof(V);
-    if (P.nphases > 0) frame_phases(v, prog + P.first, P.nphases, (uint32_t)tid, base, slot, (uint32_t)(uintptr_t)lb);
-    if (P.flags & (FP_SIGN | FP_SCALE | FP_CSCALE)) {
+    if (P->nphases > 0)
+        frame_phases(v, (const FOp *)frame_uniform((uint64_t)(uintptr_t)(prog + P->first)),
+                     __builtin_amdgcn_readfirstlane(P->nphases), (uint32_t)tid, frame_uniform(base), slot,
+                     lds);
+    if (P->flags & (FP_SIGN | FP_SCALE | FP_CSCALE)) {
         uint32_t s = ft.sign;
-        for (int c = 0; c < P.ncross; c++) {
-            const FConst<FCross> x = frame_const<FCross>(prog + P.cross) + c;
+        for (int c = 0; c < P->ncross; c++) {
+            const FConst<FCross> x = frame_const<FCross>(prog + P->cross) + c;
             const uint32_t a = (uint32_t)__popcll(x->ga & base) & 1u, b = (uint32_t)__popcll(x->gb & base) & 1u;
             const uint32_t fa = x->wa ^ (0u - ((uint32_t)__popc(x->ta & tid) & 1u));
             const uint32_t fb = x->wb ^ (0u - ((uint32_t)__popc(x->tb & tid) & 1u));
             s ^= (a ? fb : 0u) ^ (b ? fa : 0u) ^ (a & b ? 0xFFFFu : 0u);
         }
-        const R sr = (R)P.scale_r, si = (R)P.scale_i;
-        const bool cplx = (P.flags & FP_CSCALE) != 0;
+        const R sr = (R)P->scale_r, si = (R)P->scale_i;
+        if (P->flags & FP_CSCALE) {
 #pragma unroll
-        for (int j = 0; j < 16; j++) {
-            const bool neg = (s >> j) & 1u;
-            const R r = neg ? -sr : sr;
-            if (cplx) {
-                const cplx_t<R> y = cmul(cplx_t<R>{v[j].x, v[j].y}, r, neg ? -si : si);
+            for (int j = 0; j < 16; j++) {
+                const bool neg = (s >> j) & 1u;
+                const cplx_t<R> y = cmul(cplx_t<R>{v[j].x, v[j].y}, neg ? -sr : sr, neg ? -si : si);
                 v[j].x = y.x;
                 v[j].y = y.y;
-            } else {
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < 16; j++) {
+                const R r = (s >> j) & 1u ? -sr : sr;
                 v[j].x *= r;
                 v[j].y *= r;
             }
         }
     }
-    if (P.flags & FP_OUT) {
-        const FConst<FOut> o = frame_const<FOut>(prog + P.out);
+    if (P->flags & FP_OUT) {
+        const FConst<FOut> o = frame_const<FOut>(prog + P->out);
         using SharedV = __attribute__((address_space(3))) V;
 #pragma unroll
-        for (int j = 0; j < 16; j++) *(SharedV *)(lb + (slot ^ o->from[j])) = v[j];
+        for (int j = 0; j < 16; j++) *(SharedV *)(uintptr_t)(lds + (slot ^ o->from[j])) = v[j];
         uint32_t os = ft.out_slot;
-        for (int c = 0; c < P.nshift; c++) {
-            const FConst<FShift> x = frame_const<FShift>(prog + P.shift) + c;
+        for (int c = 0; c < P->nshift; c++) {
+            const FConst<FShift> x = frame_const<FShift>(prog + P->shift) + c;
             os ^= (__popcll(x->gmask & base) & 1) ? x->off : 0u;
         }
         lds_barrier();
 #pragma unroll
-        for (int j = 0; j < 16; j++) v[j] = *(const SharedV *)(lb + (os ^ o->off[j]));
+        for (int j = 0; j < 16; j++) v[j] = *(const SharedV *)(uintptr_t)(lds + (os ^ o->off[j]));
         // Between two changes a thread writes only slots that it alone has
         // read; the output's permutation breaks that, so nothing is written
         // (by the next tile) before every thread has read.

@@ -41,23 +41,15 @@ struct Step {
     double c, s;      // of theta/2
 };
 
-// The gates waiting on one qubit: their product u and, while they are at
-// most four, the steps they came from (a trailing Pauli X of H included as
-// x_after).
+// The gates waiting on one qubit: up to three steps, applied in order and
+// times phase, or, for longer runs, their product u (three Euler rotations
+// are shorter then).
 struct Pending {
-    cd   u[4];
-    bool has = false;
-    Step st[4];
+    Step st[3];
     int  nst = 0;
-    bool listed = true;   // st describes u up to `phase`
+    bool folded = false;
     cd   phase = 1.0;
-    void clear()
-    {
-        has = false;
-        nst = 0;
-        listed = true;
-        phase = 1.0;
-    }
+    cd   u[4];
 };
 
 class Lowering {
@@ -87,34 +79,24 @@ class Lowering {
         return p[k & 3];
     }
 
-    // a single-qubit gate u = phase * (product of steps, first applied first)
-    void gate_1q(int q, const cd u[4], const Step *st, int nst, cd phase)
+    // a single-qubit gate: phase times a step
+    void step(int q, int axis, double c, double sn, cd phase = 1.0)
     {
         Pending &p = pend_[(size_t)q];
-        if (!p.has) {
-            for (int i = 0; i < 4; i++) p.u[i] = u[i];
-            p.has = true;
-        } else {
-            const cd a = p.u[0], b = p.u[1], c = p.u[2], d = p.u[3];
-            p.u[0] = u[0] * a + u[1] * c;
-            p.u[1] = u[0] * b + u[1] * d;
-            p.u[2] = u[2] * a + u[3] * c;
-            p.u[3] = u[2] * b + u[3] * d;
-        }
-        if (!p.listed) return;
         p.phase *= phase;
-        for (int i = 0; i < nst; i++) {
-            if (p.nst && p.st[p.nst - 1].axis == st[i].axis) {   // same axis: angles add
-                Step &l = p.st[p.nst - 1];
-                const double c = l.c * st[i].c - l.s * st[i].s, s = l.c * st[i].s + l.s * st[i].c;
-                l.c = c;
-                l.s = s;
-            } else if (p.nst < 3) {
-                p.st[p.nst++] = st[i];
-            } else {
-                p.listed = false;   // three Euler rotations are shorter
-                return;
-            }
+        const Step st{axis, c, sn};
+        if (p.folded) {
+            fold(p, st);
+        } else if (p.nst && p.st[p.nst - 1].axis == axis) {   // same axis: angles add
+            Step &l = p.st[p.nst - 1];
+            l = Step{axis, l.c * c - l.s * sn, l.s * c + l.c * sn};
+        } else if (p.nst < 3) {
+            p.st[p.nst++] = st;
+        } else {
+            step_matrix(p.st[0], p.u);
+            for (int i = 1; i < 3; i++) fold(p, p.st[i]);
+            fold(p, st);
+            p.folded = true;
         }
     }
 
@@ -124,25 +106,22 @@ class Lowering {
     void flush(int q, int keep)
     {
         Pending &p = pend_[(size_t)q];
-        if (!p.has) return;
-        if (!p.listed) euler(p);
+        if (!p.nst) {
+            phase_ *= p.phase;
+            p.phase = 1.0;
+            return;
+        }
+        if (p.folded) euler(p);
         phase_ *= p.phase;
+        p.phase = 1.0;
         const uint64_t b = 1ull << q;
         int m = p.nst;
-        const bool hold = m > 0 && p.st[m - 1].axis == keep;
+        const bool hold = p.st[m - 1].axis == keep;
         if (hold) m--;
         for (int i = 0; i < m; i++)
             rot(p.st[i].axis == 2 ? 0 : b, p.st[i].axis == 0 ? 0 : b, p.st[i].c, p.st[i].s);
-        if (hold) {
-            const Step l = p.st[m];
-            p.clear();
-            p.has = true;
-            p.nst = 1;
-            p.st[0] = l;
-            step_matrix(l, p.u);
-        } else {
-            p.clear();
-        }
+        if (hold) p.st[0] = p.st[m];
+        p.nst = hold ? 1 : 0;
     }
 
     static void step_matrix(const Step &l, cd u[4])
@@ -153,7 +132,18 @@ class Lowering {
     }
 
   private:
-    // u = phase RZ(beta) RY(gamma) RZ(delta).  A sum or difference that an
+    static void fold(Pending &p, const Step &l)
+    {
+        cd m[4];
+        step_matrix(l, m);
+        const cd a = p.u[0], b = p.u[1], c = p.u[2], d = p.u[3];
+        p.u[0] = m[0] * a + m[1] * c;
+        p.u[1] = m[0] * b + m[1] * d;
+        p.u[2] = m[2] * a + m[3] * c;
+        p.u[3] = m[2] * b + m[3] * d;
+    }
+
+    // u = RZ(beta) RY(gamma) RZ(delta) times a phase (into p.phase).  A sum or difference that an
     // entry of modulus 0 leaves open is taken as 0; each is known up to 2 pi,
     // and the one of the smaller entry takes the branch that agrees with the
     // phase the larger entry gives.
@@ -163,19 +153,21 @@ class Lowering {
         const double h = hypot(c, s);
         double sum = c > 0.0 ? arg(p.u[3] * conj(p.u[0])) : 0.0;      // beta + delta
         double dif = s > 0.0 ? arg(-p.u[2] * conj(p.u[1])) : 0.0;     // beta - delta
+        cd ph;
         if (c >= s) {
-            p.phase = p.u[0] / c * std::polar(1.0, 0.5 * sum);
-            if (s > 0.0 && real(p.u[2] * conj(p.phase * std::polar(1.0, 0.5 * dif))) < 0.0) dif += 2.0 * M_PI;
+            ph = p.u[0] / c * std::polar(1.0, 0.5 * sum);
+            if (s > 0.0 && real(p.u[2] * conj(ph * std::polar(1.0, 0.5 * dif))) < 0.0) dif += 2.0 * M_PI;
         } else {
-            p.phase = p.u[2] / s * std::polar(1.0, -0.5 * dif);
-            if (c > 0.0 && real(p.u[0] * conj(p.phase * std::polar(1.0, -0.5 * sum))) < 0.0) sum += 2.0 * M_PI;
+            ph = p.u[2] / s * std::polar(1.0, -0.5 * dif);
+            if (c > 0.0 && real(p.u[0] * conj(ph * std::polar(1.0, -0.5 * sum))) < 0.0) sum += 2.0 * M_PI;
         }
         const double beta = 0.5 * (sum + dif), delta = 0.5 * (sum - dif);
-        p.nst = 0;
-        p.st[p.nst++] = Step{2, cos(0.5 * delta), sin(0.5 * delta)};
-        p.st[p.nst++] = Step{1, c / h, s / h};
-        p.st[p.nst++] = Step{2, cos(0.5 * beta), sin(0.5 * beta)};
-        p.listed = true;
+        p.phase *= ph;
+        p.st[0] = Step{2, cos(0.5 * delta), sin(0.5 * delta)};
+        p.st[1] = Step{1, c / h, s / h};
+        p.st[2] = Step{2, cos(0.5 * beta), sin(0.5 * beta)};
+        p.nst = 3;
+        p.folded = false;
     }
 
     std::vector<FGate>  &out_;
@@ -185,55 +177,56 @@ class Lowering {
 
 }  // namespace
 
-bool frame_lower(const moonlab_hip_gate_t *g, int ng, int n, std::vector<FGate> &out, cd &phase)
+bool frame_lower(const moonlab_hip_gate_t *g, int ng, int n, std::vector<FGate> &out, cd &phase, bool any_angle)
 {
     phase = 1.0;
     Lowering L(n, out, phase);
     const double r8 = 0.70710678118654752440;            // cos(pi/4)
     const double c8 = cos(M_PI / 8.0), s8 = sin(M_PI / 8.0);
+    const cd I(0.0, 1.0);
+    static_assert(MOONLAB_HIP_GATE_RY == MOONLAB_HIP_GATE_RX + 1 && MOONLAB_HIP_GATE_RZ == MOONLAB_HIP_GATE_RX + 2,
+                  "axis = type - RX");
     for (int i = 0; i < ng; i++) {
         const moonlab_hip_gate_t &x = g[i];
         if (!gate_valid(x, n)) return false;
-        if (!std::isfinite(x.theta) || !std::isfinite(x.phi) || !std::isfinite(x.lam)) return false;
+        if (!any_angle && (!std::isfinite(x.theta) || !std::isfinite(x.phi) || !std::isfinite(x.lam))) return false;
         const int t = x.target, c = x.control, e = x.extra;
         const uint64_t T = t >= 0 ? 1ull << t : 0, C = c >= 0 ? 1ull << c : 0;
-        cd u[4];
-        if (gate_matrix_1q(x, u)) {
-            const double co = cos(x.theta / 2.0), si = sin(x.theta / 2.0);
-            Step st[3];
-            int ns = 0;
-            cd ph = 1.0;
-            switch (x.type) {
-            case MOONLAB_HIP_GATE_I: continue;
-            case MOONLAB_HIP_GATE_X: st[ns++] = Step{0, 0.0, 1.0}; ph = cd(0, 1); break;
-            case MOONLAB_HIP_GATE_Y: st[ns++] = Step{1, 0.0, 1.0}; ph = cd(0, 1); break;
-            case MOONLAB_HIP_GATE_Z: st[ns++] = Step{2, 0.0, 1.0}; ph = cd(0, 1); break;
-            case MOONLAB_HIP_GATE_H:   // X RY(pi/2)
-                st[ns++] = Step{1, r8, r8};
-                st[ns++] = Step{0, 0.0, 1.0};
-                ph = cd(0, 1);
-                break;
-            case MOONLAB_HIP_GATE_S: st[ns++] = Step{2, r8, r8}; ph = cd(r8, r8); break;
-            case MOONLAB_HIP_GATE_SDG: st[ns++] = Step{2, r8, -r8}; ph = cd(r8, -r8); break;
-            case MOONLAB_HIP_GATE_T: st[ns++] = Step{2, c8, s8}; ph = cd(c8, s8); break;
-            case MOONLAB_HIP_GATE_TDG: st[ns++] = Step{2, c8, -s8}; ph = cd(c8, -s8); break;
-            case MOONLAB_HIP_GATE_PHASE: st[ns++] = Step{2, co, si}; ph = cd(co, si); break;
-            case MOONLAB_HIP_GATE_RX: st[ns++] = Step{0, co, si}; break;
-            case MOONLAB_HIP_GATE_RY: st[ns++] = Step{1, co, si}; break;
-            case MOONLAB_HIP_GATE_RZ: st[ns++] = Step{2, co, si}; break;
-            case MOONLAB_HIP_GATE_U3: {   // e^(i (phi + lam) / 2) RZ(phi) RY(theta) RZ(lam)
-                const double cp = cos(x.phi / 2.0), sp = sin(x.phi / 2.0);
-                const double cl = cos(x.lam / 2.0), sl = sin(x.lam / 2.0);
-                st[ns++] = Step{2, cl, sl};
-                st[ns++] = Step{1, co, si};
-                st[ns++] = Step{2, cp, sp};
-                ph = cd(cp, sp) * cd(cl, sl);
-                break;
-            }
-            default: return false;
-            }
-            L.gate_1q(t, u, st, ns, ph);
+        double si, co;
+        switch (x.type) {
+        case MOONLAB_HIP_GATE_I: continue;
+        case MOONLAB_HIP_GATE_X: L.step(t, 0, 0.0, 1.0, I); continue;
+        case MOONLAB_HIP_GATE_Y: L.step(t, 1, 0.0, 1.0, I); continue;
+        case MOONLAB_HIP_GATE_Z: L.step(t, 2, 0.0, 1.0, I); continue;
+        case MOONLAB_HIP_GATE_H:   // X RY(pi/2)
+            L.step(t, 1, r8, r8);
+            L.step(t, 0, 0.0, 1.0, I);
             continue;
+        case MOONLAB_HIP_GATE_S: L.step(t, 2, r8, r8, cd(r8, r8)); continue;
+        case MOONLAB_HIP_GATE_SDG: L.step(t, 2, r8, -r8, cd(r8, -r8)); continue;
+        case MOONLAB_HIP_GATE_T: L.step(t, 2, c8, s8, cd(c8, s8)); continue;
+        case MOONLAB_HIP_GATE_TDG: L.step(t, 2, c8, -s8, cd(c8, -s8)); continue;
+        case MOONLAB_HIP_GATE_PHASE:
+            sincos(x.theta / 2.0, &si, &co);
+            L.step(t, 2, co, si, cd(co, si));
+            continue;
+        case MOONLAB_HIP_GATE_RX:
+        case MOONLAB_HIP_GATE_RY:
+        case MOONLAB_HIP_GATE_RZ:
+            sincos(x.theta / 2.0, &si, &co);
+            L.step(t, x.type - MOONLAB_HIP_GATE_RX, co, si);
+            continue;
+        case MOONLAB_HIP_GATE_U3: {   // e^(i (phi + lam) / 2) RZ(phi) RY(theta) RZ(lam)
+            double sp, cp, sl, cl;
+            sincos(x.theta / 2.0, &si, &co);
+            sincos(x.phi / 2.0, &sp, &cp);
+            sincos(x.lam / 2.0, &sl, &cl);
+            L.step(t, 2, cl, sl, cd(cl, sl));
+            L.step(t, 1, co, si);
+            L.step(t, 2, cp, sp, cd(cp, sp));
+            continue;
+        }
+        default: break;
         }
         switch (x.type) {
         case MOONLAB_HIP_GATE_CNOT:
@@ -486,8 +479,8 @@ class PassBuilder {
         int k = 0;
         for (int q = 0; q < 64 && k < nb; q++)
             if (set & (1ull << q)) {
-                local[q] = k;
-                P.qubits[k++] = (int8_t)q;
+                local[q] = k++;
+                P.mask |= 1ull << q;
             }
         image(gates, local, nb);
         P.first = (int32_t)prog_.size();
@@ -565,34 +558,44 @@ class PassBuilder {
         }
     }
 
-    static bool commute(const Row &a, const Row &b) { return par((a.x & b.z) ^ (b.x & a.z)) == 0; }
+    // x and z of an image in one word; two commute when parity(a & swap(b)) is 0
+    static uint32_t packed(const Row &p) { return p.x | (p.z << 16); }
+    static uint32_t swapped(uint32_t v) { return (v >> 16) | (v << 16); }
 
     // Rotations of rest_ that a phase takes, in order: those whose direction
     // is one of its (up to four) basis vectors and that commute with every
-    // rotation put off.  fixed: the basis is given whole.
+    // rotation put off.  fixed: the basis is given whole.  "Commutes with
+    // every one" is checked against a basis of their span (at most 2 x tile
+    // bits words); once that is full nothing more can be taken.
     int scan(uint32_t *basis, int &nbasis, bool fixed)
     {
-        constexpr size_t kMaxDeferred = 48;   // bounds planning time
         take_.clear();
         def_.clear();
+        uint32_t span[2 * kFrameMaxTileBits];   // swapped words, echelon form by leading bit
+        int rank = 0;
+        const size_t m = rest_.size();
         size_t i = 0;
-        for (; i < rest_.size() && def_.size() < kMaxDeferred; i++) {
-            const LRot &o = rots_[(size_t)rest_[i]];
+        for (; i < m && rank < 2 * nb_; i++) {
+            const int id = rest_[i];
+            const uint32_t w = pack_[(size_t)id], x = w & 0xFFFFu;
             bool ok = true;
-            for (int d : def_)
-                if (!commute(o.p, rots_[(size_t)d].p)) {
-                    ok = false;
-                    break;
-                }
-            if (ok && o.p.x) {
+            for (int d = 0; d < rank && ok; d++) ok = !(__builtin_popcount(w & span[d]) & 1);
+            if (ok && x) {
                 bool in = false;
-                for (int b = 0; b < nbasis; b++) in = in || basis[b] == o.p.x;
+                for (int b = 0; b < nbasis; b++) in = in || basis[b] == x;
                 if (!in) {
-                    if (!fixed && nbasis < kFrameRegBits && independent(basis, nbasis, o.p.x)) basis[nbasis++] = o.p.x;
+                    if (!fixed && nbasis < kFrameRegBits && independent(basis, nbasis, x)) basis[nbasis++] = x;
                     else ok = false;
                 }
             }
-            (ok ? take_ : def_).push_back(rest_[i]);
+            if (ok) {
+                take_.push_back(id);
+                continue;
+            }
+            def_.push_back(id);
+            uint32_t v = swapped(w);
+            for (int d = 0; d < rank; d++) v = std::min(v, v ^ span[d]);   // clears span[d]'s leading bit
+            if (v) span[rank++] = v;
         }
         def_.insert(def_.end(), rest_.begin() + (long)i, rest_.end());
         return (int)take_.size();
@@ -600,20 +603,28 @@ class PassBuilder {
 
     void phases(FPass &P, Layout &cur)
     {
+        nb_ = P.nbits;
         rest_.resize(rots_.size());
-        for (size_t i = 0; i < rest_.size(); i++) rest_[i] = (int)i;
+        pack_.resize(rots_.size());
+        for (size_t i = 0; i < rest_.size(); i++) {
+            rest_[i] = (int)i;
+            pack_[i] = packed(rots_[i].p);
+        }
         double grown = 0.0;
         size_t hpos = 0;   // header of the latest phase
         while (!rest_.empty()) {
-            // candidates: the current layout (no exchange through LDS), a
+            // candidates: for the first phase the layout the tile enters in
+            // (no exchange through LDS; later phases have used up theirs), a
             // basis grown greedily, and bases seeded by the next pending directions
             uint32_t best[kFrameRegBits], b[kFrameRegBits];
-            int nbest = kFrameRegBits, nb = kFrameRegBits;
+            int nbest = kFrameRegBits, nb = kFrameRegBits, got = 0;
             memcpy(best, cur.r, sizeof best);
-            int got = scan(best, nbest, true);
-            if (got > 0) got++;   // a layout change costs about as much as eight rotations' arithmetic, mostly hidden
-            best_take_.swap(take_);
-            best_def_.swap(def_);
+            if (P.nphases == 0) {
+                got = scan(best, nbest, true);
+                if (got > 0) got++;   // a layout change costs about eight rotations' arithmetic, mostly hidden
+                best_take_.swap(take_);
+                best_def_.swap(def_);
+            }
             auto candidate = [&](uint32_t seed) {
                 nb = 0;
                 if (seed) b[nb++] = seed;
@@ -651,8 +662,7 @@ class PassBuilder {
             if (h.relayout) cur = L;
             for (int i = 0; i < kFrameRegBits; i++) h.nm[i] = 0u - (1u << cur.piv[i]);
             for (int j = 0; j < 16; j++) h.off[j] = slot_bytes(reg_index(cur, j), bytes_);
-            // in the layout of the phase before (its scan stopped at the
-            // planning bound): its rotations go on
+            // in the layout of the phase before: its rotations go on
             const bool join = !h.relayout && P.nphases > 0;
             if (!join) {
                 hpos = prog_.size();
@@ -841,9 +851,10 @@ class PassBuilder {
         prog_.push_back(f);
     }
 
-    int                    bytes_, look_;
+    int                    bytes_, look_, nb_ = 0;
     std::vector<FPass>    &passes_;
     std::vector<FOp>      &prog_;
+    std::vector<uint32_t>  pack_;
     std::vector<Row>       X_, Z_;
     std::vector<LRot>      rots_;
     std::vector<Quad>      quads_;

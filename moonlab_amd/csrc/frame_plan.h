@@ -23,8 +23,13 @@ struct FGate {
 };
 
 // Gate list -> rotations and frame gates, and the global phase they leave
-// out.  False on an invalid gate or qubit or a parameter that is not finite.
-bool frame_lower(const moonlab_hip_gate_t *g, int ng, int n, std::vector<FGate> &out, std::complex<double> &phase);
+// out.  False on an invalid gate or qubit, or, unless any_angle, a parameter
+// that is not finite (whose rotation would reach every amplitude).
+bool frame_lower(const moonlab_hip_gate_t *g, int ng, int n, std::vector<FGate> &out, std::complex<double> &phase,
+                 bool any_angle = false);
+
+// Seeds per tile set and register basis of the batch engine's plans.
+constexpr int kBatchLookahead = 0;
 
 // Plan passes over tile sets of tb qubits (n <= tb: one pass over max(n, 4)
 // qubits) that keep the lowest anchor_bits qubits.  amp_bytes: 16 or 8.

@@ -112,7 +112,7 @@ struct FPass {
     int32_t  out, cross, shift, table;
     int32_t  ncross, nshift;
     double   scale_r, scale_i;
-    int8_t   qubits[16];      // tile set, ascending
+    uint64_t mask;            // the tile's qubits: tile-index bit b is its b-th lowest bit
 };
 
 }  // namespace mlx

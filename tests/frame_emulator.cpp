@@ -109,11 +109,12 @@ static double run(int n, const std::vector<moonlab_hip_gate_t> &g, int tb, int B
     for (const FPass &P : passes) {
         g_passes++;
         if (P.nbits != (n <= tb ? m : tb)) die("tile bits");
-        for (int i = 1; i < P.nbits; i++) if (P.qubits[i] <= P.qubits[i - 1]) die("tile set not ascending");
+        if (__builtin_popcountll(P.mask) != P.nbits || (P.mask >> m)) die("tile set");
+        int qs[64], k = 0; for (int q = 0; q < m; q++) if ((P.mask >> q) & 1) qs[k++] = q;
         for (uint64_t ti = 0; ti < (1ull << (m - P.nbits)); ti++) {
-            uint64_t base = ti; for (int b = 0; b < P.nbits; b++) base = ins0(base, P.qubits[b]);
+            uint64_t base = ti; for (int b = 0; b < P.nbits; b++) base = ins0(base, qs[b]);
             std::vector<cd> t(1 << P.nbits);
-            auto addr = [&](int l) { uint64_t a = base; for (int b = 0; b < P.nbits; b++) if (l & (1 << b)) a |= 1ull << P.qubits[b]; return a; };
+            auto addr = [&](int l) { uint64_t a = base; for (int b = 0; b < P.nbits; b++) if (l & (1 << b)) a |= 1ull << qs[b]; return a; };
             for (int l = 0; l < (1 << P.nbits); l++) t[l] = st[addr(l)];
             run_tile(t, P, prog, base, B);
             for (int l = 0; l < (1 << P.nbits); l++) st[addr(l)] = t[l];
