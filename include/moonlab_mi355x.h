@@ -41,7 +41,8 @@ typedef struct {
     int return_amplitudes;     /* 1: fill `amplitudes` (2 * 2^n doubles, interleaved) */
     int return_probabilities;  /* 1: fill `probabilities` (2^n doubles) */
     int return_expect_z;       /* 1: fill `expect_z` (n doubles) and `norm` */
-    int fusion_max_qubits;     /* 0: one kernel per gate; 1..5: fuse into k-qubit blocks */
+    int fusion_max_qubits;     /* 1..5: fuse into k-qubit blocks; 0: passes over many gates or one kernel
+                                * per gate, whichever reads the state less often */
     int skip_shots;            /* 1: ignore the job's shot count (state outputs only) */
     int blocked;               /* 1: cache-blocked passes (moonlab_hip_apply_gates_blocked) */
 } moonlab_mi355x_exec_options_t;

@@ -669,21 +669,19 @@ int blocked_shape(int n, int prec, const GateTuning &t, bool *reg, int *anchor, 
 // (frame_plan.h), one pass for states of 4..11 qubits, 12-qubit tiles for
 // complex128 and 13-qubit ones for complex64 (or as tuned) above.  On
 // 30-qubit random layers a pass takes less than half of the register-phase
-// engine's (figures at k_frame_pass).  False where that engine stays: it is
-// selected, the state has under 4 qubits (four register bits), or a
-// parameter is not finite (a rotation would spread it to amplitudes that the
-// gate leaves alone).
-bool plan_frames(const moonlab_hip_gate_t *g, int ng, int n, int prec, const GateTuning &t, std::vector<FPass> &passes,
-                 std::vector<FOp> &prog)
+// engine's (figures at k_frame_pass).  False where another engine stays: the
+// state has under 4 qubits (four register bits), or a parameter is not finite
+// (a rotation would spread it to amplitudes that the gate leaves alone).
+bool plan_frames(const moonlab_hip_gate_t *g, int ng, int n, int prec, const GateTuning &t, int lookahead,
+                 std::vector<FPass> &passes, std::vector<FOp> &prog)
 {
-    if (t.blocked_engine != 0 || n < kFrameRegBits) return false;
+    if (n < kFrameRegBits) return false;
     std::vector<FGate> fg;
     cd phase;
     if (!frame_lower(g, ng, n, fg, phase)) return false;
     const bool c64 = prec == MOONLAB_HIP_C64;
     const int want = t.blocked_tile_bits ? t.blocked_tile_bits : (c64 ? 13 : 12);
-    frame_plan(fg, phase, n, want >= 13 && n >= 13 ? 13 : 12, c64 ? 4 : 3, c64 ? 8 : 16, t.blocked_lookahead, passes,
-               prog);
+    frame_plan(fg, phase, n, want >= 13 && n >= 13 ? 13 : 12, c64 ? 4 : 3, c64 ? 8 : 16, lookahead, passes, prog);
     prog.push_back(FOp{});   // the kernels fetch one unit past the last rotation
     return true;
 }
@@ -696,6 +694,25 @@ template <typename T> hipError_t upload(const std::vector<T> &v, T **d, hipStrea
     hipError_t e = hipMallocAsync((void **)d, v.size() * sizeof(T), st);
     if (e == hipSuccess) e = hipMemcpyAsync(*d, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
+    return e;
+}
+
+hipError_t run_frames(moonlab_hip_state_t *s, const std::vector<FPass> &fp, std::vector<FOp> &prog)
+{
+    if (fp.empty()) return hipSuccess;
+    const int n = (int)moonlab_hip_state_n_qubits(s), prec = moonlab_hip_state_precision(s);
+    hipStream_t st = (hipStream_t)moonlab_hip_state_stream(s);
+    void *amps = moonlab_hip_state_device_ptr(s);
+    // program and passes in one upload
+    const size_t units = prog.size(), tail = (fp.size() * sizeof(FPass) + sizeof(FOp) - 1) / sizeof(FOp);
+    prog.resize(units + tail);
+    memcpy((void *)&prog[units], fp.data(), fp.size() * sizeof(FPass));
+    FOp *d_prog = nullptr;
+    hipError_t e = upload(prog, &d_prog, st);
+    const FPass *d_pass = (const FPass *)(d_prog + units);
+    for (size_t i = 0; e == hipSuccess && i < fp.size(); i++)
+        e = launch_frame_pass(amps, prec, n, fp[i], d_pass + i, d_prog, st);
+    if (d_prog) hipFreeAsync(d_prog, st);
     return e;
 }
 
@@ -1101,6 +1118,28 @@ void *batch_state_buffer(moonlab_mi355x_batch_t *b, size_t bytes)
 
 hipStream_t batch_stream(moonlab_mi355x_batch_t *b) { return b->stream; }
 
+int mlx::apply_gates_planned(moonlab_hip_state_t *s, const moonlab_hip_gate_t *g, int ng)
+{
+    std::vector<FPass> fp;
+    std::vector<FOp> prog;
+    // one kernel per gate where the passes would not save half of them: a
+    // pass takes as long as 1 to 1.5 gate kernels at 30 qubits (7-9 ms, 5.4 ms)
+    const int n = (int)moonlab_hip_state_n_qubits(s);
+    const GateTuning tune = gate_tuning();
+    // Lookahead: two seeds plan 800 gates on 20 qubits into 12 passes in half
+    // the time (0.2 ms) of the eight the blocked path takes (13 passes); none
+    // makes 22.  From 26 qubits on a pass (0.5 ms) is worth more than planning.
+    const int look = n < 26 ? std::min(2, tune.blocked_lookahead) : tune.blocked_lookahead;
+    if (ng > 1 && plan_frames(g, ng, n, moonlab_hip_state_precision(s), tune, look, fp, prog) &&
+        2 * fp.size() <= (size_t)ng) {
+        const hipError_t e = run_frames(s, fp, prog);
+        if (e == hipSuccess) return MOONLAB_HIP_OK;
+        return set_last_error(e == hipErrorOutOfMemory ? MOONLAB_HIP_ERR_OUT_OF_MEMORY : MOONLAB_HIP_ERR_DRIVER,
+                              "apply_gates", e);
+    }
+    return moonlab_hip_apply_gates(s, g, ng);
+}
+
 extern "C" {
 
 moonlab_hip_status_t moonlab_hip_apply_gates_blocked(moonlab_hip_state_t *s, const moonlab_hip_gate_t *g,
@@ -1119,20 +1158,8 @@ moonlab_hip_status_t moonlab_hip_apply_gates_blocked(moonlab_hip_state_t *s, con
     };
     std::vector<FPass> fp;
     std::vector<FOp> prog;
-    if (plan_frames(g, ng, n, prec, tune, fp, prog)) {
-        if (fp.empty()) return MOONLAB_HIP_OK;
-        // program and passes in one upload
-        const size_t units = prog.size(), tail = (fp.size() * sizeof(FPass) + sizeof(FOp) - 1) / sizeof(FOp);
-        prog.resize(units + tail);
-        memcpy((void *)&prog[units], fp.data(), fp.size() * sizeof(FPass));
-        FOp *d_prog = nullptr;
-        hipError_t e = upload(prog, &d_prog, st);
-        const FPass *d_pass = (const FPass *)(d_prog + units);
-        for (size_t i = 0; e == hipSuccess && i < fp.size(); i++)
-            e = launch_frame_pass(amps, prec, n, fp[i], d_pass + i, d_prog, st);
-        if (d_prog) hipFreeAsync(d_prog, st);
-        return status(e);
-    }
+    if (tune.blocked_engine == 0 && plan_frames(g, ng, n, prec, tune, tune.blocked_lookahead, fp, prog))
+        return status(run_frames(s, fp, prog));
     std::vector<GOp> gops;
     if (!lower(g, ng, n, gops)) return MOONLAB_HIP_ERR_INVALID_QUBIT;
     std::vector<BPass> passes;
@@ -1172,7 +1199,9 @@ int moonlab_hip_blocked_pass_count(const moonlab_hip_gate_t *g, int ng, int n, i
     if (precision != MOONLAB_HIP_C128 && precision != MOONLAB_HIP_C64) return MOONLAB_HIP_ERR_BAD_ARG;
     std::vector<FPass> fp;
     std::vector<FOp> prog;
-    if (plan_frames(g, ng, n, precision, gate_tuning(), fp, prog)) return (int)fp.size();
+    const GateTuning tune = gate_tuning();
+    if (tune.blocked_engine == 0 && plan_frames(g, ng, n, precision, tune, tune.blocked_lookahead, fp, prog))
+        return (int)fp.size();
     std::vector<GOp> gops;
     if (!lower(g, ng, n, gops)) return MOONLAB_HIP_ERR_INVALID_QUBIT;
     std::vector<BPass> passes;

@@ -154,7 +154,6 @@ int run_circuit_gates(const RunRequest &rq, const moonlab_hip_gate_t *gl, int ng
     moonlab_hip_state_t *s = nullptr;
     int st = acquire_state(rq.num_qubits, rq.precision, &s);
     if (st) return st;
-    std::vector<moonlab_hip_gate_t> g(gl, gl + ng);
     // a caller-chosen stream (a serving worker's) replaces the pooled state's own for this run
     hipStream_t own = rq.stream ? state_bind_stream(s, (hipStream_t)rq.stream) : nullptr;
     hipStream_t stream = (hipStream_t)moonlab_hip_state_stream(s);
@@ -163,11 +162,14 @@ int run_circuit_gates(const RunRequest &rq, const moonlab_hip_gate_t *gl, int ng
     hipEventCreate(&e1);
     hipEventRecord(e0, stream);
     if (rq.blocked)
-        st = moonlab_hip_apply_gates_blocked(s, g.data(), ng);
+        st = moonlab_hip_apply_gates_blocked(s, gl, ng);
     else if (rq.fusion_max > 0)
-        st = apply_fused(s, g.data(), ng, rq.fusion_max);
+        st = apply_fused(s, gl, ng, rq.fusion_max);
+    else if (rq.per_gate || (rq.precision == MOONLAB_HIP_C64 && rq.num_draws > 0))
+        // complex64 shots: another order of rounding could move an outcome
+        st = moonlab_hip_apply_gates(s, gl, ng);
     else
-        st = moonlab_hip_apply_gates(s, g.data(), ng);
+        st = apply_gates_planned(s, gl, ng);
     if (!st && rq.num_draws > 0) {
         rr.outcomes.resize((size_t)rq.num_draws);
         st = moonlab_hip_sample(s, rq.draws, rq.num_draws, rr.outcomes.data());

@@ -55,6 +55,7 @@ struct RunRequest {
     void               *stream = nullptr;   // run on this HIP stream instead of the state's own
 };
 
+    bool                per_gate = false;   // one kernel per gate, whatever the circuit
 struct RunResult {
     std::vector<uint64_t> outcomes;
     std::vector<double>   amps;         // 2 * 2^n (widened for complex64)

@@ -170,6 +170,7 @@ void run_single(Req *r, int mode, hipStream_t stream)
     rq.want_probs = r->want_probs;
     rq.blocked = mode == 1;
     rq.fusion_max = mode == 2 ? 5 : 0;
+    rq.per_gate = mode == 0;
     rq.stream = stream;
     mlx::RunResult rr;
     r->status = mlx::run_circuit_gates(rq, r->gates.data(), (int)r->gates.size(), rr);

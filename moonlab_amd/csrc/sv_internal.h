@@ -36,6 +36,10 @@ GateTuning &gate_tuning();
 // Record the text moonlab_hip_last_error() returns on this thread (returns st).
 moonlab_hip_status_t set_last_error(moonlab_hip_status_t st, const char *what, hipError_t e = hipSuccess);
 
+// A gate list as rotation passes where those are at most half as many, one
+// kernel per gate otherwise (batch.cpp).
+int apply_gates_planned(moonlab_hip_state_t *s, const moonlab_hip_gate_t *g, int ng);
+
 // Point a state's work at another stream (waits for the state's current
 // stream first); returns the stream it used before.
 hipStream_t state_bind_stream(moonlab_hip_state_t *s, hipStream_t st);
