@@ -12,6 +12,7 @@ from __future__ import annotations
 import ctypes
 import enum
 import os
+import weakref
 from dataclasses import dataclass
 from typing import List, Optional, Sequence, Tuple
 
@@ -441,6 +442,21 @@ class ExecResults:
     num_workers_used: int
 
 
+def _take(results, field: str, count: int, free: str) -> Optional[np.ndarray]:
+    """results.field (count doubles of the library's, or null) as an array
+    that owns them: the library's free function runs when the last view of
+    the array goes."""
+    p = getattr(results, field)
+    if not p:
+        return None
+    buf = (ctypes.c_double * count).from_address(ctypes.addressof(p.contents))
+    keep = type(results)()
+    setattr(keep, field, p)
+    setattr(results, field, None)
+    weakref.finalize(buf, getattr(lib(), free), ctypes.byref(keep)).atexit = False
+    return np.frombuffer(buf, dtype=np.float64)
+
+
 class Job:
     """A moonlab job (scheduler.h:45-210)."""
 
@@ -510,9 +526,9 @@ class Job:
         if rc != MOONLAB_SCHED_OK:
             return rc, None
         out = JobResults(res.num_qubits, res.total_shots,
-                         [res.outcomes[i] for i in range(res.total_shots)],
+                         res.outcomes[:res.total_shots],
                          res.num_workers_used,
-                         [res.worker_seconds[i] for i in range(res.num_workers_used)])
+                         res.worker_seconds[:res.num_workers_used])
         lib().moonlab_job_results_free(ctypes.byref(res))
         return rc, out
 
@@ -535,9 +551,9 @@ class Job:
         try:
             outc = np.ctypeslib.as_array(r.outcomes, (r.total_shots,)).copy() \
                 if r.total_shots else np.zeros(0, np.uint64)
-            amps = np.ctypeslib.as_array(r.amplitudes, (2 * dim,)).copy().view(np.complex128) \
-                if r.amplitudes else None
-            probs = np.ctypeslib.as_array(r.probabilities, (dim,)).copy() if r.probabilities else None
+            amps = _take(r, "amplitudes", 2 * dim, "moonlab_mi355x_results_free")
+            amps = amps.view(np.complex128) if amps is not None else None
+            probs = _take(r, "probabilities", dim, "moonlab_mi355x_results_free")
             z = np.ctypeslib.as_array(r.expect_z, (n,)).copy() if r.expect_z else None
             return ExecResults(n, r.precision, outc, amps, probs, z, r.norm, r.device_seconds,
                                r.wall_seconds, r.num_workers_used)
@@ -627,8 +643,7 @@ class Circuit:
             n = r.num_qubits
             outc = np.ctypeslib.as_array(r.outcomes, (r.num_shots,)).copy() \
                 if r.outcomes else np.zeros(0, np.uint64)
-            probs = np.ctypeslib.as_array(r.probabilities, (1 << n,)).copy() \
-                if r.probabilities else None
+            probs = _take(r, "probabilities", 1 << n, "moonlab_qgtl_results_free")
             return CircuitResults(n, outc, probs)
         finally:
             lib().moonlab_qgtl_results_free(ctypes.byref(r))

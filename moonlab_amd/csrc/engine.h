@@ -3,10 +3,13 @@
 #pragma once
 
 #include <stdint.h>
+#include <stdlib.h>
 
+#include <utility>
 #include <vector>
 
 #include "../../include/moonlab_hip_statevec.h"
+#include "../../include/moonlab_scheduler.h"
 
 namespace mlx {
 
@@ -52,14 +55,44 @@ struct RunRequest {
     bool                want_z;
     int                 fusion_max;     // 0 = unfused
     bool                blocked;        // cache-blocked tile passes
+    bool                per_gate = false;   // one kernel per gate, whatever the circuit
     void               *stream = nullptr;   // run on this HIP stream instead of the state's own
 };
 
-    bool                per_gate = false;   // one kernel per gate, whatever the circuit
+// Doubles the device writes and the C results hand over (free() releases
+// them).  Not cleared, and on 2 MiB pages from 4 MiB up: clearing a vector of
+// the 20-qubit amplitudes first took 3 ms, twice what their download takes.
+class HostBuf {
+  public:
+    HostBuf() = default;
+    HostBuf(HostBuf &&o) noexcept : p_(o.p_), n_(o.n_) { o.p_ = nullptr, o.n_ = 0; }
+    HostBuf &operator=(HostBuf &&o) noexcept
+    {
+        std::swap(p_, o.p_);
+        std::swap(n_, o.n_);
+        return *this;
+    }
+    ~HostBuf() { free(p_); }
+    bool    alloc(size_t n);   // false: out of memory
+    double *data() const { return p_; }
+    size_t  size() const { return n_; }
+    double *release()
+    {
+        double *p = p_;
+        p_ = nullptr;
+        n_ = 0;
+        return p;
+    }
+
+  private:
+    double *p_ = nullptr;
+    size_t  n_ = 0;
+};
+
 struct RunResult {
     std::vector<uint64_t> outcomes;
-    std::vector<double>   amps;         // 2 * 2^n (widened for complex64)
-    std::vector<double>   probs;
+    HostBuf               amps;         // 2 * 2^n (widened for complex64)
+    HostBuf               probs;
     std::vector<double>   z;
     double                norm = 0.0;
     double                device_seconds = 0.0;
@@ -70,5 +103,13 @@ struct RunResult {
 int run_circuit(const RunRequest &rq, RunResult &rr);
 // The same with gates of the full code table (rq.gates is ignored).
 int run_circuit_gates(const RunRequest &rq, const moonlab_hip_gate_t *gates, int num_gates, RunResult &rr);
+
+// The gates and seed of a job of this library's own scheduler.  Absent in
+// the plugin, whose jobs belong to the host process: there the address is null.
+struct JobView {
+    uint64_t                    seed;
+    const std::vector<GateRec> *gates;
+};
+__attribute__((weak, visibility("hidden"))) JobView own_job(const moonlab_job_t *job);
 
 }  // namespace mlx

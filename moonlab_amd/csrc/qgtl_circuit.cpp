@@ -177,11 +177,7 @@ int moonlab_qgtl_execute(moonlab_qgtl_circuit_t *c, const moonlab_qgtl_exec_opti
     memset(out, 0, sizeof(*out));
     out->num_qubits = c->num_qubits;
     out->num_shots = opts->num_shots;
-    if (opts->return_probabilities) {
-        out->probabilities = (double *)malloc(rr.probs.size() * sizeof(double));
-        if (!out->probabilities) return MOONLAB_QGTL_OOM;
-        memcpy(out->probabilities, rr.probs.data(), rr.probs.size() * sizeof(double));
-    }
+    out->probabilities = rr.probs.release();   // null unless asked for
     if (opts->num_shots > 0) {
         out->outcomes = (uint64_t *)malloc((size_t)opts->num_shots * sizeof(uint64_t));
         if (!out->outcomes) {

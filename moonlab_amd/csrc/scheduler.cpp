@@ -61,6 +61,8 @@ void ensure_default(void) { pthread_once(&g_once, register_default); }
 // Process-wide count of completion-hook fires (scheduler.c:30).
 std::atomic<uint64_t> g_mi355x_hook_fires{0};
 
+mlx::JobView mlx::own_job(const moonlab_job_t *job) { return {job->rng_seed, &job->gates}; }
+
 extern "C" {
 
 moonlab_job_t *moonlab_job_create(int n)

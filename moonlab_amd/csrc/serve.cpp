@@ -54,7 +54,7 @@ struct Req {
     bool                            done = false;
     std::vector<uint64_t>           outcomes;
     std::vector<double>             z;
-    std::vector<double>             probs;
+    mlx::HostBuf                    probs;
     double                          norm = 0;
 };
 
