@@ -672,8 +672,12 @@ int blocked_shape(int n, int prec, const GateTuning &t, bool *reg, int *anchor, 
 // engine's (figures at k_frame_pass).  False where another engine stays: the
 // state has under 4 qubits (four register bits), or a parameter is not finite
 // (a rotation would spread it to amplitudes that the gate leaves alone).
-bool plan_frames(const moonlab_hip_gate_t *g, int ng, int n, int prec, const GateTuning &t, int lookahead,
-                 std::vector<FPass> &passes, std::vector<FOp> &prog)
+// One lookahead seed for four of the op engines': the rotations' tile sets and
+// bases gain nothing past two (30 qubits, depth 10: 22 passes without, 12 with
+// two, 13 with eight, 97 against 101 ms; 27 qubits, depth 25, complex64: 13.8
+// against 14.4 ms), and two plan in half the time of eight.
+bool plan_frames(const moonlab_hip_gate_t *g, int ng, int n, int prec, const GateTuning &t, std::vector<FPass> &passes,
+                 std::vector<FOp> &prog)
 {
     if (n < kFrameRegBits) return false;
     std::vector<FGate> fg;
@@ -681,7 +685,8 @@ bool plan_frames(const moonlab_hip_gate_t *g, int ng, int n, int prec, const Gat
     if (!frame_lower(g, ng, n, fg, phase)) return false;
     const bool c64 = prec == MOONLAB_HIP_C64;
     const int want = t.blocked_tile_bits ? t.blocked_tile_bits : (c64 ? 13 : 12);
-    frame_plan(fg, phase, n, want >= 13 && n >= 13 ? 13 : 12, c64 ? 4 : 3, c64 ? 8 : 16, lookahead, passes, prog);
+    frame_plan(fg, phase, n, want >= 13 && n >= 13 ? 13 : 12, c64 ? 4 : 3, c64 ? 8 : 16,
+               (t.blocked_lookahead + 3) / 4, passes, prog);
     prog.push_back(FOp{});   // the kernels fetch one unit past the last rotation
     return true;
 }
@@ -1125,12 +1130,7 @@ int mlx::apply_gates_planned(moonlab_hip_state_t *s, const moonlab_hip_gate_t *g
     // one kernel per gate where the passes would not save half of them: a
     // pass takes as long as 1 to 1.5 gate kernels at 30 qubits (7-9 ms, 5.4 ms)
     const int n = (int)moonlab_hip_state_n_qubits(s);
-    const GateTuning tune = gate_tuning();
-    // Lookahead: two seeds plan 800 gates on 20 qubits into 12 passes in half
-    // the time (0.2 ms) of the eight the blocked path takes (13 passes); none
-    // makes 22.  From 26 qubits on a pass (0.5 ms) is worth more than planning.
-    const int look = n < 26 ? std::min(2, tune.blocked_lookahead) : tune.blocked_lookahead;
-    if (ng > 1 && plan_frames(g, ng, n, moonlab_hip_state_precision(s), tune, look, fp, prog) &&
+    if (ng > 1 && plan_frames(g, ng, n, moonlab_hip_state_precision(s), gate_tuning(), fp, prog) &&
         2 * fp.size() <= (size_t)ng) {
         const hipError_t e = run_frames(s, fp, prog);
         if (e == hipSuccess) return MOONLAB_HIP_OK;
@@ -1158,8 +1158,7 @@ moonlab_hip_status_t moonlab_hip_apply_gates_blocked(moonlab_hip_state_t *s, con
     };
     std::vector<FPass> fp;
     std::vector<FOp> prog;
-    if (tune.blocked_engine == 0 && plan_frames(g, ng, n, prec, tune, tune.blocked_lookahead, fp, prog))
-        return status(run_frames(s, fp, prog));
+    if (tune.blocked_engine == 0 && plan_frames(g, ng, n, prec, tune, fp, prog)) return status(run_frames(s, fp, prog));
     std::vector<GOp> gops;
     if (!lower(g, ng, n, gops)) return MOONLAB_HIP_ERR_INVALID_QUBIT;
     std::vector<BPass> passes;
@@ -1200,7 +1199,7 @@ int moonlab_hip_blocked_pass_count(const moonlab_hip_gate_t *g, int ng, int n, i
     std::vector<FPass> fp;
     std::vector<FOp> prog;
     const GateTuning tune = gate_tuning();
-    if (tune.blocked_engine == 0 && plan_frames(g, ng, n, precision, tune, tune.blocked_lookahead, fp, prog))
+    if (tune.blocked_engine == 0 && plan_frames(g, ng, n, precision, tune, fp, prog))
         return (int)fp.size();
     std::vector<GOp> gops;
     if (!lower(g, ng, n, gops)) return MOONLAB_HIP_ERR_INVALID_QUBIT;
