@@ -382,6 +382,73 @@ std::vector<FusedBlock> plan_fusion_best(const moonlab_hip_gate_t *g, int ng, in
     return b.size() < a.size() ? b : a;
 }
 
+std::vector<BlockTile> plan_block_tiles(const std::vector<FusedBlock> &blocks, int n, int tile, int anchor)
+{
+    std::vector<uint64_t> mask(blocks.size(), 0);
+    for (size_t i = 0; i < blocks.size(); i++)
+        for (int q : blocks[i].qubits) mask[i] |= 1ull << q;
+    const uint64_t low = (1ull << anchor) - 1ull;
+    std::vector<int> rest(blocks.size()), left;
+    for (size_t i = 0; i < rest.size(); i++) rest[i] = (int)i;
+    // the pending blocks that fit in `set` (or in what it grows to), in order;
+    // stops once every qubit of the set is held by a block put off
+    auto scan = [&](uint64_t &set, bool grow, std::vector<int> *take, std::vector<int> *off) {
+        uint64_t held = 0;
+        size_t got = 0, k = 0;
+        for (; k < rest.size() && (grow || (set & ~held)); k++) {
+            const uint64_t m = mask[(size_t)rest[k]];
+            const bool fits = !(m & held) && (!(m & ~set) || (grow && __builtin_popcountll(set | m) <= tile));
+            if (fits) {
+                if (grow) set |= m;
+                got++;
+                if (take) take->push_back(rest[k]);
+            } else {
+                held |= m;
+                if (off) off->push_back(rest[k]);
+            }
+        }
+        if (off) off->insert(off->end(), rest.begin() + (long)k, rest.end());
+        return got;
+    };
+    std::vector<BlockTile> out;
+    while (!rest.empty()) {
+        uint64_t best = low;
+        size_t most = scan(best, true, nullptr, nullptr);
+        for (int s = anchor; s + (tile - anchor) <= n; s++) {
+            uint64_t w = low | (((1ull << (tile - anchor)) - 1ull) << s);
+            const size_t got = scan(w, false, nullptr, nullptr);
+            if (got > most) most = got, best = w;
+        }
+        // the greedy set takes the first pending block at least
+        BlockTile t;
+        left.clear();
+        scan(best, false, &t.members, &left);
+        for (int q = 0; q < n && __builtin_popcountll(best) < tile; q++) best |= 1ull << q;
+        t.qubits = best;
+        rest.swap(left);
+        out.push_back(std::move(t));
+    }
+    return out;
+}
+
+std::vector<cd> widen_block(const FusedBlock &b, const std::vector<int> &qubits)
+{
+    const size_t D = (size_t)1 << qubits.size(), d = (size_t)1 << b.qubits.size();
+    std::vector<size_t> own(D, 0);   // b's row of row r
+    size_t inside = 0;               // bits of r that are b's
+    for (size_t j = 0, k = 0; j < qubits.size(); j++) {
+        if (k >= b.qubits.size() || b.qubits[k] != qubits[j]) continue;
+        inside |= (size_t)1 << j;
+        for (size_t r = 0; r < D; r++) own[r] |= (r >> j & 1) << k;
+        k++;
+    }
+    std::vector<cd> m(D * D, cd(0.0));
+    for (size_t r = 0; r < D; r++)
+        for (size_t c = 0; c < D; c++)
+            if (((r ^ c) & ~inside) == 0) m[r * D + c] = b.mat[own[r] * d + own[c]];
+    return m;
+}
+
 int apply_fused(moonlab_hip_state_t *s, const moonlab_hip_gate_t *g, int ng, int kmax)
 {
     for (int i = 0; i < ng; i++) {
@@ -400,26 +467,56 @@ int apply_fused(moonlab_hip_state_t *s, const moonlab_hip_gate_t *g, int ng, int
                   (hipStream_t)moonlab_hip_state_stream(s)};
     const bool f = d.prec == MOONLAB_HIP_C64;
     const size_t ab = f ? 8 : 16;
-    // every matrix of 3+ qubits goes to the device in one copy
-    std::vector<size_t> off(blocks.size(), 0);
-    size_t total = 0;
-    for (size_t i = 0; i < blocks.size(); i++)
-        if (blocks[i].qubits.size() >= 3 && !blocks[i].only_gate) {
-            off[i] = total;
-            total += blocks[i].mat.size() * ab;
-        }
-    std::vector<unsigned char> host(total);
-    for (size_t i = 0; i < blocks.size(); i++) {
-        if (blocks[i].qubits.size() < 3 || blocks[i].only_gate) continue;
-        const std::vector<cd> &m = blocks[i].mat;
-        if (f) {
-            float *p = (float *)(host.data() + off[i]);
-            for (size_t j = 0; j < m.size(); j++) { p[2 * j] = (float)m[j].real(); p[2 * j + 1] = (float)m[j].imag(); }
-        } else {
-            double *p = (double *)(host.data() + off[i]);
-            for (size_t j = 0; j < m.size(); j++) { p[2 * j] = m[j].real(); p[2 * j + 1] = m[j].imag(); }
+    // Passes over the state: tiles of several blocks where the state has one
+    // (128 contiguous bytes at least: the lowest 4 or 3 qubits in every tile),
+    // else one block each.
+    std::vector<BlockTile> tiles;
+    if (d.n >= kDenseTileBits) {
+        tiles = plan_block_tiles(blocks, d.n, kDenseTileBits, f ? 4 : 3);
+    } else {
+        tiles.resize(blocks.size());
+        for (size_t i = 0; i < blocks.size(); i++) tiles[i].members.push_back((int)i);
+    }
+    // steps and every matrix of 3+ qubits go to the device in one copy
+    std::vector<DenseStep> steps;
+    std::vector<unsigned char> mats;
+    std::vector<size_t> first(tiles.size(), 0), off(blocks.size(), 0);
+    std::vector<bool> joint(tiles.size(), false);
+    for (size_t t = 0; t < tiles.size(); t++) {
+        // a lone gate's own kernel reads half of the state or less
+        double passes = 0.0;
+        for (int i : tiles[t].members) passes += blocks[(size_t)i].only_gate ? 0.5 : 1.0;
+        joint[t] = tiles[t].members.size() > 1 && passes >= 1.5;
+        first[t] = steps.size();
+        for (int i : tiles[t].members) {
+            const FusedBlock &b = blocks[(size_t)i];
+            const size_t at = off[(size_t)i] = mats.size();
+            if (joint[t]) {
+                std::vector<int> qs = b.qubits;
+                for (int q = 0; qs.size() < 3; q++)
+                    if ((tiles[t].qubits >> q & 1) && std::find(b.qubits.begin(), b.qubits.end(), q) == b.qubits.end())
+                        qs.push_back(q);
+                std::sort(qs.begin(), qs.end());
+                const int k = (int)qs.size();
+                int local[5];
+                for (int j = 0; j < k; j++) local[j] = __builtin_popcountll(tiles[t].qubits & ((1ull << qs[(size_t)j]) - 1ull));
+                steps.emplace_back();
+                dense_step(steps.back(), d.prec, k, local, (uint32_t)(at / 16));
+                mats.resize(at + dense_operand_bytes(d.prec, k));
+                dense_operand(d.prec, k, (k == (int)b.qubits.size() ? b.mat : widen_block(b, qs)).data(), &mats[at]);
+            } else if (b.qubits.size() >= 3 && !b.only_gate) {
+                mats.resize(at + b.mat.size() * ab);
+                for (size_t j = 0; j < b.mat.size(); j++) {
+                    const float v[2] = {(float)b.mat[j].real(), (float)b.mat[j].imag()};
+                    memcpy(&mats[at + j * ab], f ? (const void *)v : (const void *)&b.mat[j], ab);
+                }
+            }
         }
     }
+    const size_t at = (steps.size() * sizeof(DenseStep) + 255) / 256 * 256, total = at + mats.size();
+    std::vector<unsigned char> host(total);
+    if (!steps.empty()) memcpy(host.data(), steps.data(), steps.size() * sizeof(DenseStep));
+    if (!mats.empty()) memcpy(host.data() + at, mats.data(), mats.size());
     void *dm = nullptr;
     hipError_t e = hipSuccess;
     if (total) {
@@ -427,24 +524,33 @@ int apply_fused(moonlab_hip_state_t *s, const moonlab_hip_gate_t *g, int ng, int
         if (e == hipSuccess) e = hipMemcpyAsync(dm, host.data(), total, hipMemcpyHostToDevice, d.stream);
         if (e == hipSuccess) e = hipStreamSynchronize(d.stream);   // `host` is local
     }
+    const char *d_mats = (const char *)dm + at;
     std::vector<double> m2;
-    for (size_t i = 0; e == hipSuccess && i < blocks.size(); i++) {
-        const FusedBlock &b = blocks[i];
-        const int k = (int)b.qubits.size();
-        if (b.only_gate) {   // a lone gate keeps its own kernel (a CZ touches a quarter of the state)
-            e = launch_gate(d, *b.only_gate);
+    for (size_t t = 0; e == hipSuccess && t < tiles.size(); t++) {
+        if (joint[t]) {
+            e = launch_block_tiles(d, tiles[t].qubits, (const DenseStep *)dm + first[t], (int)tiles[t].members.size(),
+                                   d_mats);
             continue;
         }
-        if (k >= 3) {
-            e = launch_dense_dev(d, k, b.qubits.data(), (const char *)dm + off[i]);
-            continue;
+        for (size_t i = 0; e == hipSuccess && i < tiles[t].members.size(); i++) {
+            const FusedBlock &b = blocks[(size_t)tiles[t].members[i]];
+            const int k = (int)b.qubits.size();
+            if (b.only_gate) {   // its own kernel (a CZ touches a quarter of the state)
+                e = launch_gate(d, *b.only_gate);
+                continue;
+            }
+            if (k >= 3) {
+                e = launch_dense_dev(d, k, b.qubits.data(), d_mats + off[(size_t)tiles[t].members[i]]);
+                continue;
+            }
+            m2.resize(b.mat.size() * 2);
+            for (size_t j = 0; j < b.mat.size(); j++) {
+                m2[2 * j] = b.mat[j].real();
+                m2[2 * j + 1] = b.mat[j].imag();
+            }
+            e = k == 1 ? launch_matrix_1q(d, b.qubits[0], m2.data())
+                       : launch_matrix_2q(d, b.qubits[0], b.qubits[1], m2.data());
         }
-        m2.resize(b.mat.size() * 2);
-        for (size_t j = 0; j < b.mat.size(); j++) {
-            m2[2 * j] = b.mat[j].real();
-            m2[2 * j + 1] = b.mat[j].imag();
-        }
-        e = k == 1 ? launch_matrix_1q(d, b.qubits[0], m2.data()) : launch_matrix_2q(d, b.qubits[0], b.qubits[1], m2.data());
     }
     if (dm) hipFreeAsync(dm, d.stream);
     if (e == hipErrorOutOfMemory) return MOONLAB_HIP_ERR_OUT_OF_MEMORY;

@@ -47,6 +47,22 @@ constexpr int kFusionSeeds = 8;
 std::vector<FusedBlock> plan_fusion_windows(const moonlab_hip_gate_t *g, int ng, int kmax, int seeds, int n);
 std::vector<FusedBlock> plan_fusion_best(const moonlab_hip_gate_t *g, int ng, int kmax);
 
+// Blocks that one pass over the state applies: a set of `tile` qubits and the
+// members (indices into the plan) that act inside it, in order.
+struct BlockTile {
+    uint64_t         qubits = 0;
+    std::vector<int> members;
+};
+
+// The plan's blocks in passes over tiles of `tile` qubits, each keeping the
+// lowest `anchor`: blocks move past pending ones on other qubits only.  A
+// tile is the one of all windows of neighbouring qubits (and of the set grown
+// greedily) that takes the most pending blocks.
+std::vector<BlockTile> plan_block_tiles(const std::vector<FusedBlock> &blocks, int n, int tile, int anchor);
+
+// Block b's unitary on `qubits` (ascending, a superset of b.qubits).
+std::vector<cd> widen_block(const FusedBlock &b, const std::vector<int> &qubits);
+
 // Apply a gate list through fusion (returns a moonlab_hip_status_t value).
 int apply_fused(moonlab_hip_state_t *s, const moonlab_hip_gate_t *g, int ng, int kmax);
 

@@ -6,6 +6,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <complex>
+
 #include "../../include/moonlab_hip_statevec.h"
 
 namespace mlx {
@@ -39,6 +41,25 @@ moonlab_hip_status_t set_last_error(moonlab_hip_status_t st, const char *what, h
 // A gate list as rotation passes where those are at most half as many, one
 // kernel per gate otherwise (batch.cpp).
 int apply_gates_planned(moonlab_hip_state_t *s, const moonlab_hip_gate_t *g, int ng);
+
+// One block of a pass over 12-qubit tiles (k_block_tiles): local bits q
+// (ascending, qmask), the LDS slot of each block row, and where the matrix's
+// operands start in the pass's buffer, in 16-byte chunks.
+constexpr int kDenseTileBits = 12;
+struct DenseStep {
+    int32_t  k;          // 3..5
+    uint32_t mat;
+    uint32_t qmask;
+    int32_t  q[5];
+    uint32_t row[32];
+};
+void dense_step(DenseStep &st, int prec, int k, const int *local, uint32_t mat);
+// A k-qubit matrix (row-major) as the operands the pass reads, and their size.
+size_t dense_operand_bytes(int prec, int k);
+void   dense_operand(int prec, int k, const std::complex<double> *m, void *out);
+// nsteps blocks inside the tile set `qubits` (kDenseTileBits of them, the low
+// one among them); steps and matrices on the device
+hipError_t launch_block_tiles(const SvDev &s, uint64_t qubits, const DenseStep *d_steps, int nsteps, const void *d_mats);
 
 // Point a state's work at another stream (waits for the state's current
 // stream first); returns the stream it used before.

@@ -28,6 +28,8 @@
 // D[4 v + l / 16][l % 16] for FP64.  The FP64 path loads A with its rows
 // permuted (A row i = real row 4 (i % 4) + i / 4), which puts both results in
 // the FP32 order, so one write-back serves both.
+#include "batch_device.h"
+#include "frame_device.h"
 #include "sv_device.h"
 #include "sv_internal.h"
 
@@ -46,7 +48,7 @@ template <> struct Acc<float> {
         return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
     }
     // real-matrix row that A row i (= lane % 16) carries
-    static __device__ __forceinline__ int a_row(int i) { return i; }
+    static __host__ __device__ __forceinline__ int a_row(int i) { return i; }
 };
 template <> struct Acc<double> {
     using type = mfma_d4;
@@ -54,7 +56,7 @@ template <> struct Acc<double> {
     {
         return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
     }
-    static __device__ __forceinline__ int a_row(int i) { return 4 * (i & 3) + (i >> 2); }
+    static __host__ __device__ __forceinline__ int a_row(int i) { return 4 * (i & 3) + (i >> 2); }
 };
 
 // 16-byte global slot: one complex128 amplitude or two adjacent complex64
@@ -168,10 +170,10 @@ struct Block {
     // Block row of accumulator v of lane group q = l / 16 in a 16-row tile
     // of the 3M products: (v & 1) + 2 q + 8 (v / 2), so one store (fixed v)
     // covers rows that differ in bits 1..2, as in the real-embedding form.
-    static __device__ __forceinline__ int m3_row(int v, int q) { return (v & 1) + 2 * q + 8 * (v >> 1); }
+    static __host__ __device__ __forceinline__ int m3_row(int v, int q) { return (v & 1) + 2 * q + 8 * (v >> 1); }
     // block row that A row i carries: accumulator v holds D[4 q + v] for
     // FP32 and D[4 v + q] for FP64
-    static __device__ __forceinline__ int m3_arow(int i)
+    static __host__ __device__ __forceinline__ int m3_arow(int i)
     {
         if constexpr (sizeof(R) == 4) return m3_row(i & 3, i >> 2);
         else return m3_row(i >> 2, i & 3);
@@ -199,6 +201,48 @@ struct Block {
                 }
             }
     }
+    // The same operands from the order k_block_tiles reads them in: entry e =
+    // NS rt + s of lane l (a complex, or the one real of the real embedding)
+    // lies in 16-byte chunk 64 (e / EPC) + l, so a wave's load is contiguous.
+    static constexpr int ENTRIES = NRT * NS, EPC = 16 / ((M3 ? 2 : 1) * (int)sizeof(R));
+    __device__ __forceinline__ void load_ordered(const float4 *p, int lane)
+    {
+#pragma unroll
+        for (int c = 0; c < ENTRIES / EPC; c++) {
+            const float4 x = p[64 * c + lane];
+            R v[16 / sizeof(R)];
+            __builtin_memcpy(v, &x, 16);
+#pragma unroll
+            for (int i = 0; i < EPC; i++) {
+                const int e = EPC * c + i, rt = e / NS, s = e % NS;
+                if constexpr (M3) {
+                    Am[0][rt][s] = v[2 * i];
+                    Am[1][rt][s] = v[2 * i + 1];
+                    Am[2][rt][s] = v[2 * i] + v[2 * i + 1];
+                } else {
+                    Am[0][rt][s] = v[i];
+                }
+            }
+        }
+    }
+    static void order(const std::complex<double> *m, R *out)
+    {
+        for (int l = 0; l < 64; l++)
+            for (int e = 0; e < ENTRIES; e++) {
+                const int rt = e / NS, col = 4 * (e % NS) + (l >> 4);
+                R *o = out + (16 / sizeof(R)) * (size_t)(64 * (e / EPC) + l) + (M3 ? 2 : 1) * (e % EPC);
+                if constexpr (M3) {
+                    const std::complex<double> x = m[(16 * rt + m3_arow(l & 15)) * D + col];
+                    o[0] = (R)x.real();
+                    o[1] = (R)x.imag();
+                } else {
+                    const int row = 16 * rt + AccT::a_row(l & 15);
+                    const std::complex<double> x = m[(row >> 1) * D + (col >> 1)];
+                    const int ra = row & 1, cb = col & 1;
+                    o[0] = (R)(ra == cb ? x.real() : (ra == 0 ? -x.imag() : x.imag()));
+                }
+            }
+    }
     // real embedding: accumulator v of row tile rt holds real row
     // 16 rt + 4 (l / 16) + v (the FP64 A rows are permuted by a_row to give
     // the FP32 order), i.e. block row 8 rt + 2 (l / 16) + v / 2
@@ -207,7 +251,9 @@ struct Block {
         if constexpr (M3) return 16 * (o >> 2) + m3_row(o & 3, lane >> 4);
         else return 8 * (o >> 1) + 2 * (lane >> 4) + (o & 1);
     }
-    // get(c): amplitude c of this lane's group; put(o, y): output o
+    // block row of this lane's B operand at step s
+    static __device__ __forceinline__ int in_row(int s, int lane) { return M3 ? 4 * s + (lane >> 4) : 2 * s + (lane >> 5); }
+    // get(s): amplitude in_row(s) of this lane's group; put(o, y): output o
     template <class Get, class Put>
     __device__ __forceinline__ void apply(int lane, Get get, Put put) const
     {
@@ -215,7 +261,7 @@ struct Block {
             R br[NS], bi[NS], bs[NS];
 #pragma unroll
             for (int s = 0; s < NS; s++) {
-                const cplx_t<R> x = get(4 * s + (lane >> 4));
+                const cplx_t<R> x = get(s);
                 br[s] = x.x;
                 bi[s] = x.y;
                 bs[s] = x.x + x.y;
@@ -240,9 +286,8 @@ struct Block {
             R B[NS];
 #pragma unroll
             for (int s = 0; s < NS; s++) {
-                const int kk = 4 * s + (lane >> 4);
-                const cplx_t<R> x = get(kk >> 1);
-                B[s] = (kk & 1) ? x.y : x.x;
+                const cplx_t<R> x = get(s);
+                B[s] = (lane & 16) ? x.y : x.x;
             }
             typename AccT::type acc[NRT];
 #pragma unroll
@@ -337,7 +382,7 @@ __global__ __launch_bounds__(kThreads) void k_dense_mfma(cplx_t<R> *__restrict__
             const int g = 64 * j + 16 * wave + (lane & 15);
             const int go = offg_lo[g & 63] | offg_hi[g >> 6];
             blk.apply(
-                lane, [&](int c) { return lds[padded(offq[c] | go)]; },
+                lane, [&](int s) { return lds[padded(offq[Block<R, K>::in_row(s, lane)] | go)]; },
                 [&](int o, const cplx_t<R> &y) { lds[padded(offq[Block<R, K>::out_row(o, lane)] | go)] = y; });
         }
         lds_barrier();
@@ -346,6 +391,101 @@ __global__ __launch_bounds__(kThreads) void k_dense_mfma(cplx_t<R> *__restrict__
         for (int i = 0; i < PER; i++)
             st_slot<NT>((SlotT *)&a[base | dhi[hi0 + HSTEP * i]], get_slot(lds, padded(A * (tid + kThreads * i))));
         lds_barrier();   // every wave has read its write-back values before the next tile lands
+    }
+}
+
+// Several blocks in one pass: a workgroup holds a tile of 2^12 amplitudes in
+// LDS and applies every block whose qubits lie inside, so the state crosses
+// HBM once for all of them: 2.6 five-qubit (4.5 four-qubit, 7 three-qubit)
+// blocks of SU(2) + CZ layers.  Bound by the matrix cores, 64 to 76 % busy (one
+// block per pass was bound by HBM, at 5.3 TB/s): depth 12 on 31 qubits,
+// complex64, 414 -> 292 ms in five-qubit blocks, 589 -> 229 in four-qubit ones
+// and 1214 -> 378 in three-qubit ones; 30 qubits complex128 417 -> 297, 594 ->
+// 240 and 1290 -> 405 ms.  12-qubit tiles: 13 qubits take 4 % fewer passes
+// with half the workgroups on a CU to overlap them.
+constexpr int kBlockTileBits = kDenseTileBits;
+
+// LDS slot of tile index x: linear over GF(2), bits that lanes differ in
+// folded onto the bank bits; bit 0 stays, so complex64 pairs stay together.
+template <typename R> __device__ __forceinline__ uint32_t tile_slot(uint32_t x)
+{
+    if constexpr (sizeof(R) == 8) return (uint32_t)lds_slot<16>((int)x);
+    else return x ^ ((x >> 4 ^ x >> 8) & 14u);
+}
+
+template <typename R, int K>
+__device__ __forceinline__ void tile_block(cplx_t<R> *lds, FConst<DenseStep> st, const float4 *mats, int lane,
+                                           int wave)
+{
+    using B = Block<R, K>;
+    B blk;
+    blk.load_ordered(mats, lane);
+    // rows as slots: the lane's part and, by step or output, a uniform part
+    const int qi = B::M3 ? lane >> 4 : lane >> 5, qo = lane >> 4;
+    const uint32_t rin = (qi & 1 ? st->row[1] : 0u) ^ (qi & 2 ? st->row[2] : 0u);
+    const uint32_t rout = (qo & 1 ? st->row[2] : 0u) ^ (qo & 2 ? st->row[4] : 0u);
+    uint32_t x = (uint32_t)(lane & 15) | (uint32_t)wave << 4, step = 64u;
+    for (int j = 0; j < K; j++) {
+        const uint32_t low = (1u << st->q[j]) - 1u;
+        x += x & ~low;
+        step += step & ~low;
+    }
+#pragma unroll 1
+    for (int it = 0; it < (1 << (kBlockTileBits - K - 6)); it++) {
+        const uint32_t g = tile_slot<R>(x);
+        blk.apply(
+            lane, [&](int s) { return lds[g ^ rin ^ st->row[B::M3 ? 4 * s : 2 * s]]; },
+            [&](int o, const cplx_t<R> &y) {
+                lds[g ^ rout ^ st->row[B::M3 ? 16 * (o >> 2) + (o & 1) + 8 * ((o >> 1) & 1) : o]] = y;
+            });
+        x = ((x | st->qmask) + step) & ~st->qmask;
+    }
+}
+
+// The tile's loads wait for nothing but each other and nothing runs ahead: a
+// CU's other workgroups (four for complex64, two for complex128) cover them.
+// Keeping the matrices in LDS and loading the next tile during the products
+// measured the same (288 ms against 292 for 66 blocks of 31 qubits).
+template <typename R, bool NT>
+__global__ __launch_bounds__(kThreads, sizeof(R) == 8 ? 2 : 4) void
+k_block_tiles(cplx_t<R> *__restrict__ a, uint64_t ntiles, uint64_t mask, const DenseStep *__restrict__ steps,
+              int nsteps, const float4 *__restrict__ mats)
+{
+    constexpr int T = 1 << kBlockTileBits, A = Slot<R>::A, PER = T / A / kThreads, HSTEP = kThreads * A / 64;
+    using SlotT = typename Slot<R>::type;
+    __shared__ cplx_t<R> lds[T];
+    __shared__ uint64_t dlo[64], dhi[T / 64];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if (tid < 64) dlo[tid] = frame_deposit((uint64_t)tid, mask);
+    else if (tid < 128) dhi[tid - 64] = frame_deposit((uint64_t)(tid - 64) << 6, mask);
+    __syncthreads();
+    const uint64_t lo = dlo[A * (tid & (64 / A - 1))];
+    const int hi0 = tid / (64 / A);
+    const TileWalk walk{blockIdx.x, gridDim.x, ntiles};
+    uint64_t base = frame_uniform(frame_deposit(walk.t, ~mask));
+    const uint64_t bstep = frame_uniform(frame_deposit(walk.step, ~mask));
+    for (uint64_t t = walk.t; t < walk.end; t += walk.step) {
+        SlotT in[PER];
+#pragma unroll
+        for (int i = 0; i < PER; i++) in[i] = ld_slot<NT>((const SlotT *)&a[(base | lo) | dhi[hi0 + HSTEP * i]]);
+#pragma unroll
+        for (int i = 0; i < PER; i++) put_slot(lds, (int)tile_slot<R>(A * (tid + kThreads * i)), in[i]);
+        lds_barrier();
+        for (int b = 0; b < nsteps; b++) {
+            const FConst<DenseStep> st = (FConst<DenseStep>)(uintptr_t)(steps + b);
+            const float4 *m = mats + st->mat;
+            if (st->k == 5) tile_block<R, 5>(lds, st, m, lane, wave);
+            else if (st->k == 4) tile_block<R, 4>(lds, st, m, lane, wave);
+            else tile_block<R, 3>(lds, st, m, lane, wave);
+            lds_barrier();
+        }
+#pragma unroll
+        for (int i = 0; i < PER; i++)
+            st_slot<NT>((SlotT *)&a[(base | lo) | dhi[hi0 + HSTEP * i]],
+                        get_slot(lds, (int)tile_slot<R>(A * (tid + kThreads * i))));
+        base = frame_step(base, bstep, mask);
+        lds_barrier();   // every thread has read its values before the next tile lands
     }
 }
 
@@ -434,7 +574,66 @@ hipError_t dispatch_k(const SvDev &s, const int *qubits, const void *d_mat, bool
     return hipErrorInvalidValue;
 }
 
+template <typename R, bool NT>
+void run_block_tiles(const SvDev &s, uint64_t mask, const DenseStep *steps, int nsteps, const void *mats,
+                     uint64_t ntiles)
+{
+    // as many tiles per workgroup as the rotation passes take, for the same reasons
+    uint64_t per = 8;
+    while (per > 1 && ntiles / per < 1024) per >>= 1;
+    k_block_tiles<R, NT><<<(unsigned)(ntiles / per), kThreads, 0, s.stream>>>((cplx_t<R> *)s.amps, ntiles, mask, steps,
+                                                                             nsteps, (const float4 *)mats);
+}
+
 }  // namespace
+
+void dense_step(DenseStep &st, int prec, int k, const int *local, uint32_t mat)
+{
+    st = DenseStep{};
+    st.k = k;
+    st.mat = mat;
+    for (int j = 0; j < k; j++) {
+        st.q[j] = local[j];
+        st.qmask |= 1u << local[j];
+    }
+    for (int r = 0; r < (1 << k); r++) {
+        uint32_t x = 0;
+        for (int j = 0; j < k; j++) x |= (uint32_t)(r >> j & 1) << local[j];
+        st.row[r] = prec == MOONLAB_HIP_C64 ? x ^ ((x >> 4 ^ x >> 8) & 14u) : (uint32_t)lds_slot<16>((int)x);
+    }
+}
+
+size_t dense_operand_bytes(int prec, int k)
+{
+    // 4^k complex entries; the real embedding of 3 qubits holds 256 reals
+    return (prec == MOONLAB_HIP_C64 ? 8 : 16) * (k == 3 ? (size_t)128 : (size_t)1 << (2 * k));
+}
+
+void dense_operand(int prec, int k, const std::complex<double> *m, void *out)
+{
+    auto go = [&](auto r) {
+        using R = decltype(r);
+        if (k == 5) Block<R, 5>::order(m, (R *)out);
+        else if (k == 4) Block<R, 4>::order(m, (R *)out);
+        else Block<R, 3>::order(m, (R *)out);
+    };
+    if (prec == MOONLAB_HIP_C64) go(float());
+    else go(double());
+}
+
+hipError_t launch_block_tiles(const SvDev &s, uint64_t qubits, const DenseStep *d_steps, int nsteps, const void *d_mats)
+{
+    if (__builtin_popcountll(qubits) != kDenseTileBits || s.n < kDenseTileBits || (s.n < 64 && qubits >> s.n))
+        return hipErrorInvalidValue;
+    const bool f = s.prec == MOONLAB_HIP_C64;
+    const uint64_t ntiles = 1ull << (s.n - kDenseTileBits);
+    const bool nt = (1ull << s.n) * (f ? 8ull : 16ull) >= gate_tuning().nt_min_bytes;
+    if (f) nt ? run_block_tiles<float, true>(s, qubits, d_steps, nsteps, d_mats, ntiles)
+              : run_block_tiles<float, false>(s, qubits, d_steps, nsteps, d_mats, ntiles);
+    else nt ? run_block_tiles<double, true>(s, qubits, d_steps, nsteps, d_mats, ntiles)
+            : run_block_tiles<double, false>(s, qubits, d_steps, nsteps, d_mats, ntiles);
+    return hipGetLastError();
+}
 
 // Dense k-qubit block on the matrix cores; false when the state is too small
 // for a 2^(k+6)-amplitude tile (the caller then uses the VALU kernel).
