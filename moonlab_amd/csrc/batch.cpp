@@ -47,10 +47,13 @@ hipError_t launch_reg_pass(void *amps, int prec, int n, const BPass &P, const BO
 hipError_t launch_frame_pass(void *amps, int prec, int n, const FPass &P, const FPass *d_pass, const FOp *d_prog,
                              hipStream_t st);
 
-hipError_t launch_batch(const BInst *insts, const int32_t *order, int n128, int n64, int *counter, const FPass *passes,
-                        const FOp *prog, double2 *scratch, uint64_t slot_amps, double *tile_scratch,
+hipError_t launch_batch(int prec, const BInst *insts, const int32_t *order, int count, int *counter, const FPass *passes,
+                        const FOp *prog, double2 *scratch, uint64_t slot_amps, double2 *own, double *tile_scratch,
                         uint64_t tile_slot, const double *draws, double *obs, uint64_t *outcomes,
                         const PauliT *terms, void *state_out, int grid, hipStream_t st);
+hipError_t launch_batch_pass(int prec, const BInst *insts, const int32_t *list, const int32_t *first_tile, int count,
+                             int level, int tiles, const FPass *passes, const FOp *prog, double2 *own, hipStream_t st);
+hipError_t launch_reset_counters(int *counters, hipStream_t st);
 
 // A Pauli string over n qubits (s[q] in "IXYZ" acts on qubit q, strlen == n,
 // pauli_term_t of vqe.h:101-105) as masks; false on any other character or
@@ -751,6 +754,9 @@ struct moonlab_mi355x_batch {
     void       *d_scratch = nullptr;
     size_t      scratch_cap = 0;
     hipEvent_t  e0 = nullptr, e1 = nullptr;
+    // the complex64 circuits of a mixed batch run beside the complex128 ones
+    hipStream_t aux = nullptr;
+    hipEvent_t  fork = nullptr, join = nullptr;
     // HIP graph of the last batch shape (see moonlab_mi355x_batch_set_graphs)
     bool            use_graphs = true;
     hipGraphExec_t  gexec = nullptr;
@@ -819,6 +825,11 @@ int host_threads(size_t gates, int parts)
     return (int)std::min(most, 1 + gates / 1000);
 }
 
+// One workgroup's time on a tile (12 qubits, complex128): a pass's loads,
+// layouts and stores, each rotation or frame gate of the circuit, and a
+// launch of one pass of many circuits, in microseconds as measured.
+constexpr double kTilePassUs = 6.0, kTileGateUs = 0.25, kLevelUs = 20.0;
+
 int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int count,
               moonlab_mi355x_batch_stats_t *stats, const BatchStateOut *state_out = nullptr)
 {
@@ -833,6 +844,7 @@ int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int
         if (items[i].num_pauli_terms < 0 || (items[i].num_pauli_terms > 0 && !items[i].pauli_terms))
             return MOONLAB_SCHED_BAD_ARG;
     std::vector<std::pair<double, int>> cost((size_t)count);
+    std::vector<double> work((size_t)count);   // estimated microseconds on one workgroup
     int64_t obs_total = 0, out_total = 0;
     int max_big = 0;
 
@@ -874,6 +886,9 @@ int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int
             frame_plan(gates, phase, n, tbmax, 4, it.precision == MOONLAB_HIP_C64 ? 8 : 16, kBatchLookahead, c.passes,
                        c.ops);
             I.num_passes = (int)c.passes.size() - I.first_pass;
+            I.slot_offset = -1;
+            const double tiles = n > I.tile_bits ? (double)(1ull << (n - I.tile_bits)) : 1.0;
+            work[(size_t)i] = tiles * (kTilePassUs * (I.num_passes + 1) + kTileGateUs * (double)gates.size());
             // longest first: sweeps x amplitudes (resident circuits: ops x tile)
             const double sweeps = n > I.tile_bits ? (double)(I.num_passes + 2) * 4.0 : 0.2 * (double)gates.size();
             cost[(size_t)i] = {-(sweeps * (double)(1ull << n)), i};
@@ -933,22 +948,74 @@ int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int
         if (prec == MOONLAB_HIP_C128) n128 = (int)order.size();
     }
 
+    // Circuits larger than a tile whose passes are spread over the whole chip,
+    // one launch per pass for all of them, longest first in each precision:
+    // when the longest circuit on one workgroup would outlast the sum of all
+    // spread evenly, the launches and the reading of its tiles at the end.
+    struct Spread {
+        std::vector<int32_t> list, first;   // circuits; their first tile, and the sum
+        std::vector<int>     count, tiles;  // by level
+    } spread[2];
+    uint64_t own_amps = 0;
+    {
+        double longest = 0.0, all = 0.0, read = 0.0;
+        int levels = 0;
+        uint64_t amps = 0;
+        for (int i = 0; i < count; i++) {
+            const BInst &I = insts[(size_t)i];
+            all += work[(size_t)i];
+            if (I.n <= I.tile_bits || I.num_passes < 1) continue;
+            longest = std::max(longest, work[(size_t)i]);
+            read = std::max(read, kTilePassUs * (double)(1ull << (I.n - I.tile_bits)));
+            levels = std::max(levels, I.num_passes);
+            amps += 1ull << I.n;
+        }
+        const double even = all / (b->num_cus * 2);
+        if (amps <= (1ull << 28) && std::max(longest, even) > 1.25 * (even + read + kLevelUs * levels)) {
+            for (const int prec : {MOONLAB_HIP_C128, MOONLAB_HIP_C64}) {
+                Spread &S = spread[prec == MOONLAB_HIP_C64];
+                for (const int32_t i : order) {
+                    const BInst &I = insts[(size_t)i];
+                    if (I.prec == prec && I.n > I.tile_bits && I.num_passes > 0) S.list.push_back(i);
+                }
+                std::stable_sort(S.list.begin(), S.list.end(), [&](int32_t x, int32_t y) {
+                    return insts[(size_t)x].num_passes > insts[(size_t)y].num_passes;
+                });
+                S.first.push_back(0);
+                for (const int32_t i : S.list) {
+                    BInst &I = insts[(size_t)i];
+                    I.slot_offset = (int64_t)own_amps;
+                    own_amps += 1ull << I.n;
+                    S.first.push_back(S.first.back() + (int32_t)(1ull << (I.n - I.tile_bits)));
+                }
+                for (size_t m = S.list.size(); m > 0;) {   // circuits that reach each level
+                    const int lv = (int)S.count.size();
+                    while (m > 0 && insts[(size_t)S.list[m - 1]].num_passes <= lv) m--;
+                    if (m == 0) break;
+                    S.count.push_back((int)m);
+                    S.tiles.push_back(S.first[m]);
+                }
+            }
+        }
+    }
+
     // grid: as many workgroups as fit, bounded by the HBM slots large circuits need
     int grid = b->num_cus * b->wg_per_cu;
     if (grid > count) grid = count;
-    uint64_t slot_amps = 0, tile_slot = 0;
+    uint64_t slot_amps = 1, tile_slot = 2;
+    for (const BInst &I : insts)
+        if (I.n > I.tile_bits && I.slot_offset < 0) slot_amps = std::max<uint64_t>(slot_amps, 1ull << I.n);
     if (max_big) {
-        slot_amps = 1ull << max_big;
         tile_slot = 2ull << (max_big - (tbmax < max_big ? tbmax : max_big));
         const uint64_t per_wg = slot_amps * 16 + tile_slot * 8;
         const uint64_t budget = 16ull << 30;
         const uint64_t fit = budget / per_wg;
         if ((uint64_t)grid > fit) grid = (int)(fit ? fit : 1);
-    } else {
-        slot_amps = 1;
-        tile_slot = 2;
     }
-    const size_t scratch_bytes = (size_t)grid * (slot_amps * 16 + tile_slot * 8) + 256;
+    // the precisions run side by side: slots of their own
+    const int grid128 = std::min(grid, n128), grid64 = std::min(grid, count - n128);
+    const size_t wgs = (size_t)(grid128 + grid64);
+    const size_t scratch_bytes = wgs * (slot_amps * 16 + tile_slot * 8) + own_amps * 16 + 256;
     if (grow_dev(&b->d_scratch, &b->scratch_cap, scratch_bytes)) return MOONLAB_SCHED_OOM;
 
     auto room = [](size_t need, size_t &have) {
@@ -960,6 +1027,8 @@ int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int
     auto place = [&](size_t bytes) { const size_t o = off; off = (off + bytes + 255) / 256 * 256; return o; };
     const size_t o_inst = place(insts.size() * sizeof(BInst));
     const size_t o_order = place(order.size() * sizeof(int32_t));
+    const size_t o_spread[2] = {place((2 * spread[0].list.size() + 1) * sizeof(int32_t)),
+                                place((2 * spread[1].list.size() + 1) * sizeof(int32_t))};
     const size_t o_pass = place(room(total_passes, b->room_passes) * sizeof(FPass));
     const size_t o_ops = place(room(total_ops + 1, b->room_ops) * sizeof(FOp));
     const size_t o_draw = place((draws.size() + 1) * sizeof(double));
@@ -975,6 +1044,12 @@ int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int
     char *hp = (char *)b->h_prog;
     memcpy(hp + o_inst, insts.data(), insts.size() * sizeof(BInst));
     memcpy(hp + o_order, order.data(), order.size() * sizeof(int32_t));
+    for (int p = 0; p < 2; p++) {
+        const Spread &S = spread[p];
+        if (S.list.empty()) continue;
+        memcpy(hp + o_spread[p], S.list.data(), S.list.size() * sizeof(int32_t));
+        memcpy(hp + o_spread[p] + S.list.size() * sizeof(int32_t), S.first.data(), S.first.size() * sizeof(int32_t));
+    }
     {
         FPass *hpass = (FPass *)(hp + o_pass);
         FOp *hops = (FOp *)(hp + o_ops);
@@ -1001,25 +1076,55 @@ int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int
     char *dp = (char *)b->d_prog;
     char *dr = (char *)b->d_res;
     double2 *scratch = (double2 *)b->d_scratch;
-    double *tile_scratch = (double *)((char *)b->d_scratch + (size_t)grid * slot_amps * 16);
+    double2 *own = scratch + wgs * slot_amps;
+    double *tile_scratch = (double *)(own + own_amps);
 
-    // the device step: upload, queue reset + persistent launch, download
+    // the device step: upload, queue reset, passes of the spread circuits and
+    // the persistent launch by precision, download
     auto step = [&]() -> hipError_t {
+        const bool beside = n128 > 0 && n128 < count;
         hipError_t r = hipMemcpyAsync(dp, hp, prog_bytes, hipMemcpyHostToDevice, b->stream);
-        if (r == hipSuccess)
-            r = launch_batch((const BInst *)(dp + o_inst), (const int32_t *)(dp + o_order), n128, count - n128, b->d_counter,
-                             (const FPass *)(dp + o_pass), (const FOp *)(dp + o_ops), scratch, slot_amps,
-                             tile_scratch, tile_slot, (const double *)(dp + o_draw), (double *)(dr + r_obs),
-                             (uint64_t *)(dr + r_out), (const PauliT *)(dp + o_pauli), d_state, grid, b->stream);
+        if (r == hipSuccess) r = launch_reset_counters(b->d_counter, b->stream);
+        if (r == hipSuccess && beside) r = hipEventRecord(b->fork, b->stream);
+        if (r == hipSuccess && beside) r = hipStreamWaitEvent(b->aux, b->fork, 0);
+        const BInst *d_inst = (const BInst *)(dp + o_inst);
+        const FPass *d_pass = (const FPass *)(dp + o_pass);
+        const FOp *d_ops = (const FOp *)(dp + o_ops);
+        for (int p = 0; p < 2; p++) {
+            const int cnt = p ? count - n128 : n128, prec = p ? MOONLAB_HIP_C64 : MOONLAB_HIP_C128;
+            const Spread &S = spread[p];
+            const hipStream_t st = beside && p ? b->aux : b->stream;
+            const int32_t *d_list = (const int32_t *)(dp + o_spread[p]);
+            for (size_t lv = 0; r == hipSuccess && lv < S.count.size(); lv++)
+                r = launch_batch_pass(prec, d_inst, d_list, d_list + S.list.size(), S.count[lv], (int)lv, S.tiles[lv],
+                                      d_pass, d_ops, own, st);
+            const size_t wg0 = p ? (size_t)grid128 : 0;
+            if (r == hipSuccess && cnt > 0)
+                r = launch_batch(prec, d_inst, (const int32_t *)(dp + o_order) + (p ? n128 : 0), cnt, b->d_counter + p,
+                                 d_pass, d_ops, scratch + wg0 * slot_amps, slot_amps, own,
+                                 tile_scratch + wg0 * tile_slot, tile_slot, (const double *)(dp + o_draw),
+                                 (double *)(dr + r_obs), (uint64_t *)(dr + r_out), (const PauliT *)(dp + o_pauli),
+                                 d_state, p ? grid64 : grid128, st);
+        }
+        if (beside) {   // also after an error: the fork is always joined
+            const hipError_t j = hipEventRecord(b->join, b->aux);
+            const hipError_t w = j == hipSuccess ? hipStreamWaitEvent(b->stream, b->join, 0) : j;
+            if (r == hipSuccess) r = w;
+        }
         if (r == hipSuccess) r = hipMemcpyAsync(b->h_res, dr, res_bytes, hipMemcpyDeviceToHost, b->stream);
         return r;
     };
     // everything the captured nodes bake in: buffers, sizes, offsets, launch shape
-    const std::vector<uint64_t> key = {(uint64_t)(uintptr_t)dp, (uint64_t)(uintptr_t)dr,
+    std::vector<uint64_t> key = {(uint64_t)(uintptr_t)dp, (uint64_t)(uintptr_t)dr,
                                        (uint64_t)(uintptr_t)hp, (uint64_t)(uintptr_t)b->h_res,
                                        (uint64_t)(uintptr_t)b->d_scratch, prog_bytes, res_bytes, o_inst, o_order,
                                        o_pass, o_ops, o_draw, r_obs, r_out, (uint64_t)count, (uint64_t)grid,
-                                       slot_amps, tile_slot, o_pauli, (uint64_t)(uintptr_t)d_state, (uint64_t)n128};
+                                       slot_amps, tile_slot, o_pauli, (uint64_t)(uintptr_t)d_state, (uint64_t)n128,
+                                       own_amps, o_spread[0], o_spread[1]};
+    for (const Spread &S : spread) {
+        key.push_back(S.count.size());
+        for (size_t lv = 0; lv < S.count.size(); lv++) key.push_back((uint64_t)S.count[lv] << 32 | (uint32_t)S.tiles[lv]);
+    }
     // A shape seen for the first time runs eagerly; its second run is captured
     // and launched as a graph; later runs of it replay that graph.
     bool replayed = false;
@@ -1228,7 +1333,9 @@ moonlab_mi355x_batch_t *moonlab_mi355x_batch_create(void)
     if (b->num_cus <= 0) b->num_cus = 256;
     if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess ||
         hipMalloc((void **)&b->d_counter, 256) != hipSuccess || hipEventCreate(&b->e0) != hipSuccess ||
-        hipEventCreate(&b->e1) != hipSuccess) {
+        hipEventCreate(&b->e1) != hipSuccess || hipStreamCreateWithFlags(&b->aux, hipStreamNonBlocking) != hipSuccess ||
+        hipEventCreateWithFlags(&b->fork, hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&b->join, hipEventDisableTiming) != hipSuccess) {
         moonlab_mi355x_batch_free(b);
         return nullptr;
     }
@@ -1262,6 +1369,9 @@ void moonlab_mi355x_batch_free(moonlab_mi355x_batch_t *b)
     if (b->gexec) hipGraphExecDestroy(b->gexec);
     if (b->e0) hipEventDestroy(b->e0);
     if (b->e1) hipEventDestroy(b->e1);
+    if (b->fork) hipEventDestroy(b->fork);
+    if (b->join) hipEventDestroy(b->join);
+    if (b->aux) hipStreamDestroy(b->aux);
     if (b->stream) hipStreamDestroy(b->stream);
     delete b;
 }

@@ -521,9 +521,58 @@ __device__ __forceinline__ int cdf_find(const double *cdf, int T, double u)
     return lo;
 }
 
+// A tile of |0..0> other than the first is zero, and so it leaves a pass,
+// unless a parameter was not finite (the scale holds every cosine).
+__device__ __forceinline__ bool zero_stays_zero(FConst<FPass> P)
+{
+    return P->scale_r - P->scale_r == 0.0 && P->scale_i - P->scale_i == 0.0;
+}
+
+// Pass `level` of the circuits list[0..): one workgroup per tile, those of
+// circuit i from first_tile[i] on.  Few circuits past a tile's size, one
+// workgroup each, leave most of the chip idle: 39 circuits of 10 to 16 qubits
+// took 3.1 ms, the time of the longest one's 14 passes over 16 tiles.
+template <typename R>
+__global__ __launch_bounds__(NT, 2) void k_batch_pass(const BInst *__restrict__ insts, const int32_t *__restrict__ list,
+                                                      const int32_t *__restrict__ first_tile, int count, int level,
+                                                      const FPass *__restrict__ passes, const FOp *__restrict__ prog,
+                                                      double2 *__restrict__ own)
+{
+    using V = typename FVec<R>::t;
+    __shared__ double2 tile[1 << kBatchMaxTileBits];
+    const FConst<int32_t> ft0 = (FConst<int32_t>)(uintptr_t)first_tile;
+    int lo = 0, hi = count;   // the last circuit that starts at or before this tile
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (ft0[mid] <= (int)blockIdx.x) lo = mid;
+        else hi = mid;
+    }
+    const FConst<BInst> I = (FConst<BInst>)(uintptr_t)(insts + ((FConst<int32_t>)(uintptr_t)list)[lo]);
+    const FConst<FPass> P = (FConst<FPass>)(uintptr_t)(passes + I->first_pass + level);
+    const int tid = threadIdx.x, nb = I->tile_bits, threads = 1 << (nb - kFrameRegBits);
+    const bool active = tid < threads;
+    const uint64_t mask = P->mask;
+    const uint64_t base = frame_uniform(frame_deposit((uint64_t)((int)blockIdx.x - ft0[lo]), ~mask));
+    cplx_t<R> *slot = (cplx_t<R> *)(own + I->slot_offset);
+    constexpr uint32_t B = (uint32_t)sizeof(cplx_t<R>);
+    const BatchTile bt = batch_tile<R>(mask, nb, tid);
+    V v[16];
+    if (level > 0) {
+        batch_load<R>(slot, bt, (uint32_t)base * B, v);
+    } else {
+#pragma unroll
+        for (int j = 0; j < 16; j++) v[j] = V{R(j == 0 && tid == 0 && base == 0), R(0)};
+    }
+    if (level > 0 || base == 0 || !zero_stays_zero(P)) {
+        const FrameThread ft = frame_thread(P, prog, tid, nb - kFrameRegBits, active);
+        frame_tile<R>(MLX_FRAME_LDS(tile), v, P, prog, ft, base, tid, nb);
+    }
+    if (active) batch_store<R>(slot, bt, (uint32_t)base * B, v);
+}
+
 template <typename R>
 __device__ __forceinline__ void run_circuit(Shared &sh, uint32_t lds, const BInst &I, const FPass *passes, const FOp *prog, double2 *slot_raw,
-                            double *tile_sums, const double *draws, double *obs, uint64_t *outcomes,
+                            double2 *own, double *tile_sums, const double *draws, double *obs, uint64_t *outcomes,
                             const PauliT *terms, void *state_out)
 {
     using V = typename FVec<R>::t;
@@ -534,10 +583,12 @@ __device__ __forceinline__ void run_circuit(Shared &sh, uint32_t lds, const BIns
     const int threads = 1 << (nb - kFrameRegBits);    // that hold amplitudes
     const bool active = tid < threads;
     cplx_t<R> *t = (cplx_t<R> *)sh.tile;
-    cplx_t<R> *slot = (cplx_t<R> *)slot_raw;
+    // gate passes already run by k_batch_pass on the circuit's own slot
+    const bool ready = I.slot_offset >= 0;
+    cplx_t<R> *slot = (cplx_t<R> *)(ready ? own + I.slot_offset : slot_raw);
 
     // ---- gate passes ----
-    for (int pi = 0; pi < I.num_passes; pi++) {
+    for (int pi = ready ? I.num_passes : 0; pi < I.num_passes; pi++) {
         const FConst<FPass> P = (FConst<FPass>)(uintptr_t)(passes + I.first_pass + pi);
         const uint64_t mask = P->mask;
         const FrameThread ft = frame_thread(P, prog, tid, nb - kFrameRegBits, active);
@@ -562,7 +613,7 @@ __device__ __forceinline__ void run_circuit(Shared &sh, uint32_t lds, const BIns
 #pragma unroll
                 for (int j = 0; j < 16; j++) v[j] = V{R(j == 0 && tid == 0 && base == 0), R(0)};
             }
-            frame_tile<R>(lds, v, P, prog, ft, base, tid, nb);
+            if (load || base == 0 || !zero_stays_zero(P)) frame_tile<R>(lds, v, P, prog, ft, base, tid, nb);
             if (store) batch_store<R>(slot, bt, (uint32_t)base * B, v);
             if (resident) {
                 __syncthreads();   // a layout change may still be read
@@ -831,7 +882,16 @@ __device__ __forceinline__ void run_circuit(Shared &sh, uint32_t lds, const BIns
     for (uint64_t ti = 0; ti < ntiles; ti++) {
         int mine = 0;
         for (int s = tid; s < I.num_shots; s += NT) mine |= oc[s] == (kMark | ti);
-        if (!__syncthreads_or(mine)) continue;
+        // any thread's (a flag of the kernel's own: the library's reduction
+        // over the workgroup keeps its LDS address in a register across the
+        // whole measurement, which this kernel has none left for)
+        if (tid == 0) sh.next = 0;
+        __syncthreads();
+        if (mine) sh.next = 1;
+        __syncthreads();
+        const int any = sh.next;
+        __syncthreads();
+        if (!any) continue;
         for (int l = tid; l < T; l += NT) cdf[cdf_at(l)] = p2<R>(slot[(ti << nb) | (uint64_t)l]);
         __syncthreads();
         lds_scan(sh, cdf, T, ti ? incl[ti - 1] : 0.0);
@@ -868,7 +928,7 @@ __global__ __launch_bounds__(NT, 2) void k_batch(const BInst *__restrict__ insts
                                                  int ninst, int *__restrict__ counter,
                                                  const FPass *__restrict__ passes, const FOp *__restrict__ prog,
                                                  double2 *__restrict__ scratch, uint64_t slot_amps,
-                                                 double *__restrict__ tile_scratch, uint64_t tile_slot,
+                                                 double2 *__restrict__ own, double *__restrict__ tile_scratch, uint64_t tile_slot,
                                                  const double *__restrict__ draws, double *__restrict__ obs,
                                                  uint64_t *__restrict__ outcomes, const PauliT *__restrict__ terms,
                                                  void *__restrict__ state_out)
@@ -888,7 +948,7 @@ __global__ __launch_bounds__(NT, 2) void k_batch(const BInst *__restrict__ insts
         const FConst<uint32_t> src = (FConst<uint32_t>)(uintptr_t)(insts + *(FConst<int32_t>)(uintptr_t)(order + k));
 #pragma unroll
         for (int w = 0; w < (int)(sizeof I / sizeof(uint32_t)); w++) ((uint32_t *)&I)[w] = src[w];
-        run_circuit<R>(sh, MLX_FRAME_LDS(sh.tile), I, passes, prog, slot, ts, draws, obs, outcomes, terms, state_out);
+        run_circuit<R>(sh, MLX_FRAME_LDS(sh.tile), I, passes, prog, slot, own, ts, draws, obs, outcomes, terms, state_out);
         __syncthreads();
     }
 }
@@ -1002,23 +1062,35 @@ hipError_t launch_tile_pass(void *amps, int prec, int n, const BPass &P, const B
               : tile_pass_shape<double, false>(amps, P, d_ops, ntiles, cus, threads, tile_bits, st);
 }
 
-// order: the n128 complex128 circuits, then the n64 complex64 ones; counter:
-// two queue heads; grid: workgroups at most (the two launches follow each
-// other and share the slots).
-hipError_t launch_batch(const BInst *insts, const int32_t *order, int n128, int n64, int *counter, const FPass *passes,
-                        const FOp *prog, double2 *scratch, uint64_t slot_amps, double *tile_scratch,
+hipError_t launch_batch_pass(int prec, const BInst *insts, const int32_t *list, const int32_t *first_tile, int count,
+                             int level, int tiles, const FPass *passes, const FOp *prog, double2 *own, hipStream_t st)
+{
+    auto go = [&](auto kernel) {
+        kernel<<<tiles, NT, 0, st>>>(insts, list, first_tile, count, level, passes, prog, own);
+    };
+    go(prec == MOONLAB_HIP_C64 ? k_batch_pass<float> : k_batch_pass<double>);
+    return hipGetLastError();
+}
+
+hipError_t launch_reset_counters(int *counters, hipStream_t st)
+{
+    k_reset_counter<<<1, 2, 0, st>>>(counters);
+    return hipGetLastError();
+}
+
+// order: `count` circuits of one precision; counter: their queue head; grid:
+// workgroups at most, with a slot and tile sums each.
+hipError_t launch_batch(int prec, const BInst *insts, const int32_t *order, int count, int *counter, const FPass *passes,
+                        const FOp *prog, double2 *scratch, uint64_t slot_amps, double2 *own, double *tile_scratch,
                         uint64_t tile_slot, const double *draws, double *obs, uint64_t *outcomes,
                         const PauliT *terms, void *state_out, int grid, hipStream_t st)
 {
-    k_reset_counter<<<1, 2, 0, st>>>(counter);
-    if (n128 > 0)
-        k_batch<double><<<n128 < grid ? n128 : grid, NT, 0, st>>>(insts, order, n128, counter, passes, prog, scratch,
-                                                                  slot_amps, tile_scratch, tile_slot, draws, obs,
-                                                                  outcomes, terms, state_out);
-    if (n64 > 0)
-        k_batch<float><<<n64 < grid ? n64 : grid, NT, 0, st>>>(insts, order + n128, n64, counter + 1, passes, prog,
-                                                               scratch, slot_amps, tile_scratch, tile_slot, draws, obs,
-                                                               outcomes, terms, state_out);
+    auto go = [&](auto kernel) {
+        kernel<<<count < grid ? count : grid, NT, 0, st>>>(insts, order, count, counter, passes, prog, scratch, slot_amps,
+                                                           own, tile_scratch, tile_slot, draws, obs, outcomes, terms,
+                                                           state_out);
+    };
+    go(prec == MOONLAB_HIP_C64 ? k_batch<float> : k_batch<double>);
     return hipGetLastError();
 }
 

@@ -157,6 +157,7 @@ struct BInst {
     int64_t  state_offset;  // amplitude offset of the final state in the state output buffer, -1: none
     int32_t  num_pauli;     // Pauli terms to measure
     int32_t  pad_;
+    int64_t  slot_offset;   // 16-byte units into the circuits' own slots, its gate passes already run there; -1: none
 };
 
 // One Pauli string P = i^ny X^x Z^z (Y_q = i X_q Z_q): P|i> = i^ny
