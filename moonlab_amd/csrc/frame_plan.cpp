@@ -522,12 +522,11 @@ class PassBuilder {
                 for (uint64_t m = g->z; m; m &= m - 1) times(zrow(__builtin_ctzll(m)));
                 p.s = ((k - __builtin_popcount(p.x & p.z)) >> 1) & 1;
                 rots_.push_back(LRot{p, g->t});
-                if (bytes_ == 8) {   // the norm the rounded tangent leaves, not the exact cosine
-                    const double tf = (double)(float)g->t;
-                    scale *= copysign(1.0 / sqrt(1.0 + tf * tf), g->scale);
-                } else {
-                    scale *= g->scale;
-                }
+                // the norm that the rounded tangent leaves, not the cosine
+                const long double t = bytes_ == 8 ? (long double)(float)g->t : (long double)g->t;
+                grow_ *= 1.0L + t * t;
+                if (grow_ > 0x1p1000L) settle();
+                if (g->scale < 0.0) scale = -scale;
                 break;
             }
             case FG_CX: {
@@ -556,6 +555,14 @@ class PassBuilder {
             }
             }
         }
+    }
+
+    // squared growth of the norm into the scale
+    void settle()
+    {
+        const long double f = 1.0L / sqrtl(grow_);
+        scale = cd((double)(f * scale.real()), (double)(f * scale.imag()));
+        grow_ = 1.0L;
     }
 
     // x and z of an image in one word; two commute when parity(a & swap(b)) is 0
@@ -781,6 +788,7 @@ class PassBuilder {
         P.ncross = (int32_t)cross.size();
         for (const FCross &c : cross) push(c);
         // the scale, when this pass is the last or it has run far from 1
+        settle();
         const double mag = log2(abs(scale));
         if (scale != cd(1.0) && (last || fabs(mag) > 20.0)) {
             // the phase waits for the last pass
@@ -855,6 +863,7 @@ class PassBuilder {
     std::vector<FPass>    &passes_;
     std::vector<FOp>      &prog_;
     std::vector<uint32_t>  pack_;
+    long double            grow_ = 1.0L;
     std::vector<Row>       X_, Z_;
     std::vector<LRot>      rots_;
     std::vector<Quad>      quads_;
@@ -868,7 +877,7 @@ void frame_plan(const std::vector<FGate> &gates, cd phase, int n, int tb, int an
                 int lookahead, std::vector<FPass> &passes, std::vector<FOp> &prog)
 {
     PassBuilder B(amp_bytes, lookahead, passes, prog);
-    B.scale = phase;
+    B.scale = phase / abs(phase);   // every gate is unitary: its factors' roundings go
     std::vector<const FGate *> rest, cur, later;
     rest.reserve(gates.size());
     for (const FGate &g : gates) rest.push_back(&g);
