@@ -755,6 +755,7 @@ struct moonlab_mi355x_batch {
     size_t      scratch_cap = 0;
     hipEvent_t  e0 = nullptr, e1 = nullptr;
     // the complex64 circuits of a mixed batch run beside the complex128 ones
+    // (made when there is a mixed batch)
     hipStream_t aux = nullptr;
     hipEvent_t  fork = nullptr, join = nullptr;
     // HIP graph of the last batch shape (see moonlab_mi355x_batch_set_graphs)
@@ -1081,8 +1082,13 @@ int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int
 
     // the device step: upload, queue reset, passes of the spread circuits and
     // the persistent launch by precision, download
+    const bool beside = n128 > 0 && n128 < count;
+    if (beside && !b->aux &&
+        (hipEventCreateWithFlags(&b->fork, hipEventDisableTiming) != hipSuccess ||
+         hipEventCreateWithFlags(&b->join, hipEventDisableTiming) != hipSuccess ||
+         hipStreamCreateWithFlags(&b->aux, hipStreamNonBlocking) != hipSuccess))
+        return MOONLAB_SCHED_INTERNAL;
     auto step = [&]() -> hipError_t {
-        const bool beside = n128 > 0 && n128 < count;
         hipError_t r = hipMemcpyAsync(dp, hp, prog_bytes, hipMemcpyHostToDevice, b->stream);
         if (r == hipSuccess) r = launch_reset_counters(b->d_counter, b->stream);
         if (r == hipSuccess && beside) r = hipEventRecord(b->fork, b->stream);
@@ -1333,9 +1339,7 @@ moonlab_mi355x_batch_t *moonlab_mi355x_batch_create(void)
     if (b->num_cus <= 0) b->num_cus = 256;
     if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess ||
         hipMalloc((void **)&b->d_counter, 256) != hipSuccess || hipEventCreate(&b->e0) != hipSuccess ||
-        hipEventCreate(&b->e1) != hipSuccess || hipStreamCreateWithFlags(&b->aux, hipStreamNonBlocking) != hipSuccess ||
-        hipEventCreateWithFlags(&b->fork, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&b->join, hipEventDisableTiming) != hipSuccess) {
+        hipEventCreate(&b->e1) != hipSuccess) {
         moonlab_mi355x_batch_free(b);
         return nullptr;
     }
