@@ -53,6 +53,8 @@ hipError_t launch_batch(int prec, const BInst *insts, const int32_t *order, int 
                         const PauliT *terms, void *state_out, int grid, hipStream_t st);
 hipError_t launch_batch_pass(int prec, const BInst *insts, const int32_t *list, const int32_t *first_tile, int count,
                              int level, int tiles, const FPass *passes, const FOp *prog, double2 *own, hipStream_t st);
+hipError_t launch_batch_pauli(int prec, const BInst *insts, const int32_t *list, const int32_t *first, int count,
+                              int groups, const PauliT *terms, const double2 *own, double *obs, hipStream_t st);
 hipError_t launch_reset_counters(int *counters, hipStream_t st);
 
 // A Pauli string over n qubits (s[q] in "IXYZ" acts on qubit q, strlen == n,
@@ -830,6 +832,7 @@ int host_threads(size_t gates, int parts)
 // layouts and stores, each rotation or frame gate of the circuit, and a
 // launch of one pass of many circuits, in microseconds as measured.
 constexpr double kTilePassUs = 6.0, kTileGateUs = 0.25, kLevelUs = 20.0;
+constexpr double kPauliUs = 3.4;   // a Pauli string on a tile in k_batch
 
 int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int count,
               moonlab_mi355x_batch_stats_t *stats, const BatchStateOut *state_out = nullptr)
@@ -888,6 +891,7 @@ int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int
                        c.ops);
             I.num_passes = (int)c.passes.size() - I.first_pass;
             I.slot_offset = -1;
+            I.pauli_slot = -1;
             const double tiles = n > I.tile_bits ? (double)(1ull << (n - I.tile_bits)) : 1.0;
             work[(size_t)i] = tiles * (kTilePassUs * (I.num_passes + 1) + kTileGateUs * (double)gates.size());
             // longest first: sweeps x amplitudes (resident circuits: ops x tile)
@@ -1000,6 +1004,37 @@ int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int
         }
     }
 
+    // Pauli strings by workgroups of their own where the circuit with most to
+    // measure would keep its workgroup longer than storing the states and one
+    // more launch take (states up to 4 GiB).
+    struct Strings {
+        std::vector<int32_t> list, first;   // circuits; their first workgroup, and the sum
+    } strings[2];
+    {
+        double most = 0.0;
+        uint64_t amps = own_amps;
+        for (const BInst &I : insts) {
+            if (I.num_pauli == 0) continue;
+            most = std::max(most, kPauliUs * I.num_pauli * ldexp(1.0, I.n - kBatchMaxTileBits));
+            if (I.slot_offset < 0) amps += 1ull << I.n;
+        }
+        if (most > 30.0 && amps <= (1ull << 28)) {
+            for (const int32_t i : order) {
+                BInst &I = insts[(size_t)i];
+                if (I.num_pauli == 0) continue;
+                I.pauli_slot = I.slot_offset;
+                if (I.pauli_slot < 0) {
+                    I.pauli_slot = (int64_t)own_amps;
+                    own_amps += 1ull << I.n;
+                }
+                Strings &S = strings[I.prec == MOONLAB_HIP_C64];
+                if (S.list.empty()) S.first.push_back(0);
+                S.list.push_back(i);
+                S.first.push_back(S.first.back() + (I.num_pauli + kPauliChunk - 1) / kPauliChunk);
+            }
+        }
+    }
+
     // grid: as many workgroups as fit, bounded by the HBM slots large circuits need
     int grid = b->num_cus * b->wg_per_cu;
     if (grid > count) grid = count;
@@ -1030,6 +1065,8 @@ int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int
     const size_t o_order = place(order.size() * sizeof(int32_t));
     const size_t o_spread[2] = {place((2 * spread[0].list.size() + 1) * sizeof(int32_t)),
                                 place((2 * spread[1].list.size() + 1) * sizeof(int32_t))};
+    const size_t o_strings[2] = {place((2 * strings[0].list.size() + 1) * sizeof(int32_t)),
+                                 place((2 * strings[1].list.size() + 1) * sizeof(int32_t))};
     const size_t o_pass = place(room(total_passes, b->room_passes) * sizeof(FPass));
     const size_t o_ops = place(room(total_ops + 1, b->room_ops) * sizeof(FOp));
     const size_t o_draw = place((draws.size() + 1) * sizeof(double));
@@ -1045,11 +1082,14 @@ int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int
     char *hp = (char *)b->h_prog;
     memcpy(hp + o_inst, insts.data(), insts.size() * sizeof(BInst));
     memcpy(hp + o_order, order.data(), order.size() * sizeof(int32_t));
+    auto place_list = [&](size_t at, const std::vector<int32_t> &list, const std::vector<int32_t> &first) {
+        if (list.empty()) return;
+        memcpy(hp + at, list.data(), list.size() * sizeof(int32_t));
+        memcpy(hp + at + list.size() * sizeof(int32_t), first.data(), first.size() * sizeof(int32_t));
+    };
     for (int p = 0; p < 2; p++) {
-        const Spread &S = spread[p];
-        if (S.list.empty()) continue;
-        memcpy(hp + o_spread[p], S.list.data(), S.list.size() * sizeof(int32_t));
-        memcpy(hp + o_spread[p] + S.list.size() * sizeof(int32_t), S.first.data(), S.first.size() * sizeof(int32_t));
+        place_list(o_spread[p], spread[p].list, spread[p].first);
+        place_list(o_strings[p], strings[p].list, strings[p].first);
     }
     {
         FPass *hpass = (FPass *)(hp + o_pass);
@@ -1111,6 +1151,11 @@ int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int
                                  tile_scratch + wg0 * tile_slot, tile_slot, (const double *)(dp + o_draw),
                                  (double *)(dr + r_obs), (uint64_t *)(dr + r_out), (const PauliT *)(dp + o_pauli),
                                  d_state, p ? grid64 : grid128, st);
+            const Strings &Q = strings[p];
+            const int32_t *d_str = (const int32_t *)(dp + o_strings[p]);
+            if (r == hipSuccess && !Q.list.empty())
+                r = launch_batch_pauli(prec, d_inst, d_str, d_str + Q.list.size(), (int)Q.list.size(), Q.first.back(),
+                                       (const PauliT *)(dp + o_pauli), own, (double *)(dr + r_obs), st);
         }
         if (beside) {   // also after an error: the fork is always joined
             const hipError_t j = hipEventRecord(b->join, b->aux);
@@ -1126,7 +1171,8 @@ int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int
                                        (uint64_t)(uintptr_t)b->d_scratch, prog_bytes, res_bytes, o_inst, o_order,
                                        o_pass, o_ops, o_draw, r_obs, r_out, (uint64_t)count, (uint64_t)grid,
                                        slot_amps, tile_slot, o_pauli, (uint64_t)(uintptr_t)d_state, (uint64_t)n128,
-                                       own_amps, o_spread[0], o_spread[1]};
+                                       own_amps, o_spread[0], o_spread[1], o_strings[0], o_strings[1]};
+    for (const Strings &Q : strings) key.push_back(Q.list.empty() ? 0 : (uint64_t)Q.list.size() << 32 | (uint32_t)Q.first.back());
     for (const Spread &S : spread) {
         key.push_back(S.count.size());
         for (size_t lv = 0; lv < S.count.size(); lv++) key.push_back((uint64_t)S.count[lv] << 32 | (uint32_t)S.tiles[lv]);

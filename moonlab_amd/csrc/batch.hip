@@ -62,7 +62,8 @@ struct Shared {
 
 // Block reduction of v[0..nv): wave butterflies, then waves summed in order.
 // Result j lands in out[j] (for j < nv) on every thread after the call.
-__device__ __forceinline__ void block_reduce(Shared &sh, double *v, int nv, double *out)
+template <typename S>
+__device__ __forceinline__ void block_reduce(S &sh, double *v, int nv, double *out)
 {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (int j = 0; j < nv; j++) {
@@ -570,6 +571,75 @@ __global__ __launch_bounds__(NT, 2) void k_batch_pass(const BInst *__restrict__ 
     if (active) batch_store<R>(slot, bt, (uint32_t)base * B, v);
 }
 
+// Pauli strings of the circuits list[0..), eight to a workgroup: those of
+// circuit i from workgroup first[i] on, its final state in its own slot.  The
+// sums run in measure_pauli_tile's order, so both give the same bits.  Bound
+// by the partners' loads from L2 (512 KiB per tile of 12 qubits).  The
+// persistent kernel measures a circuit's strings one workgroup per circuit, at
+// 3.4 us per string and tile, most of it address and parity arithmetic: 100
+// strings of four 15-qubit circuits took 2.5 ms, here 0.27 ms.
+template <typename R>
+__global__ __launch_bounds__(NT) void k_batch_pauli(const BInst *__restrict__ insts, const int32_t *__restrict__ list,
+                                                    const int32_t *__restrict__ first, int count,
+                                                    const PauliT *__restrict__ terms, const double2 *__restrict__ own,
+                                                    double *__restrict__ obs)
+{
+    using V = typename FVec<R>::t;
+    constexpr int PER = (1 << kBatchMaxTileBits) / NT;
+    __shared__ struct {
+        double red[NW][kPauliChunk], res[kPauliChunk];
+    } sh;
+    const FConst<int32_t> f0 = (FConst<int32_t>)(uintptr_t)first;
+    int lo = 0, hi = count;   // the last circuit that starts at or before this workgroup
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (f0[mid] <= (int)blockIdx.x) lo = mid;
+        else hi = mid;
+    }
+    const FConst<BInst> I = (FConst<BInst>)(uintptr_t)(insts + ((FConst<int32_t>)(uintptr_t)list)[lo]);
+    const int tid = threadIdx.x, n = I->n, nb = I->tile_bits;
+    const int c0 = kPauliChunk * ((int)blockIdx.x - f0[lo]);
+    const int cnt = I->num_pauli - c0 < kPauliChunk ? I->num_pauli - c0 : kPauliChunk;
+    const FConst<PauliT> term = (FConst<PauliT>)(uintptr_t)(terms + I->pauli_offset + c0);
+    const cplx_t<R> *slot = (const cplx_t<R> *)(own + I->pauli_slot);
+    const int T = n <= nb ? 1 << n : 1 << nb;
+    double acc = 0.0;
+    for (uint64_t base = 0; base < 1ull << n; base += (uint64_t)T) {
+        V a[PER];
+#pragma unroll
+        for (int e = 0; e < PER; e++) {
+            const int l = tid + NT * e;
+            a[e] = l < T ? frame_ld<R, false>(&slot[base + (uint64_t)l]) : V{R(0), R(0)};
+        }
+        double v[kPauliChunk];
+#pragma unroll
+        for (int j = 0; j < kPauliChunk; j++) {
+            v[j] = 0.0;
+            if (j >= cnt) continue;   // uniform across the block
+            const uint64_t x = term[j].x, z = term[j].z;
+            const int ny = term[j].ny & 3;
+            const int own_par = (__popcll(z & base) ^ __popcll(z & (uint64_t)tid)) & 1;
+            double s = 0.0;
+#pragma unroll
+            for (int e = 0; e < PER; e++) {
+                const int l = tid + NT * e;
+                if (l >= T) continue;
+                const V b = frame_ld<R, false>(&slot[(base + (uint64_t)l) ^ x]);
+                const double br = (double)b.x, bi = (double)b.y, ar = (double)a[e].x, ai = (double)a[e].y;
+                const double re = fmar(br, ar, bi * ai);     // Re conj(b) a
+                const double im = fmar(br, ai, -(bi * ar));  // Im conj(b) a
+                const double c = ny == 0 ? re : ny == 1 ? -im : ny == 2 ? -re : im;
+                s += (own_par ^ (__popcll(z & (uint64_t)(NT * e)) & 1)) ? -c : c;
+            }
+            v[j] = s;
+        }
+        block_reduce(sh, v, cnt, sh.res);
+        if (tid < cnt) acc += sh.res[tid];
+        __syncthreads();
+    }
+    if (tid < cnt) obs[I->obs_offset + obs_size(n) + c0 + tid] = acc;
+}
+
 template <typename R>
 __device__ __forceinline__ void run_circuit(Shared &sh, uint32_t lds, const BInst &I, const FPass *passes, const FOp *prog, double2 *slot_raw,
                             double2 *own, double *tile_sums, const double *draws, double *obs, uint64_t *outcomes,
@@ -636,9 +706,11 @@ __device__ __forceinline__ void run_circuit(Shared &sh, uint32_t lds, const BIns
         __syncthreads();
     }
 
-    // ---- the final state, when asked for (geometric-tensor overlaps) ----
-    if (I.state_offset >= 0) {
-        cplx_t<R> *so = (cplx_t<R> *)state_out + I.state_offset;
+    // ---- the final state, when asked for (geometric-tensor overlaps) or
+    // measured by k_batch_pauli and not in the circuit's own slot yet ----
+    for (int k = 0; k < 2; k++) {
+        if (k ? I.pauli_slot < 0 || ready : I.state_offset < 0) continue;
+        cplx_t<R> *so = k ? (cplx_t<R> *)(own + I.pauli_slot) : (cplx_t<R> *)state_out + I.state_offset;
         const uint64_t dim = 1ull << n;
         if (resident) {
             for (uint64_t i = tid; i < dim; i += NT) so[i] = t[lds_slot<(int)sizeof(V)>((int)i)];
@@ -653,11 +725,12 @@ __device__ __forceinline__ void run_circuit(Shared &sh, uint32_t lds, const BIns
     const int nhigh = resident ? 0 : n - nb, tb = nb - kFrameRegBits;
     const int nzz = n > 1 ? n - 1 : 0;
     double *pauli_out = obs + I.obs_offset + obs_size(n);
-    for (int k = tid; k < I.num_pauli; k += NT) pauli_out[k] = 0.0;
+    const int npauli = I.pauli_slot >= 0 ? 0 : I.num_pauli;
+    for (int k = tid; k < npauli; k += NT) pauli_out[k] = 0.0;
     ObsAcc acc;
     double hi = 0.0, hzz = 0.0;   // thread i: P(1) of qubit nb + i; thread 64 + i: <ZZ> of (nb - 1 + i, nb + i)
     double xs[3][4] = {};         // <X> of the register bits, of tile bits 0..3 and of the four below the register bits
-    const bool lds_tile = want_x || I.num_pauli > 0;
+    const bool lds_tile = want_x || npauli > 0;
     __syncthreads();
     for (uint64_t ti = 0; ti < ntiles; ti++) {
         V v[16];
@@ -714,9 +787,9 @@ __device__ __forceinline__ void run_circuit(Shared &sh, uint32_t lds, const BIns
                     }
                 }
             }
-            if (I.num_pauli > 0)
+            if (npauli > 0)
                 measure_pauli_tile<R>(sh, lds, resident ? 1 << n : 1 << nb, ti << nb, slot, terms + I.pauli_offset,
-                                      I.num_pauli, pauli_out);
+                                      npauli, pauli_out);
             __syncthreads();   // before the next tile is written
         }
     }
@@ -1069,6 +1142,14 @@ hipError_t launch_batch_pass(int prec, const BInst *insts, const int32_t *list, 
         kernel<<<tiles, NT, 0, st>>>(insts, list, first_tile, count, level, passes, prog, own);
     };
     go(prec == MOONLAB_HIP_C64 ? k_batch_pass<float> : k_batch_pass<double>);
+    return hipGetLastError();
+}
+
+hipError_t launch_batch_pauli(int prec, const BInst *insts, const int32_t *list, const int32_t *first, int count,
+                              int groups, const PauliT *terms, const double2 *own, double *obs, hipStream_t st)
+{
+    auto go = [&](auto kernel) { kernel<<<groups, NT, 0, st>>>(insts, list, first, count, terms, own, obs); };
+    go(prec == MOONLAB_HIP_C64 ? k_batch_pauli<float> : k_batch_pauli<double>);
     return hipGetLastError();
 }
 

@@ -158,6 +158,7 @@ struct BInst {
     int32_t  num_pauli;     // Pauli terms to measure
     int32_t  pad_;
     int64_t  slot_offset;   // 16-byte units into the circuits' own slots, its gate passes already run there; -1: none
+    int64_t  pauli_slot;    // likewise, where k_batch_pauli finds its final state; -1: k_batch measures its strings
 };
 
 // One Pauli string P = i^ny X^x Z^z (Y_q = i X_q Z_q): P|i> = i^ny
@@ -179,6 +180,7 @@ enum : int32_t {
 // Observable block per instance, FP64: [norm, P1[n], ZZ[n-1], X[n]].
 __host__ __device__ inline int64_t obs_size(int n) { return 1 + n + (n > 1 ? n - 1 : 0) + n; }
 
+constexpr int kPauliChunk = 8;   // Pauli strings of one workgroup of k_batch_pauli
 constexpr int kBatchMaxTileBits = 12;
 constexpr int kBatchThreads = 256;
 constexpr int kBatchMaxQubits = 24;
