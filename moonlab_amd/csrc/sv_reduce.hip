@@ -194,13 +194,109 @@ __device__ __forceinline__ uint64_t tile_of(const double *__restrict__ incl, uin
     return lo;
 }
 
+// The 256 threads' probabilities of a tile, thread t's from index ept t on in
+// p, and the cumulative sum before them (base: the tiles before).  The tile is
+// loaded with lanes on neighbouring amplitudes and passes through LDS (ps, one
+// pad per 16).
+template <typename R>
+__device__ __forceinline__ double tile_cdf(double *ps, double *wtot, const cplx_t<R> *__restrict__ ta, int tsize,
+                                           int ept, double base, double (&p)[kEpt])
+{
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+#pragma unroll
+    for (int e = 0; e < kEpt; e++) {
+        const int i = e * kRedThreads + tid;
+        if (i < tsize) ps[i + (i >> 4)] = prob<R>(ta[i]);
+    }
+    __syncthreads();
+    double s = 0.0;
+#pragma unroll
+    for (int e = 0; e < kEpt; e++) {
+        const int i = tid * ept + e;
+        p[e] = e < ept && i < tsize ? ps[i + (i >> 4)] : 0.0;
+        s += p[e];
+    }
+    double x = s;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const double y = __shfl_up(x, off, 64);
+        if (lane >= off) x += y;
+    }
+    if (lane == 63) wtot[wave] = x;
+    __syncthreads();
+    double c = base;
+    for (int w = 0; w < wave; w++) c += wtot[w];
+    return c + (x - s);
+}
+
+// Cumulative probabilities of every index, one workgroup per tile, and the
+// shots by one thread each: two searches of dependent loads.  For eight shots
+// per tile or more: 4096 shots at 14 qubits read each tile a thousand times
+// in k_sample, 51 us; here 14 us for both.  The sums are k_sample's.
+template <typename R>
+__global__ __launch_bounds__(kRedThreads) void k_cdf(const cplx_t<R> *__restrict__ a, int tile_bits,
+                                                     const double *__restrict__ tile_incl, double *__restrict__ cdf)
+{
+    __shared__ double ps[(1 << kTileBits) + (1 << kTileBits) / 16];
+    __shared__ double wtot[4];
+    const int tid = threadIdx.x, tsize = 1 << tile_bits, ept = tsize >= kRedThreads ? tsize / kRedThreads : 1;
+    const uint64_t t = blockIdx.x;
+    double p[kEpt];
+    double c = tile_cdf<R>(ps, wtot, a + (t << tile_bits), tsize, ept, t ? tile_incl[t - 1] : 0.0, p);
+#pragma unroll
+    for (int e = 0; e < kEpt; e++) {   // a thread's own entries: read by itself alone
+        const int i = tid * ept + e;
+        c += p[e];
+        if (e < ept && i < tsize) ps[i + (i >> 4)] = c;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < kEpt; e++) {
+        const int i = e * kRedThreads + tid;
+        if (i < tsize) cdf[(t << tile_bits) + (uint64_t)i] = ps[i + (i >> 4)];
+    }
+}
+
+template <typename R>
+__global__ __launch_bounds__(64) void k_find(const cplx_t<R> *__restrict__ a, int tile_bits, uint64_t ntiles,
+                                             const double *__restrict__ tile_incl,
+                                             const double *__restrict__ tile_sums, const double *__restrict__ cdf,
+                                             const double *__restrict__ us, int nshots, uint64_t *__restrict__ out)
+{
+    const int shot = blockIdx.x * 64 + threadIdx.x;
+    if (shot >= nshots) return;
+    const double u = us[shot];
+    // first index of v[0..n) above u
+    auto above = [&](const double *v, uint64_t n) {
+        uint64_t lo = 0, hi = n;
+        while (lo < hi) {
+            const uint64_t mid = (lo + hi) >> 1;
+            if (u < v[mid]) hi = mid;
+            else lo = mid + 1;
+        }
+        return lo;
+    };
+    const uint64_t T = 1ull << tile_bits;
+    for (uint64_t t = above(tile_incl, ntiles); t < ntiles; t++) {
+        const uint64_t l = above(cdf + t * T, T);
+        if (l < T) {
+            out[shot] = t * T + l;
+            return;
+        }
+    }
+    // u >= total mass: the last index with nonzero probability, else 0
+    uint64_t t = ntiles, l = 0;
+    while (t > 0 && !(tile_sums[t - 1] > 0.0)) t--;
+    if (t > 0)
+        for (l = T - 1; l > 0 && !(prob<R>(a[(t - 1) * T + l]) > 0.0); l--) {}
+    out[shot] = t > 0 ? (t - 1) * T + l : 0;
+}
+
 // One block per shot: upper_bound over the tile prefix, then a block scan of
 // the chosen tile; the first index with u < cdf_i wins.  Bound by the tiles'
-// bytes from L2 and two or three dependent loads.  The tile is loaded with
-// lanes on neighbouring amplitudes and its probabilities pass through LDS (one
-// pad per 16); each thread reading its own 16 amplitudes, a 256-byte stride
-// between lanes, and one thread searching took 127 us for 2048 shots at 24
-// qubits and 67 us for 4096 at 14 (now 41 and 51 us).
+// bytes from L2 and two or three dependent loads; each thread reading its own
+// 16 amplitudes, a 256-byte stride between lanes, and one thread searching
+// took 127 us for 2048 shots at 24 qubits (now 41).
 template <typename R>
 __global__ __launch_bounds__(kRedThreads) void k_sample(const cplx_t<R> *__restrict__ a, int tile_bits,
                                                         uint64_t ntiles,
@@ -221,35 +317,10 @@ __global__ __launch_bounds__(kRedThreads) void k_sample(const cplx_t<R> *__restr
     const int ept = tsize >= kRedThreads ? tsize / kRedThreads : 1;
 
     for (uint64_t t = tile_of(tile_incl, ntiles, u, lane); t < ntiles; t++) {
-        const cplx_t<R> *ta = a + (t << tile_bits);
-        const double base = t ? tile_incl[t - 1] : 0.0;
         const int first_idx = tid * ept;
-#pragma unroll
-        for (int e = 0; e < kEpt; e++) {
-            const int i = e * kRedThreads + tid;
-            if (i < tsize) ps[i + (i >> 4)] = prob<R>(ta[i]);
-        }
-        __syncthreads();
         double p[kEpt];
-        double s = 0.0;
-#pragma unroll
-        for (int e = 0; e < kEpt; e++) {
-            const int i = first_idx + e;
-            p[e] = e < ept && i < tsize ? ps[i + (i >> 4)] : 0.0;
-            s += p[e];
-        }
-        double x = s;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const double y = __shfl_up(x, off, 64);
-            if (lane >= off) x += y;
-        }
-        if (lane == 63) wtot[wave] = x;
         if (tid == 0) s_first = INT_MAX;
-        __syncthreads();
-        double c = base;
-        for (int w = 0; w < wave; w++) c += wtot[w];
-        c += x - s;
+        double c = tile_cdf<R>(ps, wtot, a + (t << tile_bits), tsize, ept, t ? tile_incl[t - 1] : 0.0, p);
         int mine = INT_MAX;
 #pragma unroll
         for (int e = 0; e < kEpt; e++) {
@@ -434,13 +505,25 @@ hipError_t launch_sample(const SvDev &s, const ReduceWs &w, const double *d_u, i
                          uint64_t *d_out)
 {
     if (nshots <= 0) return hipSuccess;
-    if (s.prec == MOONLAB_HIP_C64)
-        k_sample<float><<<nshots, kRedThreads, 0, s.stream>>>((const float2 *)s.amps, w.tile_bits, w.ntiles,
-                                                               w.tile_incl, w.tile_sums, d_u, nshots, d_out);
-    else
-        k_sample<double><<<nshots, kRedThreads, 0, s.stream>>>((const double2 *)s.amps, w.tile_bits, w.ntiles,
-                                                                w.tile_incl, w.tile_sums, d_u, nshots, d_out);
-    return hipGetLastError();
+    auto go = [&](auto r) {
+        using R = decltype(r);
+        const cplx_t<R> *a = (const cplx_t<R> *)s.amps;
+        if ((uint64_t)nshots < 8 * w.ntiles || s.n > 25) {   // 256 MiB of sums at most
+            k_sample<R><<<nshots, kRedThreads, 0, s.stream>>>(a, w.tile_bits, w.ntiles, w.tile_incl, w.tile_sums, d_u,
+                                                              nshots, d_out);
+            return hipGetLastError();
+        }
+        double *cdf = nullptr;
+        hipError_t e = hipMallocAsync((void **)&cdf, sizeof(double) << s.n, s.stream);
+        if (e != hipSuccess) return e;
+        k_cdf<R><<<(unsigned)w.ntiles, kRedThreads, 0, s.stream>>>(a, w.tile_bits, w.tile_incl, cdf);
+        k_find<R><<<(nshots + 63) / 64, 64, 0, s.stream>>>(a, w.tile_bits, w.ntiles, w.tile_incl, w.tile_sums, cdf, d_u,
+                                                           nshots, d_out);
+        e = hipGetLastError();
+        hipError_t f = hipFreeAsync(cdf, s.stream);
+        return e == hipSuccess ? f : e;
+    };
+    return s.prec == MOONLAB_HIP_C64 ? go(float()) : go(double());
 }
 
 hipError_t launch_probabilities(const SvDev &s, double *d_p)
