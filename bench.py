@@ -167,15 +167,15 @@ FP64_PEAK_TFLOPS = 78.6
 
 
 def hea_flops(inst) -> float:
-    """Algorithmic FP64 flops of the HEA/TFIM batch: each RY and RZ a dense
-    complex 2x2 on 2^(n-1) pairs (4 complex multiply-adds, 28 flops per pair),
-    CZ sign flips counted as free, and the observables: |a|^2 (3 flops) plus
+    """FP64 flops of the HEA/TFIM batch as the engine runs it: each RY and RZ a
+    rotation 1 - i t P (one multiply-add per real component, 4 flops per
+    amplitude; a dense 2x2 would be 14), CZ free, and the observables: |a|^2 (3 flops) plus
     n - 1 ZZ accumulations per amplitude, and 2 Re(a_i* a_j) (4 flops) per pair
     for each <X_q>."""
     f = 0.0
     for n, L, _, _ in inst:
         D = 1 << n
-        f += 2 * L * n * (D // 2) * 28 + D * 3 + D * (n - 1) + n * (D // 2) * 4
+        f += 2 * L * n * D * 4 + D * 3 + D * (n - 1) + n * (D // 2) * 4
     return f
 
 
@@ -422,9 +422,9 @@ def fusion_cpu_baseline(n: int, gates: np.ndarray, budget_s: float) -> dict | No
 def run_blocked_workload(m, n: int, depth: int) -> dict:
     """The large-request engine: the n-qubit random-layer circuit (the
     serving stream's circuit family; H layer first) run as cache-blocked
-    register-phase passes (k_reg_pass), beside the same circuit as fused
+    rotation passes (k_frame_pass), beside the same circuit as fused
     <= 5-qubit MFMA blocks and as one kernel per gate, per precision.  The
-    complex128 register-engine state is checked against the per-gate state
+    complex128 state is checked against the per-gate state
     (fidelity, and max |amplitude| difference over 64 random runs of 4096
     amplitudes)."""
     from moonlab_amd import workloads
@@ -541,7 +541,8 @@ def run_fusion_workload(m, depth: int, cases) -> dict:
             "block_qubits_hist": {str(k): ks.count(k) for k in sorted(set(ks))},
             "device_seconds": round(t_fused, 4),
             "ms_per_block": round(t_fused / passes * 1e3, 3),
-            "state_TB_per_s": round(passes * 2 * D * amp_b / t_fused / 1e12, 3),
+            # as if every block read and wrote the state (several share a pass)
+            "block_TB_per_s": round(passes * 2 * D * amp_b / t_fused / 1e12, 3),
             "mfma_TFLOP_per_s": round(tflops, 2),
             "mfma_peak_TFLOP_per_s": peak,
             "mfma_frac": round(tflops / peak, 4),
@@ -581,7 +582,7 @@ def main() -> int:
     ap.add_argument("--workload", choices=("sweep", "fusion", "blocked", "batch", "serving"), default="sweep",
                     help="sweep: the 30-qubit gate sweep (with the batch and serving legs); "
                          "fusion: 32q complex64 and 33q complex128 SU(2)+CZ depth 60 on fused MFMA blocks; "
-                         "blocked: cache-blocked register-phase passes; "
+                         "blocked: cache-blocked rotation passes; "
                          "batch: the batch leg alone; serving: the served stream alone (both for profiler runs)")
     ap.add_argument("--fusion-depth", type=int, default=60)
     ap.add_argument("--fusion-cases", default="32:c64,33:c128")
@@ -604,14 +605,14 @@ def main() -> int:
         wall = time.perf_counter() - t0
         c128 = res["c128"]
         print(json.dumps({
-            "metric": "circuits/s, complex128, cache-blocked register-phase passes (large-request path)",
+            "metric": "circuits/s, complex128, cache-blocked rotation passes (large-request path)",
             "value": round(1.0 / c128["register_seconds"], 3), "unit": "circuits/s", "n_gpus": 1, "steps": 1,
             "warmup": 1, "ms_per_step": round(wall * 1e3, 1), "higher_is_better": True, "scaling": "weak",
             "vs_baseline": None, "dtype": "f64", "data": "synthetic",
             "config": {"workload": f"{args.qubits}-qubit random-layer circuit (H layer, depth {depth} of "
-                                   "RX|RY|RZ + CNOT brickwork), cache-blocked register-phase passes",
+                                   "RX|RY|RZ + CNOT brickwork), cache-blocked rotation passes",
                        "qubits": args.qubits, "depth": depth},
-            "roofline": {"bound": "hbm", "kernel": "k_reg_pass<double>",
+            "roofline": {"bound": "hbm", "kernel": "k_frame_pass<double>",
                          "achieved": round(c128["register_TB_per_s_per_pass"] * 1e3, 1), "peak": HBM_PEAK_GBS,
                          "unit": "GB/s", "frac": round(c128["register_TB_per_s_per_pass"] * 1e3 / HBM_PEAK_GBS, 4),
                          "traffic": None},
