@@ -203,7 +203,8 @@ MOONLAB_API moonlab_hip_status_t moonlab_hip_set_blocked_engine(int engine);
  * starting at, centred on and ending at the op's target) and the set taking
  * the most ops wins (about 2.8x fewer passes than the greedy choice on
  * 30-qubit random layers of depth 40); 0: both sets grow greedily in
- * circuit order.  Process-wide, like the other tuning calls. */
+ * circuit order.  The rotation engine takes a quarter as many seeds (more
+ * than two gain it nothing).  Process-wide, like the other tuning calls. */
 MOONLAB_API moonlab_hip_status_t moonlab_hip_set_blocked_lookahead(int windows);
 
 /* ---- Reductions ---------------------------------------------------------- */

@@ -949,7 +949,8 @@ def set_streaming_threshold(nbytes: int) -> None:
 
 
 def set_blocked_lookahead(windows: int = 8) -> None:
-    """Seed ops per pass and phase of the blocked planner's lookahead (0: greedy)."""
+    """Seed ops per pass and phase of the blocked planner's lookahead (0: greedy);
+    the rotation engine takes a quarter as many."""
     _check_hip(lib().moonlab_hip_set_blocked_lookahead(windows), "set_blocked_lookahead")
 
 
