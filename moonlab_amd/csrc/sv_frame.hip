@@ -15,7 +15,12 @@ namespace {
 // One pass: a workgroup of 2^(TB-4) threads streams tiles of 2^TB amplitudes.
 // Tiles enter and leave in the IO layout (lanes over the low tile bits: runs
 // of contiguous amplitudes); the next tile's loads are issued before the
-// current tile's rotations.
+// current tile's rotations.  Bound by latency: two waves per SIMD (complex128;
+// registers and LDS hold no more) between loads, layout changes and rotations.
+// A 30-qubit complex128 pass of 27 rotations takes 8.3 ms, 4.1 TB/s, with the
+// vector ALUs at 36 % and LDS at 28 %; the register-phase engine's took 15.5.
+// Its parts alone: an empty pass 5.5-6.5 ms, a rotation 0.076 ms (72 % of the
+// FP64 rate), a change of layout 0.27-0.4 ms.
 template <typename R, bool NT, int TB, int WPE>
 __global__ __launch_bounds__(1 << (TB - 4), WPE) void k_frame_pass(cplx_t<R> *__restrict__ a, const FPass *__restrict__ pass,
                                                                    const FOp *__restrict__ prog, uint64_t ntiles)
@@ -58,7 +63,9 @@ __global__ __launch_bounds__(1 << (TB - 4), WPE) void k_frame_pass(cplx_t<R> *__
     }
 }
 
-// A whole state of 4..11 qubits as one tile of one workgroup.
+// A whole state of 4..11 qubits as one tile of one workgroup: a chain of
+// rotations, 106 of them on 10 qubits in 60 us where a kernel for each of the
+// circuit's 202 gates took 0.8 ms.
 template <typename R>
 __global__ __launch_bounds__(128) void k_frame_small(cplx_t<R> *__restrict__ a,
                                                      const FPass *__restrict__ pass,
