@@ -525,7 +525,10 @@ class PassBuilder {
                 // the norm that the rounded tangent leaves, not the cosine
                 const long double t = bytes_ == 8 ? (long double)(float)g->t : (long double)g->t;
                 grow_ *= 1.0L + t * t;
-                if (grow_ > 0x1p1000L) settle();
+                if (grow_ > 0x1p1000L) {   // 2^1000 of it move to the exponent
+                    grow_ *= 0x1p-1000L;
+                    exp_ -= 500;
+                }
                 if (g->scale < 0.0) scale = -scale;
                 break;
             }
@@ -557,12 +560,15 @@ class PassBuilder {
         }
     }
 
-    // squared growth of the norm into the scale
+    // The pass's factor 2^exp_ / sqrt(grow_) into the scale.  Only here, where
+    // the growth and the rescalings that took it back on the way (phases) have
+    // met: either alone is 2^-500 for a thousand rotations.
     void settle()
     {
-        const long double f = 1.0L / sqrtl(grow_);
+        const long double f = ldexpl(1.0L / sqrtl(grow_), (int)exp_);
         scale = cd((double)(f * scale.real()), (double)(f * scale.imag()));
         grow_ = 1.0L;
+        exp_ = 0;
     }
 
     // x and z of an image in one word; two commute when parity(a & swap(b)) is 0
@@ -683,10 +689,10 @@ class PassBuilder {
                 // stored values grow by 1 / cos: rescale before single precision could overflow
                 grown += 0.5 * log2(1.0 + o.t * o.t);
                 if (grown > 32.0) {
-                    const double f = exp2(-floor(grown));
+                    const double k = floor(grown), f = exp2(-k);
                     prog_.push_back(FOp{FARM_SCALE, 0, 0, f, (float)f, 0});
-                    scale /= f;
-                    grown -= floor(grown);
+                    exp_ += (int64_t)k;
+                    grown -= k;
                 }
             }
             const int32_t nops = (int32_t)(prog_.size() - hpos) - kFPhaseUnits;
@@ -863,7 +869,8 @@ class PassBuilder {
     std::vector<FPass>    &passes_;
     std::vector<FOp>      &prog_;
     std::vector<uint32_t>  pack_;
-    long double            grow_ = 1.0L;
+    long double            grow_ = 1.0L;   // the pass's squared growth of the norm ...
+    int64_t                exp_ = 0;       // ... and what is to be multiplied back, as a power of two
     std::vector<Row>       X_, Z_;
     std::vector<LRot>      rots_;
     std::vector<Quad>      quads_;
