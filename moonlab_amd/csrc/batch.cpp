@@ -35,6 +35,7 @@
 #include "../../include/moonlab_mi355x.h"
 #include "batch_device.h"
 #include "batch_plan.h"
+#include "engine.h"
 #include "frame_plan.h"
 #include "fusion.h"
 #include "sv_internal.h"
@@ -834,6 +835,69 @@ int host_threads(size_t gates, int parts)
 constexpr double kTilePassUs = 6.0, kTileGateUs = 0.25, kLevelUs = 20.0;
 constexpr double kPauliUs = 3.4;   // a Pauli string on a tile in k_batch
 
+// A circuit with a parameter that is not finite, one kernel per gate, so that
+// NaN reaches the amplitudes the gate acts on and no others; what it measures
+// is read from its amplitudes on the host.
+int run_plain(moonlab_mi355x_batch_item_t &it, const PauliT *pauli, hipStream_t stream)
+{
+    RunRequest rq{};
+    rq.num_qubits = it.num_qubits;
+    rq.precision = it.precision;
+    rq.want_amps = rq.want_z = true;
+    rq.per_gate = true;
+    rq.stream = stream;
+    RunResult rr;
+    const int st = run_circuit_gates(rq, it.gates, it.num_gates, rr);
+    if (st) return st == MOONLAB_HIP_ERR_OUT_OF_MEMORY ? MOONLAB_SCHED_OOM : MOONLAB_SCHED_INTERNAL;
+    const int n = it.num_qubits;
+    const uint64_t dim = 1ull << n;
+    const cd *a = (const cd *)rr.amps.data();
+    auto par = [](uint64_t x) { return (__builtin_popcountll(x) & 1) != 0; };
+    // <P> = sum of Re[conj(a_(i ^ x)) a_i i^ny] with a sign (PauliT)
+    auto expect = [&](uint64_t x, uint64_t z, int ny) {
+        double s = 0.0;
+        for (uint64_t i = 0; i < dim; i++) {
+            const cd u = a[i ^ x], v = a[i];
+            const double re = u.real() * v.real() + u.imag() * v.imag(), im = u.real() * v.imag() - u.imag() * v.real();
+            const double c = ny == 0 ? re : ny == 1 ? -im : ny == 2 ? -re : im;
+            s += par(i & z) ? -c : c;
+        }
+        return s;
+    };
+    if (it.norm) *it.norm = rr.norm;
+    if (it.expect_z)
+        for (int q = 0; q < n; q++) it.expect_z[q] = it.observables & MOONLAB_MI355X_OBS_Z ? rr.z[(size_t)q] : 1.0;
+    if (it.zz_chain)
+        for (int q = 0; q + 1 < n; q++)
+            it.zz_chain[q] = it.observables & MOONLAB_MI355X_OBS_ZZ ? expect(0, 3ull << q, 0) : 0.0;
+    if (it.expect_x)
+        for (int q = 0; q < n; q++) it.expect_x[q] = it.observables & MOONLAB_MI355X_OBS_X ? expect(1ull << q, 0, 0) : 0.0;
+    double e = 0.0;
+    for (int k = 0; k < it.num_pauli_terms; k++) {
+        const double v = expect(pauli[k].x, pauli[k].z, pauli[k].ny & 3);
+        if (it.pauli_expect) it.pauli_expect[k] = v;
+        e += it.pauli_terms[k].coefficient * v;
+    }
+    if (it.num_pauli_terms > 0 && it.pauli_energy) *it.pauli_energy = e;
+    // shots: first index with u < cumulative probability, else the last with any
+    if (it.num_shots > 0) {
+        std::vector<double> cdf;   // up to the first NaN: nothing is below one
+        uint64_t last = 0;
+        double s = 0.0;
+        for (uint64_t i = 0; i < dim; i++) {
+            const double p = std::norm(a[i]);
+            s += p;
+            if (s == s) cdf.push_back(s);
+            if (p > 0.0) last = i;
+        }
+        for (int k = 0; k < it.num_shots; k++) {
+            const uint64_t i = (uint64_t)(std::upper_bound(cdf.begin(), cdf.end(), it.draws[k]) - cdf.begin());
+            it.outcomes[k] = i < cdf.size() ? i : last;
+        }
+    }
+    return MOONLAB_SCHED_OK;
+}
+
 int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int count,
               moonlab_mi355x_batch_stats_t *stats, const BatchStateOut *state_out = nullptr)
 {
@@ -849,6 +913,7 @@ int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int
             return MOONLAB_SCHED_BAD_ARG;
     std::vector<std::pair<double, int>> cost((size_t)count);
     std::vector<double> work((size_t)count);   // estimated microseconds on one workgroup
+    std::vector<char> plain((size_t)count, 0); // circuits that run_plain runs (an empty one in their place here)
     int64_t obs_total = 0, out_total = 0;
     int max_big = 0;
 
@@ -868,6 +933,22 @@ int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int
     auto plan_chunk = [&](Chunk &c) {
         std::vector<FGate> gates;
         cd phase;
+        // Gates whose parameters are not finite: NaN in every amplitude is
+        // what their rotations give too; where some amplitudes stay apart the
+        // circuit is left to run_plain (state outputs hold none of those).
+        auto lower = [&](const moonlab_mi355x_batch_item_t &it, int i) {
+            gates.clear();
+            if (frame_lower(it.gates, it.num_gates, it.num_qubits, gates, phase)) return true;
+            bool all = state_out != nullptr;
+            for (int k = 0; k < it.num_gates; k++) {
+                if (!gate_valid(it.gates[k], it.num_qubits)) return false;
+                all = all || gate_params(it.gates[k]) == PARAMS_SPOIL_ALL;
+            }
+            gates.clear();
+            plain[(size_t)i] = !all;
+            phase = 1.0;
+            return !all || frame_lower(it.gates, it.num_gates, it.num_qubits, gates, phase, true);
+        };
         for (int i = c.lo; i < c.hi; i++) {
             const moonlab_mi355x_batch_item_t &it = items[i];
             const int n = it.num_qubits;
@@ -877,8 +958,7 @@ int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int
                 c.bad = true;
                 return;
             }
-            gates.clear();
-            if (!frame_lower(it.gates, it.num_gates, n, gates, phase, true)) {
+            if (!lower(it, i)) {
                 c.bad = true;
                 return;
             }
@@ -1245,6 +1325,11 @@ int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int
             }
         }
     }
+    for (int i = 0; i < count; i++)
+        if (plain[(size_t)i]) {
+            const int rc = run_plain(items[i], pauli.data() + insts[(size_t)i].pauli_offset, b->stream);
+            if (rc) return rc;
+        }
     if (stats) {
         float ms = 0.f;
         hipEventElapsedTime(&ms, b->e0, b->e1);

@@ -523,7 +523,9 @@ __device__ __forceinline__ int cdf_find(const double *cdf, int T, double u)
 }
 
 // A tile of |0..0> other than the first is zero, and so it leaves a pass,
-// unless a parameter was not finite (the scale holds every cosine).
+// unless the pass's scale is not finite: the last one's of a circuit with a
+// parameter that is not (passes before it carry the scale on, so their zeros
+// may stay until then).
 __device__ __forceinline__ bool zero_stays_zero(FConst<FPass> P)
 {
     return P->scale_r - P->scale_r == 0.0 && P->scale_i - P->scale_i == 0.0;

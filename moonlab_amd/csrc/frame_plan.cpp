@@ -177,6 +177,25 @@ class Lowering {
 
 }  // namespace
 
+GateParams gate_params(const moonlab_hip_gate_t &g)
+{
+    const bool theta = std::isfinite(g.theta);
+    switch (g.type) {
+    case MOONLAB_HIP_GATE_RX:
+    case MOONLAB_HIP_GATE_RY:
+    case MOONLAB_HIP_GATE_RZ: return theta ? PARAMS_FINITE : PARAMS_SPOIL_ALL;
+    case MOONLAB_HIP_GATE_U3:
+        if (!theta) return PARAMS_SPOIL_ALL;
+        return std::isfinite(g.phi) && std::isfinite(g.lam) ? PARAMS_FINITE : PARAMS_SPOIL_PART;
+    case MOONLAB_HIP_GATE_PHASE:
+    case MOONLAB_HIP_GATE_CPHASE:
+    case MOONLAB_HIP_GATE_CRX:
+    case MOONLAB_HIP_GATE_CRY:
+    case MOONLAB_HIP_GATE_CRZ: return theta ? PARAMS_FINITE : PARAMS_SPOIL_PART;
+    default: return PARAMS_FINITE;   // reads none
+    }
+}
+
 bool frame_lower(const moonlab_hip_gate_t *g, int ng, int n, std::vector<FGate> &out, cd &phase, bool any_angle)
 {
     phase = 1.0;
@@ -189,7 +208,7 @@ bool frame_lower(const moonlab_hip_gate_t *g, int ng, int n, std::vector<FGate> 
     for (int i = 0; i < ng; i++) {
         const moonlab_hip_gate_t &x = g[i];
         if (!gate_valid(x, n)) return false;
-        if (!any_angle && (!std::isfinite(x.theta) || !std::isfinite(x.phi) || !std::isfinite(x.lam))) return false;
+        if (!any_angle && gate_params(x) != PARAMS_FINITE) return false;
         const int t = x.target, c = x.control, e = x.extra;
         const uint64_t T = t >= 0 ? 1ull << t : 0, C = c >= 0 ? 1ull << c : 0;
         double si, co;

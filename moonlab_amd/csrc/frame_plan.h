@@ -22,6 +22,13 @@ struct FGate {
     double    t, scale;
 };
 
+// What a gate's parameters make of a state: PARAMS_FINITE, or, where one that
+// the gate reads is not finite, NaN in every amplitude or in those of one
+// value of a qubit only (phases, controlled rotations, a U3 with its theta
+// finite).
+enum GateParams : int8_t { PARAMS_FINITE, PARAMS_SPOIL_ALL, PARAMS_SPOIL_PART };
+GateParams gate_params(const moonlab_hip_gate_t &g);
+
 // Gate list -> rotations and frame gates, and the global phase they leave
 // out.  False on an invalid gate or qubit, or, unless any_angle, a parameter
 // that is not finite (whose rotation would reach every amplitude).
