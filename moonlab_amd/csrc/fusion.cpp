@@ -431,24 +431,6 @@ std::vector<BlockTile> plan_block_tiles(const std::vector<FusedBlock> &blocks, i
     return out;
 }
 
-std::vector<cd> widen_block(const FusedBlock &b, const std::vector<int> &qubits)
-{
-    const size_t D = (size_t)1 << qubits.size(), d = (size_t)1 << b.qubits.size();
-    std::vector<size_t> own(D, 0);   // b's row of row r
-    size_t inside = 0;               // bits of r that are b's
-    for (size_t j = 0, k = 0; j < qubits.size(); j++) {
-        if (k >= b.qubits.size() || b.qubits[k] != qubits[j]) continue;
-        inside |= (size_t)1 << j;
-        for (size_t r = 0; r < D; r++) own[r] |= (r >> j & 1) << k;
-        k++;
-    }
-    std::vector<cd> m(D * D, cd(0.0));
-    for (size_t r = 0; r < D; r++)
-        for (size_t c = 0; c < D; c++)
-            if (((r ^ c) & ~inside) == 0) m[r * D + c] = b.mat[own[r] * d + own[c]];
-    return m;
-}
-
 int apply_fused(moonlab_hip_state_t *s, const moonlab_hip_gate_t *g, int ng, int kmax)
 {
     for (int i = 0; i < ng; i++) {
@@ -477,7 +459,7 @@ int apply_fused(moonlab_hip_state_t *s, const moonlab_hip_gate_t *g, int ng, int
         tiles.resize(blocks.size());
         for (size_t i = 0; i < blocks.size(); i++) tiles[i].members.push_back((int)i);
     }
-    // steps and every matrix of 3+ qubits go to the device in one copy
+    // steps and the matrices (alone: those of 3+ qubits) go to the device in one copy
     std::vector<DenseStep> steps;
     std::vector<unsigned char> mats;
     std::vector<size_t> first(tiles.size(), 0), off(blocks.size(), 0);
@@ -492,18 +474,14 @@ int apply_fused(moonlab_hip_state_t *s, const moonlab_hip_gate_t *g, int ng, int
             const FusedBlock &b = blocks[(size_t)i];
             const size_t at = off[(size_t)i] = mats.size();
             if (joint[t]) {
-                std::vector<int> qs = b.qubits;
-                for (int q = 0; qs.size() < 3; q++)
-                    if ((tiles[t].qubits >> q & 1) && std::find(b.qubits.begin(), b.qubits.end(), q) == b.qubits.end())
-                        qs.push_back(q);
-                std::sort(qs.begin(), qs.end());
-                const int k = (int)qs.size();
+                const int k = (int)b.qubits.size();
+                const int few = k == 2 && !b.only_gate ? kFewAll : b.only_gate || k < 3 ? kFew : 0;
                 int local[5];
-                for (int j = 0; j < k; j++) local[j] = __builtin_popcountll(tiles[t].qubits & ((1ull << qs[(size_t)j]) - 1ull));
+                for (int j = 0; j < k; j++)
+                    local[j] = __builtin_popcountll(tiles[t].qubits & ((1ull << b.qubits[(size_t)j]) - 1ull));
                 steps.emplace_back();
-                dense_step(steps.back(), d.prec, k, local, (uint32_t)(at / 16));
-                mats.resize(at + dense_operand_bytes(d.prec, k));
-                dense_operand(d.prec, k, (k == (int)b.qubits.size() ? b.mat : widen_block(b, qs)).data(), &mats[at]);
+                mats.resize(at + dense_operand_bytes(d.prec, k, few));
+                dense_step(steps.back(), d.prec, k, local, few, b.mat.data(), (uint32_t)(at / 16), &mats[at]);
             } else if (b.qubits.size() >= 3 && !b.only_gate) {
                 mats.resize(at + b.mat.size() * ab);
                 for (size_t j = 0; j < b.mat.size(); j++) {

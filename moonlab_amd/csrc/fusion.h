@@ -60,9 +60,6 @@ struct BlockTile {
 // greedily) that takes the most pending blocks.
 std::vector<BlockTile> plan_block_tiles(const std::vector<FusedBlock> &blocks, int n, int tile, int anchor);
 
-// Block b's unitary on `qubits` (ascending, a superset of b.qubits).
-std::vector<cd> widen_block(const FusedBlock &b, const std::vector<int> &qubits);
-
 // Apply a gate list through fusion (returns a moonlab_hip_status_t value).
 int apply_fused(moonlab_hip_state_t *s, const moonlab_hip_gate_t *g, int ng, int kmax);
 

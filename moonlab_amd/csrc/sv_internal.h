@@ -44,19 +44,27 @@ int apply_gates_planned(moonlab_hip_state_t *s, const moonlab_hip_gate_t *g, int
 
 // One block of a pass over 12-qubit tiles (k_block_tiles): local bits q
 // (ascending, qmask), the LDS slot of each block row, and where the matrix's
-// operands start in the pass's buffer, in 16-byte chunks.
+// operands start in the pass's buffer, in 16-byte chunks.  A block of one or
+// two qubits and a lone gate (1 to 3) go entry by entry (few): the matrix as
+// it is, row-major, and which of its reals are not 0 (bit 2 e: real part of
+// entry e, 2 e + 1: imaginary part; kFewAll: two qubits, every entry taken).
 constexpr int kDenseTileBits = 12;
+constexpr int kFew = 1, kFewAll = 2;
 struct DenseStep {
-    int32_t  k;          // 3..5
+    int32_t  k;          // 3..5; few: 1..3
     uint32_t mat;
     uint32_t qmask;
     int32_t  q[5];
     uint32_t row[32];
+    int32_t  few;        // 0, kFew or kFewAll
+    uint32_t nz[4];
+    uint32_t rows;       // few: rows that are not the identity's
 };
-void dense_step(DenseStep &st, int prec, int k, const int *local, uint32_t mat);
-// A k-qubit matrix (row-major) as the operands the pass reads, and their size.
-size_t dense_operand_bytes(int prec, int k);
-void   dense_operand(int prec, int k, const std::complex<double> *m, void *out);
+// A k-qubit matrix (row-major) as a step: the operands the pass reads go to
+// out, dense_operand_bytes of them.
+size_t dense_operand_bytes(int prec, int k, int few);
+void   dense_step(DenseStep &st, int prec, int k, const int *local, int few, const std::complex<double> *m,
+                  uint32_t mat, void *out);
 // nsteps blocks inside the tile set `qubits` (kDenseTileBits of them, the low
 // one among them); steps and matrices on the device
 hipError_t launch_block_tiles(const SvDev &s, uint64_t qubits, const DenseStep *d_steps, int nsteps, const void *d_mats);

@@ -442,6 +442,61 @@ __device__ __forceinline__ void tile_block(cplx_t<R> *lds, FConst<DenseStep> st,
     }
 }
 
+// A block of one or two qubits, or a lone gate, on the vector ALUs.  Entries
+// that are 0 are left out (not of a two-qubit block of several gates: ALL), so
+// an amplitude that is not finite reaches what the gate moves it to and no
+// more; widened to three qubits on the matrix cores the zeros took it to every
+// amplitude of its group.  Bound by LDS and the scalar loads of the entries.
+// Against the widened form, SU(2) + CZ layers of depth 12: 28 qubits complex128
+// in two-qubit blocks 158 -> 88 ms, one-qubit 313 -> 296 (complex64 149 ->
+// 110); 16 qubits 1.23 -> 1.05 and 2.47 -> 2.67 ms.
+template <typename R, int K, bool ALL>
+__device__ __forceinline__ void tile_few(cplx_t<R> *lds, FConst<DenseStep> st, const float4 *mat)
+{
+    constexpr int D = 1 << K;
+    FConst<R> m = (FConst<R>)(uintptr_t)mat;
+#pragma unroll 1
+    for (uint32_t i = threadIdx.x; i < (1u << (kBlockTileBits - K)); i += kThreads) {
+        if constexpr (K > 1 && !ALL) {
+            // opaque per turn: hoisted out of the loop, up to 128 tests and
+            // entries would spill the scalar registers
+            uint64_t sp = (uint64_t)(uintptr_t)st, mp = (uint64_t)(uintptr_t)m;
+            asm volatile("" : "+s"(sp), "+s"(mp));
+            st = (FConst<DenseStep>)sp;
+            m = (FConst<R>)mp;
+        }
+        uint32_t x = i;
+#pragma unroll
+        for (int j = 0; j < K; j++) x += x & (0u - (1u << st->q[j]));
+        const uint32_t g = tile_slot<R>(x), rows = st->rows;
+        cplx_t<R> a[D];
+#pragma unroll
+        for (int c = 0; c < D; c++) a[c] = lds[g ^ st->row[c]];
+#pragma unroll
+        for (int r = 0; r < D; r++) {
+            if (!ALL && !((rows >> r) & 1u)) continue;   // leaves its amplitude as it is
+            R u[2 * D];   // the row in one load, whichever entries it has
+#pragma unroll
+            for (int c = 0; c < 2 * D; c++) u[c] = m[2 * r * D + c];
+            cplx_t<R> y{R(0), R(0)};
+#pragma unroll
+            for (int c = 0; c < D; c++) {
+                const int e = r * D + c;
+                const uint32_t nz = ALL ? 3u : st->nz[e / 16] >> (2 * (e % 16));
+                if (nz & 1u) {
+                    y.x = fmar(u[2 * c], a[c].x, y.x);
+                    y.y = fmar(u[2 * c], a[c].y, y.y);
+                }
+                if (nz & 2u) {
+                    y.x = fmar(-u[2 * c + 1], a[c].y, y.x);
+                    y.y = fmar(u[2 * c + 1], a[c].x, y.y);
+                }
+            }
+            lds[g ^ st->row[r]] = y;
+        }
+    }
+}
+
 // The tile's loads wait for nothing but each other and nothing runs ahead: a
 // CU's other workgroups (four for complex64, two for complex128) cover them.
 // Keeping the matrices in LDS and loading the next tile during the products
@@ -475,7 +530,12 @@ k_block_tiles(cplx_t<R> *__restrict__ a, uint64_t ntiles, uint64_t mask, const D
         for (int b = 0; b < nsteps; b++) {
             const FConst<DenseStep> st = (FConst<DenseStep>)(uintptr_t)(steps + b);
             const float4 *m = mats + st->mat;
-            if (st->k == 5) tile_block<R, 5>(lds, st, m, lane, wave);
+            if (st->few) {
+                if (st->few == kFewAll) tile_few<R, 2, true>(lds, st, m);
+                else if (st->k == 1) tile_few<R, 1, false>(lds, st, m);
+                else if (st->k == 2) tile_few<R, 2, false>(lds, st, m);
+                else tile_few<R, 3, false>(lds, st, m);
+            } else if (st->k == 5) tile_block<R, 5>(lds, st, m, lane, wave);
             else if (st->k == 4) tile_block<R, 4>(lds, st, m, lane, wave);
             else tile_block<R, 3>(lds, st, m, lane, wave);
             lds_barrier();
@@ -587,11 +647,19 @@ void run_block_tiles(const SvDev &s, uint64_t mask, const DenseStep *steps, int 
 
 }  // namespace
 
-void dense_step(DenseStep &st, int prec, int k, const int *local, uint32_t mat)
+size_t dense_operand_bytes(int prec, int k, int few)
+{
+    // 4^k complex entries; the real embedding of 3 qubits holds 256 reals
+    return (prec == MOONLAB_HIP_C64 ? 8 : 16) * (k == 3 && !few ? (size_t)128 : (size_t)1 << (2 * k));
+}
+
+void dense_step(DenseStep &st, int prec, int k, const int *local, int few, const std::complex<double> *m, uint32_t mat,
+                void *out)
 {
     st = DenseStep{};
     st.k = k;
     st.mat = mat;
+    st.few = few;
     for (int j = 0; j < k; j++) {
         st.q[j] = local[j];
         st.qmask |= 1u << local[j];
@@ -601,19 +669,18 @@ void dense_step(DenseStep &st, int prec, int k, const int *local, uint32_t mat)
         for (int j = 0; j < k; j++) x |= (uint32_t)(r >> j & 1) << local[j];
         st.row[r] = prec == MOONLAB_HIP_C64 ? x ^ ((x >> 4 ^ x >> 8) & 14u) : (uint32_t)lds_slot<16>((int)x);
     }
-}
-
-size_t dense_operand_bytes(int prec, int k)
-{
-    // 4^k complex entries; the real embedding of 3 qubits holds 256 reals
-    return (prec == MOONLAB_HIP_C64 ? 8 : 16) * (k == 3 ? (size_t)128 : (size_t)1 << (2 * k));
-}
-
-void dense_operand(int prec, int k, const std::complex<double> *m, void *out)
-{
     auto go = [&](auto r) {
         using R = decltype(r);
-        if (k == 5) Block<R, 5>::order(m, (R *)out);
+        if (few) {
+            for (int e = 0; e < 1 << (2 * k); e++) {
+                const R x[2] = {(R)m[e].real(), (R)m[e].imag()};
+                ((R *)out)[2 * e] = x[0];
+                ((R *)out)[2 * e + 1] = x[1];
+                st.nz[e / 16] |= ((x[0] != R(0) ? 1u : 0u) | (x[1] != R(0) ? 2u : 0u)) << (2 * (e % 16));
+                const int row = e >> k, col = e & ((1 << k) - 1);
+                if (x[0] != R(row == col ? 1 : 0) || x[1] != R(0)) st.rows |= 1u << row;
+            }
+        } else if (k == 5) Block<R, 5>::order(m, (R *)out);
         else if (k == 4) Block<R, 4>::order(m, (R *)out);
         else Block<R, 3>::order(m, (R *)out);
     };
