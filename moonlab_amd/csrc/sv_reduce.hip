@@ -508,14 +508,18 @@ hipError_t launch_sample(const SvDev &s, const ReduceWs &w, const double *d_u, i
     auto go = [&](auto r) {
         using R = decltype(r);
         const cplx_t<R> *a = (const cplx_t<R> *)s.amps;
-        if ((uint64_t)nshots < 8 * w.ntiles || s.n > 25) {   // 256 MiB of sums at most
+        hipError_t e = hipSuccess;
+        double *cdf = nullptr;
+        if ((uint64_t)nshots >= 8 * w.ntiles && s.n <= 25) {   // 256 MiB of sums at most
+            e = hipMallocAsync((void **)&cdf, sizeof(double) << s.n, s.stream);
+            if (e != hipSuccess && e != hipErrorOutOfMemory) return e;
+            if (e != hipSuccess) (void)hipGetLastError();   // no room for the table: without it, then
+        }
+        if (e != hipSuccess || !cdf) {
             k_sample<R><<<nshots, kRedThreads, 0, s.stream>>>(a, w.tile_bits, w.ntiles, w.tile_incl, w.tile_sums, d_u,
                                                               nshots, d_out);
             return hipGetLastError();
         }
-        double *cdf = nullptr;
-        hipError_t e = hipMallocAsync((void **)&cdf, sizeof(double) << s.n, s.stream);
-        if (e != hipSuccess) return e;
         k_cdf<R><<<(unsigned)w.ntiles, kRedThreads, 0, s.stream>>>(a, w.tile_bits, w.tile_incl, cdf);
         k_find<R><<<(nshots + 63) / 64, 64, 0, s.stream>>>(a, w.tile_bits, w.ntiles, w.tile_incl, w.tile_sums, cdf, d_u,
                                                            nshots, d_out);

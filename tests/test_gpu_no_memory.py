@@ -1,0 +1,52 @@
+"""Calls whose optional device memory cannot be had run without it and give
+the same results.  The allocations are refused on the host, by
+tests/alloc_limit.c in a process of its own."""
+import json
+import os
+import subprocess
+import sys
+
+import pytest
+
+from conftest import ROOT
+
+pytestmark = pytest.mark.gpu
+
+HOST = """
+import ctypes, json, sys
+import numpy as np
+stub = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+sys.path.insert(0, sys.argv[2])
+import moonlab_amd as m
+limit, refused = ctypes.c_size_t.in_dll(stub, "alloc_limit_bytes"), ctypes.c_int.in_dll(stub, "alloc_refused")
+def limited(nbytes, call):
+    first = call()
+    limit.value, refused.value = nbytes, 0
+    second = call()
+    limit.value = 2 ** 64 - 1
+    return {"first": first, "second": second, "refused": refused.value}
+"""
+
+
+def run(tmp_path, code):
+    stub = str(tmp_path / "alloc_limit.so")
+    subprocess.run(["gcc", "-O2", "-shared", "-fPIC", os.path.join(ROOT, "tests", "alloc_limit.c"), "-o", stub, "-ldl"],
+                   check=True)
+    r = subprocess.run([sys.executable, "-c", HOST + code, stub, ROOT], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr
+    out = json.loads(r.stdout.strip().splitlines()[-1])
+    assert out["refused"] > 0
+    return out
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+def test_shots_without_the_cumulative_table(tmp_path, prec):
+    out = run(tmp_path, f"""
+rng = np.random.default_rng(5)
+sv = m.StateVector(16, {prec})
+a = rng.normal(size=1 << 16) + 1j * rng.normal(size=1 << 16)
+sv.load(a / np.linalg.norm(a))
+u = rng.uniform(size=8 * 16 + 40)
+print(json.dumps(limited(8 << 16, lambda: np.asarray(sv.sample(u)).tolist())))
+""")
+    assert out["first"] == out["second"]
