@@ -1042,7 +1042,7 @@ int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int
         std::vector<int>     count, tiles;  // by level
     } spread[2];
     uint64_t own_amps = 0;
-    {
+    auto spread_circuits = [&] {
         double longest = 0.0, all = 0.0, read = 0.0;
         int levels = 0;
         uint64_t amps = 0;
@@ -1082,7 +1082,7 @@ int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int
                 }
             }
         }
-    }
+    };
 
     // Pauli strings by workgroups of their own where the circuit with most to
     // measure would keep its workgroup longer than storing the states and one
@@ -1090,7 +1090,7 @@ int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int
     struct Strings {
         std::vector<int32_t> list, first;   // circuits; their first workgroup, and the sum
     } strings[2];
-    {
+    auto spread_strings = [&] {
         double most = 0.0;
         uint64_t amps = own_amps;
         for (const BInst &I : insts) {
@@ -1113,26 +1113,37 @@ int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int
                 S.first.push_back(S.first.back() + (I.num_pauli + kPauliChunk - 1) / kPauliChunk);
             }
         }
-    }
+    };
 
-    // grid: as many workgroups as fit, bounded by the HBM slots large circuits need
-    int grid = b->num_cus * b->wg_per_cu;
-    if (grid > count) grid = count;
+    // grid: as many workgroups as fit, bounded by the HBM slots large circuits
+    // need: 16 GiB with the circuits' own slots.  The precisions run side by
+    // side, on slots of their own, and share what there is.
+    int grid = 0, grid128 = 0, grid64 = 0;
+    size_t wgs = 0;
     uint64_t slot_amps = 1, tile_slot = 2;
-    for (const BInst &I : insts)
-        if (I.n > I.tile_bits && I.slot_offset < 0) slot_amps = std::max<uint64_t>(slot_amps, 1ull << I.n);
-    if (max_big) {
-        tile_slot = 2ull << (max_big - (tbmax < max_big ? tbmax : max_big));
-        const uint64_t per_wg = slot_amps * 16 + tile_slot * 8;
-        const uint64_t budget = 16ull << 30;
-        const uint64_t fit = budget / per_wg;
-        if ((uint64_t)grid > fit) grid = (int)(fit ? fit : 1);
-    }
-    // the precisions run side by side: slots of their own
-    const int grid128 = std::min(grid, n128), grid64 = std::min(grid, count - n128);
-    const size_t wgs = (size_t)(grid128 + grid64);
-    const size_t scratch_bytes = wgs * (slot_amps * 16 + tile_slot * 8) + own_amps * 16 + 256;
-    if (grow_dev(&b->d_scratch, &b->scratch_cap, scratch_bytes)) return MOONLAB_SCHED_OOM;
+    auto place_slots = [&] {
+        grid = std::min(b->num_cus * b->wg_per_cu, count);
+        grid128 = std::min(grid, n128);
+        grid64 = std::min(grid, count - n128);
+        slot_amps = 1;
+        for (const BInst &I : insts)
+            if (I.n > I.tile_bits && I.slot_offset < 0) slot_amps = std::max<uint64_t>(slot_amps, 1ull << I.n);
+        if (max_big) {
+            tile_slot = 2ull << (max_big - (tbmax < max_big ? tbmax : max_big));
+            const uint64_t fit = ((16ull << 30) - own_amps * 16) / (slot_amps * 16 + tile_slot * 8);
+            const uint64_t both = (uint64_t)(grid128 + grid64);
+            if (both > fit) {
+                grid128 = n128 ? (int)std::max<uint64_t>(fit * (uint64_t)grid128 / both, 1) : 0;
+                grid64 = count > n128 ? (int)std::max<uint64_t>(fit * (uint64_t)grid64 / both, 1) : 0;
+                grid = grid128 + grid64;
+            }
+        }
+        wgs = (size_t)(grid128 + grid64);
+        return wgs * (slot_amps * 16 + tile_slot * 8) + own_amps * 16 + 256;
+    };
+    spread_circuits();
+    spread_strings();
+    if (grow_dev(&b->d_scratch, &b->scratch_cap, place_slots())) return MOONLAB_SCHED_OOM;
 
     auto room = [](size_t need, size_t &have) {
         if (need > have || 2 * need + 128 < have) have = need + need / 8 + 64;

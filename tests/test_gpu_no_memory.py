@@ -28,14 +28,14 @@ def limited(nbytes, call):
 """
 
 
-def run(tmp_path, code):
+def run(tmp_path, code, refused=True):
     stub = str(tmp_path / "alloc_limit.so")
     subprocess.run(["gcc", "-O2", "-shared", "-fPIC", os.path.join(ROOT, "tests", "alloc_limit.c"), "-o", stub, "-ldl"],
                    check=True)
     r = subprocess.run([sys.executable, "-c", HOST + code, stub, ROOT], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
     out = json.loads(r.stdout.strip().splitlines()[-1])
-    assert out["refused"] > 0
+    assert (out["refused"] > 0) == refused
     return out
 
 
@@ -50,3 +50,14 @@ u = rng.uniform(size=8 * 16 + 40)
 print(json.dumps(limited(8 << 16, lambda: np.asarray(sv.sample(u)).tolist())))
 """)
     assert out["first"] == out["second"]
+
+
+def test_batch_scratch_of_both_precisions_in_one_budget(tmp_path):
+    # 140 circuits of 24 qubits: slots of 256 MiB, 16 GiB of them (a quarter more is asked for) for both precisions
+    out = run(tmp_path, """
+b = m.Batch()
+limit.value = (20 << 30) + (1 << 20)
+r = b.run([{"n": 24, "gates": [], "precision": k % 2} for k in range(140)])
+print(json.dumps({"refused": refused.value, "ok": all(x.norm == 1.0 and np.all(x.expect_z == 1.0) for x in r)}))
+""", refused=False)
+    assert out["ok"]
