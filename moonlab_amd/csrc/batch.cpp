@@ -1143,7 +1143,18 @@ int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int
     };
     spread_circuits();
     spread_strings();
-    if (grow_dev(&b->d_scratch, &b->scratch_cap, place_slots())) return MOONLAB_SCHED_OOM;
+    if (grow_dev(&b->d_scratch, &b->scratch_cap, place_slots())) {
+        // without slots of their own, each circuit on its workgroup
+        if (!own_amps) return MOONLAB_SCHED_OOM;
+        (void)hipGetLastError();
+        for (BInst &I : insts) I.slot_offset = I.pauli_slot = -1;
+        for (int p = 0; p < 2; p++) {
+            spread[p] = Spread();
+            strings[p] = Strings();
+        }
+        own_amps = 0;
+        if (grow_dev(&b->d_scratch, &b->scratch_cap, place_slots())) return MOONLAB_SCHED_OOM;
+    }
 
     auto room = [](size_t need, size_t &have) {
         if (need > have || 2 * need + 128 < have) have = need + need / 8 + 64;

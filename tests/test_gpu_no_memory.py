@@ -52,6 +52,25 @@ print(json.dumps(limited(8 << 16, lambda: np.asarray(sv.sample(u)).tolist())))
     assert out["first"] == out["second"]
 
 
+def test_batch_without_slots_of_its_circuits_own(tmp_path):
+    out = run(tmp_path, """
+rng = np.random.default_rng(6)
+terms = [(1.0, "".join("IXYZ"[k] for k in rng.integers(0, 4, size=12))) for _ in range(100)]
+def circuit(k):
+    gates = [(8, q, -1, -1, float(rng.uniform(0, 6))) for q in range(12)] + [(10, q + 1, q) for q in range(11)]
+    return {"n": 12, "gates": gates, "precision": k % 2, "pauli": terms}
+circuits = [circuit(k) for k in range(16)]
+b = m.Batch()
+def call():
+    global b
+    b.free()
+    b = m.Batch()
+    return [(r.norm, r.expect_z.tolist(), r.pauli_expect.tolist()) for r in b.run(circuits)]
+print(json.dumps(limited(1 << 20, call)))
+""")
+    assert out["first"] == out["second"]
+
+
 def test_batch_scratch_of_both_precisions_in_one_budget(tmp_path):
     # 140 circuits of 24 qubits: slots of 256 MiB, 16 GiB of them (a quarter more is asked for) for both precisions
     out = run(tmp_path, """
