@@ -46,7 +46,9 @@ __device__ __forceinline__ void frame_st(cplx_t<R> *p, const typename FVec<R>::t
 // before it runs, its sign (parities of a thread and a tile mask) and two
 // jumps.  A layout change is 16 LDS writes, a barrier and 16 reads per
 // thread.  The block leaves nothing in flight that it has started: every load
-// is waited for inside it.  Global loads the caller has in flight stay so.
+// is waited for inside it.  Global loads the caller has in flight stay so.  It
+// reads and writes the tile's LDS and runs barriers ("memory": the caller's
+// accesses stay on their side of it).
 #define MLX_FRAME_MACROS \
     ".ifndef mlx_frame_macros\n"                                                                          \
     ".set mlx_frame_macros, 1\n"                                                                          \
@@ -273,7 +275,7 @@ __device__ __forceinline__ void frame_st(cplx_t<R> *p, const typename FVec<R>::t
     ".LfZ%=:\n"                                                           
 
 #define MLX_FRAME_SCALARS \
-    "scc", "s36", "s37", "s38", "s39", "s40", "s41", "s42", "s43", "s44", "s45", "s46", "s47", "s48", \
+    "memory", "scc", "s36", "s37", "s38", "s39", "s40", "s41", "s42", "s43", "s44", "s45", "s46", "s47", "s48", \
         "s49", "s50", "s51", "s52", "s53", "s54", "s55", "s56", "s57", "s58", "s59", "s60", "s61", "s62", \
         "s63", "s64", "s65", "s66", "s67", "s68", "s69", "s70", "s71", "s72", "s73", "s74", "s75", "s76", \
         "s77", "s78", "s79", "s80", "s81", "s82", "s83", "s84", "s85", "s86", "s87", "s88", "s89", "s90", \
