@@ -761,6 +761,9 @@ struct moonlab_mi355x_batch {
     // (made when there is a mixed batch)
     hipStream_t aux = nullptr;
     hipEvent_t  fork = nullptr, join = nullptr;
+    // ... or after them (a server's engines: a stream more would share a
+    // hardware queue with an engine or a large worker, and the batch wait for it)
+    bool        one_stream = false;
     // HIP graph of the last batch shape (see moonlab_mi355x_batch_set_graphs)
     bool            use_graphs = true;
     hipGraphExec_t  gexec = nullptr;
@@ -1224,7 +1227,7 @@ int run_batch(moonlab_mi355x_batch_t *b, moonlab_mi355x_batch_item_t *items, int
 
     // the device step: upload, queue reset, passes of the spread circuits and
     // the persistent launch by precision, download
-    const bool beside = n128 > 0 && n128 < count;
+    const bool beside = n128 > 0 && n128 < count && !b->one_stream;
     if (beside && !b->aux &&
         (hipEventCreateWithFlags(&b->fork, hipEventDisableTiming) != hipSuccess ||
          hipEventCreateWithFlags(&b->join, hipEventDisableTiming) != hipSuccess ||
@@ -1386,6 +1389,8 @@ void *batch_state_buffer(moonlab_mi355x_batch_t *b, size_t bytes)
 }
 
 hipStream_t batch_stream(moonlab_mi355x_batch_t *b) { return b->stream; }
+
+void batch_use_one_stream(moonlab_mi355x_batch_t *b) { b->one_stream = true; }
 
 int mlx::apply_gates_planned(moonlab_hip_state_t *s, const moonlab_hip_gate_t *g, int ng)
 {
