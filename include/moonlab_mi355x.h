@@ -30,9 +30,10 @@ extern "C" {
 MOONLAB_API int moonlab_mi355x_register_backend(void);
 
 /* The backend's execute callback (moonlab_backend_execute_fn,
- * scheduler.h:235-238).  Reads the job only through the public job API
- * (moonlab_job_num_* and moonlab_job_to_json), so it also runs under the
- * reference's own scheduler.c when registered there. */
+ * scheduler.h:235-238).  The plugin library reads the job only through the
+ * public job API (moonlab_job_num_* and moonlab_job_to_json), so it also runs
+ * under the reference's own scheduler.c when registered there; the engine
+ * library takes the gates of its own scheduler's jobs as they are. */
 MOONLAB_API int moonlab_mi355x_backend_execute(const moonlab_job_t *job,
                                                moonlab_job_results_t *out, void *ctx);
 
