@@ -54,11 +54,11 @@ def sources() -> list[str]:
                   if f.endswith(".hip") or f.endswith(".cpp"))
 
 
-# Per-file device flags.  These kernels keep 16 amplitudes per thread in a
+# Per-file device flags.  sv_regpass.hip keeps 16 amplitudes per thread in a
 # register array whose op arms differ only in register indices; sinking the
 # arms' common tails merges them behind address phis that keep the array in
 # scratch memory, so that pass is off there.
-FILE_FLAGS = {f: ["-mllvm", "-simplifycfg-sink-common=false"] for f in ("sv_regpass.hip", "sv_frame.hip")}
+FILE_FLAGS = {"sv_regpass.hip": ["-mllvm", "-simplifycfg-sink-common=false"]}
 
 
 def _compile(src: str) -> str:

@@ -118,7 +118,7 @@ __host__ __device__ inline int lds_slot(int x)
 // kOpBuf descriptors, on 2 register bits: 4 amplitudes per thread.
 constexpr int kOpBuf = 32;
 constexpr int kSegRegsPass = 2;
-constexpr int kSegRegsBatch = 2;
+constexpr int kSegRegsBatch = kSegRegsPass;   // as the packing test names it
 
 struct BOp {
     int32_t  kind;
@@ -147,7 +147,6 @@ struct BInst {
     int32_t  tile_bits;     // tile bits of its passes: max(min(n, tile bits of the batch), 4)
     int32_t  first_pass;
     int32_t  num_passes;    // gate passes
-    int32_t  num_mpasses;   // measurement passes (follow the gate passes)
     int32_t  flags;         // BF_* below
     int32_t  num_shots;
     int64_t  obs_offset;    // into the FP64 observable buffer
