@@ -481,6 +481,8 @@ bool independent(const uint32_t *cols, int k, uint32_t v)
     return v != 0;
 }
 
+constexpr size_t kLookaheadOps = 4096;   // candidates are compared on (or seeded by) these pending gates
+
 class PassBuilder {
   public:
     PassBuilder(int amp_bytes, int lookahead, std::vector<FPass> &passes, std::vector<FOp> &prog)
@@ -594,11 +596,12 @@ class PassBuilder {
     static uint32_t packed(const Row &p) { return p.x | (p.z << 16); }
     static uint32_t swapped(uint32_t v) { return (v >> 16) | (v << 16); }
 
-    // Rotations of rest_ that a phase takes, in order: those whose direction
-    // is one of its (up to four) basis vectors and that commute with every
-    // rotation put off.  fixed: the basis is given whole.  "Commutes with
+    // Rotations of rest_ from head_ on that a phase takes, in order: those whose
+    // direction is one of its (up to four) basis vectors and that commute with
+    // every rotation put off.  fixed: the basis is given whole.  "Commutes with
     // every one" is checked against a basis of their span (at most 2 x tile
-    // bits words); once that is full nothing more can be taken.
+    // bits words); once that is full nothing more can be taken: the scan ends
+    // at stop_, so that a long circuit's planning stays linear.
     int scan(uint32_t *basis, int &nbasis, bool fixed)
     {
         take_.clear();
@@ -606,7 +609,7 @@ class PassBuilder {
         uint32_t span[2 * kFrameMaxTileBits];   // swapped words, echelon form by leading bit
         int rank = 0;
         const size_t m = rest_.size();
-        size_t i = 0;
+        size_t i = head_;
         for (; i < m && rank < 2 * nb_; i++) {
             const int id = rest_[i];
             const uint32_t w = pack_[(size_t)id], x = w & 0xFFFFu;
@@ -629,7 +632,7 @@ class PassBuilder {
             for (int d = 0; d < rank; d++) v = std::min(v, v ^ span[d]);   // clears span[d]'s leading bit
             if (v) span[rank++] = v;
         }
-        def_.insert(def_.end(), rest_.begin() + (long)i, rest_.end());
+        stop_ = i;
         return (int)take_.size();
     }
 
@@ -643,8 +646,9 @@ class PassBuilder {
             pack_[i] = packed(rots_[i].p);
         }
         double grown = 0.0;
-        size_t hpos = 0;   // header of the latest phase
-        while (!rest_.empty()) {
+        size_t hpos = 0, best_stop = 0;   // header of the latest phase
+        head_ = 0;
+        while (head_ < rest_.size()) {
             // candidates: for the first phase the layout the tile enters in
             // (no exchange through LDS; later phases have used up theirs), a
             // basis grown greedily, and bases seeded by the next pending directions
@@ -656,6 +660,7 @@ class PassBuilder {
                 if (got > 0) got++;   // a layout change costs about eight rotations' arithmetic, mostly hidden
                 best_take_.swap(take_);
                 best_def_.swap(def_);
+                best_stop = stop_;
             }
             auto candidate = [&](uint32_t seed) {
                 nb = 0;
@@ -667,13 +672,15 @@ class PassBuilder {
                     nbest = nb;
                     best_take_.swap(take_);
                     best_def_.swap(def_);
+                    best_stop = stop_;
                 }
             };
             candidate(0);
             if (look_ > 0) {
                 uint32_t seen[64];
                 int ns = 0;
-                for (size_t i = 0; i < rest_.size() && ns < look_ && ns < 64; i++) {
+                const size_t end = std::min(rest_.size(), head_ + kLookaheadOps);
+                for (size_t i = head_; i < end && ns < look_ && ns < 64; i++) {
                     const uint32_t x = rots_[(size_t)rest_[i]].p.x;
                     if (!x || std::find(seen, seen + ns, x) != seen + ns) continue;
                     seen[ns++] = x;
@@ -716,7 +723,9 @@ class PassBuilder {
             }
             const int32_t nops = (int32_t)(prog_.size() - hpos) - kFPhaseUnits;
             memcpy((char *)&prog_[hpos] + offsetof(FPhase, nops), &nops, sizeof nops);
-            rest_.swap(best_def_);
+            // those put off stay ahead of the ones not looked at
+            head_ = best_stop - best_def_.size();
+            std::copy(best_def_.begin(), best_def_.end(), rest_.begin() + (long)head_);
         }
     }
 
@@ -894,6 +903,7 @@ class PassBuilder {
     std::vector<LRot>      rots_;
     std::vector<Quad>      quads_;
     std::vector<int>       rest_, take_, def_, best_take_, best_def_;
+    size_t                 head_ = 0, stop_ = 0;   // rest_ before head_ is done; where a scan ended
     std::vector<uint16_t>  table_;
 };
 
@@ -927,12 +937,21 @@ void frame_plan(const std::vector<FGate> &gates, cd phase, int n, int tb, int an
         kinds[i] = kinds_of(gates[i]);
         need[i] = kinds[i].x | kinds[i].o;
     }
+    uint64_t az = 0, ax = 0, ao = 0;   // how any gate acts on the qubits
+    for (const Kinds &k : kinds) {
+        az |= k.z;
+        ax |= k.x;
+        ao |= k.o;
+    }
     const FGate *g0 = gates.data();
     uint64_t S = 0;
+    // the pending gates rest[head, lim) that a pass takes; it ends (at stop)
+    // once no gate could commute with all that are put off
+    size_t head = 0, stop = 0;
     auto scan = [&](uint64_t S0, size_t lim, std::vector<const FGate *> *take, std::vector<const FGate *> *defer) {
         uint64_t Sx = S0, bz = 0, bx = 0, bo = 0;
-        size_t taken = 0;
-        for (size_t i = 0; i < lim; i++) {
+        size_t taken = 0, i = head;
+        for (; i < lim && ((az & ~(bx | bo)) | (ax & ~(bz | bo)) | (ao & ~(bz | bx | bo))); i++) {
             const size_t id = (size_t)(rest[i] - g0);
             const Kinds &k = kinds[id];
             const bool clash = (k.z & (bx | bo)) | (k.x & (bz | bo)) | (k.o & (bz | bx | bo));
@@ -948,18 +967,18 @@ void frame_plan(const std::vector<FGate> &gates, cd phase, int n, int tb, int an
             }
         }
         if (take) S = Sx;
+        stop = i;
         return taken;
     };
-    constexpr size_t kLookaheadOps = 4096;   // candidates are compared on these pending gates
     std::vector<uint64_t> tried;
     const int free_bits = tb - anchor;
-    while (!rest.empty()) {
-        const size_t lim = std::min(rest.size(), kLookaheadOps);
+    while (head < rest.size()) {
+        const size_t lim = std::min(rest.size(), head + kLookaheadOps);
         uint64_t bestS0 = anchor_mask;
         size_t best = lookahead > 0 ? scan(anchor_mask, lim, nullptr, nullptr) : 0;
         tried.clear();
         int seeds = 0;
-        for (size_t i = 0; i < rest.size() && seeds < lookahead; i++) {
+        for (size_t i = head; i < rest.size() && seeds < lookahead; i++) {
             const uint64_t nd = need[(size_t)(rest[i] - g0)] & ~anchor_mask;
             if (!nd) continue;
             seeds++;
@@ -982,8 +1001,9 @@ void frame_plan(const std::vector<FGate> &gates, cd phase, int n, int tb, int an
         later.clear();
         scan(bestS0, rest.size(), &cur, &later);
         for (int q = 0; q < n && __builtin_popcountll(S) < nb; q++) S |= 1ull << q;
-        B.build(cur, S, nb, later.empty());
-        rest.swap(later);
+        B.build(cur, S, nb, later.empty() && stop == rest.size());
+        head = stop - later.size();
+        std::copy(later.begin(), later.end(), rest.begin() + (long)head);
     }
     if (gates.empty() && phase != cd(1.0)) B.build(cur, (1ull << nb) - 1, nb, true);
 }
