@@ -190,7 +190,9 @@ MOONLAB_API moonlab_hip_status_t moonlab_hip_set_blocked_tuning(int tile_bits, i
 /* Addition: engine of the blocked path: 0 = Pauli rotations (default; states
  * of at least 4 qubits: Clifford gates move a frame, the rest are rotations on
  * 16 amplitudes per thread; lists with a parameter that is not finite take
- * engine 2), 1 = LDS ops (one LDS sweep per op or register segment), 2 =
+ * engine 2, and states with an amplitude that is not finite, or in complex64
+ * one above 2^75, are better left to it: controlled gates become several
+ * rotations, and stored values grow on the way), 1 = LDS ops (one LDS sweep per op or register segment), 2 =
  * register phases (one op per gate, each thread keeps 16 tile amplitudes in
  * registers), 3 = register phases with 8 amplitudes per thread (twice the
  * waves, three register qubits per phase).  The register phases need 12

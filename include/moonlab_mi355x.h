@@ -43,7 +43,8 @@ typedef struct {
     int return_probabilities;  /* 1: fill `probabilities` (2^n doubles) */
     int return_expect_z;       /* 1: fill `expect_z` (n doubles) and `norm` */
     int fusion_max_qubits;     /* 1..5: fuse into k-qubit blocks; 0: passes over many gates or one kernel
-                                * per gate, whichever reads the state less often */
+                                * per gate, whichever reads the state less often (one kernel per gate
+                                * whatever the list: moonlab_hip_apply_gates on a state) */
     int skip_shots;            /* 1: ignore the job's shot count (state outputs only) */
     int blocked;               /* 1: cache-blocked passes (moonlab_hip_apply_gates_blocked) */
 } moonlab_mi355x_exec_options_t;
@@ -77,8 +78,9 @@ MOONLAB_API int moonlab_mi355x_set_state_cache_bytes(uint64_t bytes);
  *
  * Thousands of independent circuits of uneven size run in ONE kernel launch:
  * each GPU workgroup takes the next circuit from a device work queue and
- * simulates it to completion (states up to 12 qubits entirely in LDS; larger
- * ones cache-blocked through LDS from a per-workgroup HBM slot), then writes
+ * simulates it to completion (states up to 12 qubits in registers and LDS;
+ * larger ones tile by tile from a per-workgroup HBM slot, or, where few of
+ * them would leave the GPU idle, one launch per pass for all), then writes
  * the requested observables and shots.  Results for a circuit do not depend
  * on what else is in the batch (fixed per-circuit reduction order).
  * The workload shape is the reference's VQE energy loop
@@ -247,7 +249,7 @@ MOONLAB_API int moonlab_mi355x_vqe_natural_gradient(moonlab_mi355x_batch_t *b, c
  * (at most batch_max_qubits) are co-batched into persistent batch launches,
  * each batch taking everything admitted since the previous one was launched
  * (two batch engines alternate, so a batch is built while another runs);
- * larger requests run as fused blocks (or cache-blocked passes) on the large workers' streams.  A request's
+ * larger requests run as cache-blocked passes (or fused blocks) on the large workers' streams.  A request's
  * results are the same alone and in any mix. */
 
 typedef struct moonlab_mi355x_server moonlab_mi355x_server_t;
@@ -259,7 +261,7 @@ typedef struct {
     int      batch_engines;      /* concurrent batch launches (default 2) */
     int      large_workers;      /* concurrent large requests, each on its own stream (default 2) */
     int      sequential;         /* 1: plain dispatch -- one request at a time, one kernel per gate */
-    int      large_path;         /* large requests: 0 cache-blocked register-phase passes
+    int      large_path;         /* large requests: 0 cache-blocked rotation passes
                                     (default), 1 fused <= 5-qubit blocks on MFMA */
 } moonlab_mi355x_server_config_t;
 

@@ -14,7 +14,7 @@
 //     max_batch) into ONE persistent batch launch; with two engines, one batch
 //     is built and launched while the other runs, so arrivals never wait for
 //     a whole batch to drain before getting on the GPU;
-//   * large requests run as cache-blocked passes (register-phase tiles; or
+//   * large requests run as cache-blocked passes (Pauli rotations; or
 //     fused <= 5-qubit blocks on the matrix cores, large_path = 1), each large
 //     worker on one stream of its own for its whole life, overlapping with the
 //     batches on the device;

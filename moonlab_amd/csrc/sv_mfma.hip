@@ -396,8 +396,9 @@ __global__ __launch_bounds__(kThreads) void k_dense_mfma(cplx_t<R> *__restrict__
 
 // Several blocks in one pass: a workgroup holds a tile of 2^12 amplitudes in
 // LDS and applies every block whose qubits lie inside, so the state crosses
-// HBM once for all of them: 2.6 five-qubit (4.5 four-qubit, 7 three-qubit)
-// blocks of SU(2) + CZ layers.  Bound by the matrix cores, 64 to 76 % busy (one
+// HBM once for all of them: 2.2 five-qubit (4.6 four-qubit, 6 three-qubit)
+// blocks of SU(2) + CZ layers at 31 qubits complex64, 2.3 (4.3, 6.9) at 30
+// qubits complex128.  Bound by the matrix cores, 64 to 76 % busy (one
 // block per pass was bound by HBM, at 5.3 TB/s): depth 12 on 31 qubits,
 // complex64, 414 -> 292 ms in five-qubit blocks, 589 -> 229 in four-qubit ones
 // and 1214 -> 378 in three-qubit ones; 30 qubits complex128 417 -> 297, 594 ->
