@@ -708,7 +708,9 @@ template <typename T> hipError_t upload(const std::vector<T> &v, T **d, hipStrea
     return e;
 }
 
-hipError_t run_frames(moonlab_hip_state_t *s, const std::vector<FPass> &fp, std::vector<FOp> &prog)
+// no_room: set when the memory for the program could not be had (nothing ran)
+hipError_t run_frames(moonlab_hip_state_t *s, const std::vector<FPass> &fp, std::vector<FOp> &prog,
+                      bool *no_room = nullptr)
 {
     if (fp.empty()) return hipSuccess;
     const int n = (int)moonlab_hip_state_n_qubits(s), prec = moonlab_hip_state_precision(s);
@@ -720,6 +722,7 @@ hipError_t run_frames(moonlab_hip_state_t *s, const std::vector<FPass> &fp, std:
     memcpy((void *)&prog[units], fp.data(), fp.size() * sizeof(FPass));
     FOp *d_prog = nullptr;
     hipError_t e = upload(prog, &d_prog, st);
+    if (no_room) *no_room = e == hipErrorOutOfMemory && !d_prog;
     const FPass *d_pass = (const FPass *)(d_prog + units);
     for (size_t i = 0; e == hipSuccess && i < fp.size(); i++)
         e = launch_frame_pass(amps, prec, n, fp[i], d_pass + i, d_prog, st);
@@ -1401,10 +1404,13 @@ int mlx::apply_gates_planned(moonlab_hip_state_t *s, const moonlab_hip_gate_t *g
     const int n = (int)moonlab_hip_state_n_qubits(s);
     if (ng > 1 && plan_frames(g, ng, n, moonlab_hip_state_precision(s), gate_tuning(), fp, prog) &&
         2 * fp.size() <= (size_t)ng) {
-        const hipError_t e = run_frames(s, fp, prog);
+        bool no_room = false;
+        const hipError_t e = run_frames(s, fp, prog, &no_room);
         if (e == hipSuccess) return MOONLAB_HIP_OK;
-        return set_last_error(e == hipErrorOutOfMemory ? MOONLAB_HIP_ERR_OUT_OF_MEMORY : MOONLAB_HIP_ERR_DRIVER,
-                              "apply_gates", e);
+        if (!no_room)
+            return set_last_error(e == hipErrorOutOfMemory ? MOONLAB_HIP_ERR_OUT_OF_MEMORY : MOONLAB_HIP_ERR_DRIVER,
+                                  "apply_gates", e);
+        (void)hipGetLastError();   // one kernel per gate needs none
     }
     return moonlab_hip_apply_gates(s, g, ng);
 }

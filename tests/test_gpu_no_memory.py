@@ -80,3 +80,21 @@ r = b.run([{"n": 24, "gates": [], "precision": k % 2} for k in range(140)])
 print(json.dumps({"refused": refused.value, "ok": all(x.norm == 1.0 and np.all(x.expect_z == 1.0) for x in r)}))
 """, refused=False)
     assert out["ok"]
+
+
+def test_jobs_without_memory_for_their_program(tmp_path):
+    out = run(tmp_path, """
+rng = np.random.default_rng(7)
+job = m.Job(13)
+for _ in range(6):
+    for q in range(13):
+        job.add_gate(8, q, -1, float(rng.uniform(0, 6)))
+    for q in range(12):
+        job.add_gate(10, q + 1, q)
+def call():
+    r = job.execute_ex(amplitudes=True, expect_z=True, skip_shots=True)
+    return r.amplitudes.view(np.float64).tolist() + r.expect_z.tolist()
+r = limited(1, call)
+print(json.dumps({"refused": r["refused"], "worst": max(abs(a - b) for a, b in zip(r["first"], r["second"]))}))
+""")
+    assert out["worst"] < 1e-12
