@@ -98,3 +98,13 @@ r = limited(1, call)
 print(json.dumps({"refused": r["refused"], "worst": max(abs(a - b) for a, b in zip(r["first"], r["second"]))}))
 """)
     assert out["worst"] < 1e-12
+
+
+def test_small_blocks_without_memory_for_their_steps(tmp_path):
+    out = run(tmp_path, """
+from moonlab_amd import workloads
+sv, g = m.StateVector(14), workloads.su2_cz_circuit(14, 3, 1)
+r = limited(1, lambda: sv.reset().apply(g, fuse=2).amplitudes().view(np.float64).tolist())
+print(json.dumps({"refused": r["refused"], "worst": max(abs(a - b) for a, b in zip(r["first"], r["second"]))}))
+""")
+    assert out["worst"] < 1e-12
